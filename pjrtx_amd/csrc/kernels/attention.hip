@@ -38,6 +38,7 @@
 
 #include "common.h"
 #include "kernels/attention.h"
+#include "kernels/lds_dma.h"
 
 namespace pjrtx {
 namespace {
@@ -344,7 +345,9 @@ __global__ void __launch_bounds__(256, 2) attn_tiles(AttnParams p, const uint16_
 // gfx950:
 //  * K and V blocks go from global memory straight into LDS (buffer loads
 //    with the LDS destination, 16 bytes a lane), two LDS stages each, one
-//    barrier per block; no register staging.
+//    barrier per block; no register staging. The loads are lds_dma16: with
+//    the compiler's builtin the next block's K and V were waited for before
+//    this block's K and V reads ([8,32,2048,128] causal bf16: 352 -> 347 us).
 //  * V stays row-major in LDS; the V^T fragments of O^T += V^T.P^T come from
 //    transposing LDS reads (ds_read_b64_tr_b16: lane j of a 16-lane group
 //    gets element j & 3 of the rows that lanes 4e + (j >> 2) address, e =
@@ -446,10 +449,8 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
   // Buffer resources over this head's keys: rows past Skv read as zero.
   const uint32_t k_bytes = (uint32_t)(((int64_t)(p.Skv - 1) * p.k_s + D) * 2);
   const uint32_t v_bytes = (uint32_t)(((int64_t)(p.Skv - 1) * p.v_s + D) * 2);
-  const __amdgpu_buffer_rsrc_t krs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(Kp), 0, p.Skv > 0 ? (int)k_bytes : 0, 0x00020000);
-  const __amdgpu_buffer_rsrc_t vrs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(Vp), 0, p.Skv > 0 ? (int)v_bytes : 0, 0x00020000);
+  const lds_rsrc krs = make_lds_rsrc(Kp, p.Skv > 0 ? k_bytes : 0);
+  const lds_rsrc vrs = make_lds_rsrc(Vp, p.Skv > 0 ? v_bytes : 0);
   // Wave w fills rows 16w .. 16w+15 of a stage, four rows per load; the
   // lane part of each load's offset is fixed, the block part is scalar.
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -461,19 +462,18 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
     koff[i] = (uint32_t)(((int64_t)row * p.k_s + ((lslot ^ (row & 15)) * 8)) * 2);
     voff[i] = (uint32_t)(((int64_t)row * p.v_s + ((lslot ^ ((row & 7) << 1)) * 8)) * 2);
   }
+  const uint32_t klds = lds_offset(Ks + wave_u * 16 * 128), vlds = lds_offset(Vs + wave_u * 16 * 128);
   auto dma_k = [&](int kb, int stage) {
     const uint32_t sblk = (uint32_t)((int64_t)kb * PK * p.k_s * 2);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (attn_lds_ptr)(Ks + stage * PSTAGE + (wave_u * 16 + i * 4) * 128),
-                                               16, koff[i], sblk, 0, 0);
+      lds_dma16(krs, koff[i], sblk, klds + (uint32_t)(stage * PSTAGE + i * 4 * 128) * 2);
   };
   auto dma_v = [&](int kb, int stage) {
     const uint32_t sblk = (uint32_t)((int64_t)kb * PK * p.v_s * 2);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (attn_lds_ptr)(Vs + stage * PSTAGE + (wave_u * 16 + i * 4) * 128),
-                                               16, voff[i], sblk, 0, 0);
+      lds_dma16(vrs, voff[i], sblk, vlds + (uint32_t)(stage * PSTAGE + i * 4 * 128) * 2);
   };
 
   const float c2 = p.scale * 1.44269504088896340736f;
