@@ -102,6 +102,16 @@ MemRef canonicalize(Device* dev, const TensorType& t, const Dims& batch, const D
 
 }  // namespace
 
+namespace {
+// Bytes this thread may still allocate on the device: what the installed
+// fixed block has left, or no bound.
+int64_t scratch_left(Device* dev) {
+  const Arena* a = thread_arena();
+  if (!a || a->dev != dev) return int64_t(1) << 60;
+  return static_cast<int64_t>(a->cap - std::min(a->cap, (a->used + 255) & ~size_t(255)));
+}
+}  // namespace
+
 // Workgroups of the one-pass GEMV for a single product with N columns.
 int single_wide_tiles(int64_t N) {
   GemvGroup one;
@@ -140,31 +150,53 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
   if (low_precision && out_ok) {
     const bool f16 = lt.dtype == DType::kF16;
     const int out_kind = ot.dtype == DType::kBF16 ? 0 : (ot.dtype == DType::kF16 ? 1 : 2);
-    MemRef a_copy, b_copy;
-    // LHS must be K-contiguous with 16-byte aligned rows.
-    const bool a_fast = a.ok && (a.ks == 1 || K == 1) && (M == 1 || a.fs % 8 == 0) && (batch == 1 || a.bs % 8 == 0) &&
-                        aligned16(A) && K % 8 == 0;
-    if (!a_fast && K % 8 == 0) {
+    MemRef a_copy, b_copy, a_pad, b_pad;
+    // Copies the call makes must fit a fixed block (allocation-free execute)
+    // where one is installed; those that would not take the strided fallback.
+    const auto fits = [&](int64_t bytes) { return scratch_left(dev) >= bytes + 4096; };
+    // (An M-contiguous A goes to the GEMV kernels and to rows too long for
+    // 32-bit offsets as a copy.)
+    if ((!a.ok || (a.ks != 1 && K != 1 && (M <= 8 || a.ks >= int64_t(1) << 23))) && fits(lt.bytes())) {
       a_copy = canonicalize(dev, lt, op.lhs_batch, op.lhs_contract, A, true);
       A = a_copy->ptr;
       a = OperandView{batch, M, K, M * K, K, 1, true};
     }
-    // RHS: N-contiguous ([K][N]) or K-contiguous ([N][K]).
-    bool b_kmajor = b.ok && (b.ks == 1 || K == 1) && (N == 1 || b.fs % 8 == 0) && (batch == 1 || b.bs % 8 == 0) &&
-                    aligned16(B) && K % 8 == 0;
-    bool b_nmajor = b.ok && (b.fs == 1 || N == 1) && (K == 1 || b.ks % 8 == 0) && (batch == 1 || b.bs % 8 == 0) &&
-                    aligned16(B) && N % 8 == 0;
-    if (b_nmajor && N != 1) b_kmajor = false;
-    if (!b_kmajor && !b_nmajor && K % 8 == 0) {
+    if (!b.ok && fits(rt.bytes())) {
       b_copy = canonicalize(dev, rt, op.rhs_batch, op.rhs_contract, B, true);  // [batch][N][K]
       B = b_copy->ptr;
       b = OperandView{batch, N, K, N * K, K, 1, true};
-      b_kmajor = true;
     }
-    if ((a_fast || a_copy) && (b_kmajor || b_nmajor) && K % 8 == 0) {
-      if (M <= 8 && batch == 1 && !b_kmajor && !a_copy && N < (int64_t(1) << 30) &&
-          gemv_wide_fits(static_cast<int>(M), static_cast<int>(K), single_wide_tiles(N)) && N % 8 == 0 &&
-          (K == 1 || b.ks % 8 == 0)) {
+    // K-contiguous as it is, else M- or N-contiguous; an operand with rows
+    // that are not 16-byte aligned is copied into padded ones.
+    bool a_kmajor = false, b_kmajor = false;
+    const auto aligned_rows = [&](const void* p, const OperandView& v, bool kc) {
+      const int64_t ld = kc ? v.fs : v.ks, rows = kc ? v.free : v.k;
+      return aligned16(p) && (rows == 1 || ld % 8 == 0) && (batch == 1 || v.bs % 8 == 0) && (!kc || K % 8 == 0);
+    };
+    const auto pad = [&](const void** p, OperandView* v, bool kc, MemRef* mem) {
+      const int64_t rows = kc ? v->free : v->k, cols = kc ? v->k : v->free, ldp = (cols + 7) / 8 * 8;
+      if (batch >= 65536 || rows * (ldp / 8) >= (int64_t(1) << 38) || !fits(batch * rows * ldp * 2)) return false;
+      *mem = dev->allocate(static_cast<size_t>(batch * rows * ldp) * 2);
+      const int64_t rs = kc ? (v->fs ? v->fs : cols) : (v->ks ? v->ks : cols);
+      launch_pad_rows16(dev->stream(), *p, (*mem)->ptr, batch, v->bs, rows, rs, cols, ldp);
+      *p = (*mem)->ptr;
+      v->bs = rows * ldp;
+      (kc ? v->fs : v->ks) = ldp;
+      (kc ? v->ks : v->fs) = 1;
+      return true;
+    };
+    bool ready = a.ok && b.ok;
+    if (ready) {
+      a_kmajor = a.ks == 1 || K == 1;
+      b_kmajor = (b.ks == 1 || K == 1) && !(b.fs == 1 && N != 1);
+      ready = (a_kmajor || a.fs == 1 || M == 1) && (b_kmajor || b.fs == 1 || N == 1);
+    }
+    // Decode rows: W streamed once. (K may be any length for an N-contiguous
+    // W; a K-contiguous one needs 16-byte rows.)
+    if (ready && M <= 8 && (a.ks == 1 || K == 1) && aligned_rows(B, b, b_kmajor) && (b_kmajor || N % 8 == 0) &&
+        (!b_kmajor || (aligned16(A) && (M == 1 || a.fs % 8 == 0) && (batch == 1 || a.bs % 8 == 0)))) {
+      if (batch == 1 && !b_kmajor && N < (int64_t(1) << 30) &&
+          gemv_wide_fits(static_cast<int>(M), static_cast<int>(K), single_wide_tiles(N))) {
         GemvGroup g;
         g.count = 1;
         g.M = static_cast<int>(M);
@@ -179,58 +211,63 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
         launch_gemv_wide(dev->stream(), g, A, f16);
         return;
       }
-      if (M <= 8) {
-        GemvParams g;
-        g.batch = static_cast<int>(batch);
-        g.M = static_cast<int>(M);
-        g.N = static_cast<int>(N);
-        g.K = static_cast<int>(K);
-        g.ldx = a.fs ? a.fs : K;
-        g.ldw = b_kmajor ? (b.fs ? b.fs : K) : (b.ks ? b.ks : N);
-        g.ldy = N;
-        g.x_bs = a.bs;
-        g.w_bs = b.bs;
-        g.y_bs = M * N;
-        g.out_kind = out_kind;
-        MemRef part;
-        if (!b_kmajor) {
-          plan_gemv_split(&g);
-          if (g.ksplit > 1) part = dev->allocate(static_cast<size_t>(batch * g.ksplit * M * N) * 4);
-        }
+      GemvParams g;
+      g.batch = static_cast<int>(batch);
+      g.M = static_cast<int>(M);
+      g.N = static_cast<int>(N);
+      g.K = static_cast<int>(K);
+      g.ldx = a.fs ? a.fs : K;
+      g.ldw = b_kmajor ? (b.fs ? b.fs : K) : (b.ks ? b.ks : N);
+      g.ldy = N;
+      g.x_bs = a.bs;
+      g.w_bs = b.bs;
+      g.y_bs = M * N;
+      g.out_kind = out_kind;
+      MemRef part;
+      bool room = true;
+      if (!b_kmajor) {
+        plan_gemv_split(&g);
+        const int64_t bytes = batch * g.ksplit * M * N * 4;
+        if (g.ksplit > 1 && !(room = fits(bytes))) g.ksplit = 1;
+        if (g.ksplit > 1) part = dev->allocate(static_cast<size_t>(bytes));
+      }
+      if (room) {
         launch_gemv(dev->stream(), g, A, B, out, part ? static_cast<float*>(part->ptr) : nullptr, f16, b_kmajor);
         return;
       }
+    }
+    if (ready && !aligned_rows(A, a, a_kmajor)) ready = pad(&A, &a, a_kmajor, &a_pad);
+    if (ready && !aligned_rows(B, b, b_kmajor)) ready = pad(&B, &b, b_kmajor, &b_pad);
+    if (ready) {
       GemmParams g;
       g.batch = static_cast<int>(batch);
       g.M = static_cast<int>(M);
       g.N = static_cast<int>(N);
       g.K = static_cast<int>(K);
-      g.lda = a.fs ? a.fs : K;
-      g.ldb = b_kmajor ? (b.fs ? b.fs : K) : (b.ks ? b.ks : N);
+      const auto round8 = [](int64_t n) { return (n + 7) / 8 * 8; };
+      // One row only: its stride is not used; a multiple of 8.
+      g.lda = a_kmajor ? (M == 1 ? round8(K) : a.fs) : (K == 1 ? round8(M) : a.ks);
+      g.ldb = b_kmajor ? (N == 1 ? round8(K) : b.fs) : (K == 1 ? round8(N) : b.ks);
       g.ldc = N;
-      g.a_batch_stride = a.bs;
-      g.b_batch_stride = b.bs;
-      if (batch * M * N * K > 0 && blaslt_wanted(g) &&
+      g.a_batch_stride = batch == 1 ? 0 : a.bs;
+      g.b_batch_stride = batch == 1 ? 0 : b.bs;
+      if (a_kmajor && K % 8 == 0 && (b_kmajor || N % 8 == 0) && blaslt_wanted(g) &&
           blaslt_gemm(dev, g, A, B, out, f16, b_kmajor, out_kind == 2 ? 4 : 2))
         return;
-      MemRef bt;
-      if (!b_kmajor && !use_big_gemm(g, false)) {
-        // The large-tile kernel reads an N-contiguous B directly when its
-        // rows allow (N a multiple of 8); otherwise transpose B ([K][N] per
-        // batch) once, at HBM speed, when the kernel applies to the result.
-        GemmParams t = g;
-        t.ldb = K;
-        t.b_batch_stride = N * K;
-        if (use_big_gemm(t, true) && g.ldb == N && (batch == 1 || b.bs == K * N)) {
-          bt = dev->allocate(static_cast<size_t>(batch * N * K) * 2);
-          launch_transpose16(dev->stream(), B, bt->ptr, batch, K, N, K * N, N * K);
-          B = bt->ptr;
-          g = t;
-          b_kmajor = true;
-        }
+      if (gemm_fits(g, a_kmajor, b_kmajor)) {
+        // Partials of a k-split: at most 64 MiB, and what a fixed block has left.
+        const int64_t left = std::max<int64_t>(0, std::min<int64_t>(int64_t(64) << 20, scratch_left(dev) - 4096));
+        const GemmPlan plan = plan_gemm(g, left);
+        MemRef ws;
+        if (plan.workspace) ws = dev->allocate(plan.workspace);
+        launch_gemm(dev->stream(), g, plan, A, a_kmajor, B, b_kmajor, out, f16, out_kind == 2 ? 4 : 2,
+                    ws ? static_cast<float*>(ws->ptr) : nullptr);
+        return;
       }
-      launch_mfma_gemm(dev->stream(), g, A, B, out, f16, b_kmajor, out_kind == 2 ? 4 : 2);
-      return;
+      if (a_kmajor && K % 8 == 0 && (b_kmajor || N % 8 == 0)) {
+        launch_mfma_gemm(dev->stream(), g, A, B, out, f16, b_kmajor, out_kind == 2 ? 4 : 2);
+        return;
+      }
     }
   }
   // Scalar fallback with general strides.

@@ -9,24 +9,46 @@
 
 namespace pjrtx {
 
-// C[b][m][n] = sum_k A[b][m][k] * B[b][k][n]; A K-contiguous (row stride lda);
-// B N-contiguous ([K][N], row stride ldb) or K-contiguous ([N][K]); C row-major
+// C[b][m][n] = sum_k A[b][m][k] * B[b][k][n] for 16-bit inputs; A
+// K-contiguous ([M][K], row stride lda) or M-contiguous ([K][M]); B
+// N-contiguous ([K][N], row stride ldb) or K-contiguous ([N][K]); C row-major
 // with row stride ldc and batch stride M*ldc. Strides in elements.
 struct GemmParams {
   int batch = 1, M = 0, N = 0, K = 0;
   int64_t lda = 0, ldb = 0, ldc = 0;
   int64_t a_batch_stride = 0, b_batch_stride = 0;
+  int split_tiles = 1 << 30;  // 64-deep k-tiles per k-split
 };
+
+// MFMA block tiles (kernels/gemm.hip). A K-contiguous operand whose K is no
+// multiple of 8 must be zero from K to its row stride.
+constexpr int kGemmTiles = 6;
+struct GemmPlan {
+  int cfg = 0;              // block tile
+  int splits = 1;           // over K: f32 partials, summed by a second launch
+  int split_tiles = 1 << 30;
+  size_t workspace = 0;     // bytes of the partials
+};
+// True when the tile kernels take the operands: 16-byte aligned rows and
+// lane offsets below 2^31 bytes (K-contiguous rows up to 4M elements,
+// otherwise up to 16M). The base addresses must be 16-byte aligned.
+bool gemm_fits(const GemmParams& p, bool a_kmajor, bool b_kmajor);
+// Block tile and k-split with the least estimated time (environment:
+// PJRTX_GEMM_TILE forces a tile, PJRTX_BIG_GEMM_MIN_TILES=n takes 256 x 256
+// tiles for every product with at least n of them); the partials take at most
+// max_workspace bytes.
+GemmPlan plan_gemm(const GemmParams& p, int64_t max_workspace);
+void launch_gemm(hipStream_t s, GemmParams p, const GemmPlan& plan, const void* A, bool a_kmajor, const void* B,
+                 bool b_kmajor, void* C, bool f16, int out_bytes, float* workspace);
+// out[b][r][0, ldp) = in[b][r][0, cols) (batch stride bs, row stride rs),
+// then zeros, for 16-bit elements; ldp a multiple of 8.
+void launch_pad_rows16(hipStream_t s, const void* in, void* out, int64_t batch, int64_t bs, int64_t rows, int64_t rs,
+                       int64_t cols, int64_t ldp);
+
+// The same product for operands whose rows are too long for the tile
+// kernels' 32-bit lane offsets; A K-contiguous.
 void launch_mfma_gemm(hipStream_t s, const GemmParams& p, const void* A, const void* B, void* C, bool f16, bool b_kmajor,
                       int out_bytes);
-// True when the 256 x 256 tile kernel applies (M, N >= 256, 16-byte aligned
-// rows, K a multiple of 8 and, for an N-contiguous B, N too; enough tiles to
-// fill the GPU). It takes B in either layout.
-bool use_big_gemm(const GemmParams& p, bool b_kmajor);
-// out[b] = transpose(in[b]) for 16-bit elements: in [rows][cols] -> out
-// [cols][rows], batch strides in elements.
-void launch_transpose16(hipStream_t s, const void* in, void* out, int64_t batch, int64_t rows, int64_t cols,
-                        int64_t in_bs, int64_t out_bs);
 
 // Y[b][m][n] = sum_k X[b][m][k] * W[b][.]: M in 1..8 (decode rows). W is
 // [K][N] (N contiguous, row stride ldw) or, when K-major, [N][K] (K

@@ -1,6 +1,7 @@
-// dot_general kernels for gfx950.
+// dot_general kernels for gfx950 other than the MFMA block tiles of gemm.hip.
 //
-//  * mfma_gemm: C[b] = A[b] (MxK) * B[b] (KxN) for bf16 / f16 inputs with f32
+//  * mfma_gemm: operands whose rows are too long for gemm.hip's 32-bit lane
+//    offsets (4M elements and more). C[b] = A[b] (MxK) * B[b] (KxN) for bf16 / f16 inputs with f32
 //    accumulation on v_mfma_f32_16x16x32_{bf16,f16}. 128x128 block tile,
 //    BK = 64, 256 threads (4 waves in 2x2, 64x64 each), LDS double buffer,
 //    B either N-contiguous ([K][N], transposed into LDS) or K-contiguous
@@ -227,358 +228,6 @@ __global__ void __launch_bounds__(256) mfma_gemm(GemmParams p, const uint16_t* _
           const int n = n0 + wn * 64 + j * 16 + (lane & 15);
           if (m < p.M && n < p.N) Cb[(int64_t)m * p.ldc + n] = acc[i][j][r];
         }
-  }
-}
-
-// ------------------------------------------------------------- large GEMM
-// gemm_nt_256: C[b] = A[b] (M x K, K contiguous) * B[b]^T (N x K, K
-// contiguous) for products with enough 256 x 256 tiles to fill the GPU.
-//  * 256 x 256 block tile, 64-deep k-tiles, 512 threads: 2 x 4 waves of
-//    128 x 64 (4 x 2 blocks of v_mfma_f32_32x32x16, 128 f32 accumulators a
-//    lane), two waves per SIMD.
-//  * A and B k-tiles go from global memory straight into LDS (buffer loads
-//    with the LDS destination, 16 bytes a lane, eight 128-byte row pieces per
-//    instruction); two stages. Waves 0-3 issue all of the loads, so on every
-//    SIMD one of the two waves never waits on a load issue.
-//  * One barrier per k-tile, placed before the tile's last 16-deep slab: by
-//    then every wave holds its last-slab fragments in registers and has read
-//    all of the tile, so the barrier both publishes tile kt+1 (loaded during
-//    tile kt) and frees tile kt's stage for tile kt+2.
-//  * LDS rows are 64 elements (eight 16-byte chunks), chunk c of row r stored
-//    at c ^ ((r >> 1) & 7): the fragment reads of 16 consecutive rows hit
-//    distinct banks. A load places lane L's 16 bytes in slot L of its 1 KB,
-//    so the swizzle is applied on the global side (the lane filling slot
-//    (r, c) fetches chunk c ^ f(r)).
-//  * Rows past M or N and 8-element k chunks past K read as zero: the whole
-//    offset of every load is in its lane part, which the buffer range check
-//    covers, and chunks past K get an offset beyond the range.
-constexpr int GBM = 256, GBN = 256, GBK = 64, GTHREADS = 512;
-constexpr int kGemmLoadWaves = 4;  // waves 0..3 issue the LDS loads
-constexpr int kGemmLoadsPerWave = (GBM + GBN) / 8 / kGemmLoadWaves;  // 1 KB loads a load wave issues per tile
-
-typedef __attribute__((address_space(3))) void* gemm_lds_ptr;
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ int gswz(int row, int chunk) { return row * GBK + ((chunk ^ ((row >> 1) & 7)) << 3); }
-constexpr int gemm_vmcnt0() { return (7 << 4) | (15 << 8); }  // s_waitcnt vmcnt(0) alone
-
-template <bool kF16>
-__device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f32x16& c) {
-  if constexpr (kF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
-                                                   0);
-}
-
-// kBN: B is N-contiguous ([K][N], row stride ldb) instead of K-contiguous.
-// Its k-tile is then stored as 64 rows of 256 columns (512 bytes, chunk c of
-// row k at c ^ 4 (k & 3): the 32 lanes of a transposing read, 4 rows x 64
-// bytes, hit 64 distinct banks), and the B fragments come from transposing LDS
-// reads (ds_read_b64_tr_b16: lane j of a 16-lane group gets element j & 3
-// of the 8-byte pieces lanes 4 e + (j >> 2) address, e = 0..3; lanes
-// addressing 4 consecutive k rows x 16 columns return 4 consecutive k of
-// one column, half a fragment), so no transposed copy of B is made.
-template <bool kF16, int kOutBytes, bool kBN>
-__global__ void __launch_bounds__(GTHREADS, 1) gemm_nt_256(GemmParams p, const uint16_t* __restrict__ A,
-                                                            const uint16_t* __restrict__ B, void* __restrict__ C) {
-  constexpr int STAGE = (GBM + GBN) * GBK;  // elements per stage
-  __shared__ __attribute__((aligned(1024))) uint16_t smem[2 * STAGE];
-
-  const int tiles_m = (p.M + GBM - 1) / GBM, tiles_n = (p.N + GBN - 1) / GBN;
-  const int per_batch = tiles_m * tiles_n;
-  const int total = per_batch * p.batch;
-  int bid = blockIdx.x;
-  if (total % 8 == 0) bid = (bid % 8) * (total / 8) + bid / 8;  // contiguous tile runs per XCD
-  const int b = bid / per_batch;
-  const int t = bid - b * per_batch;
-  const int group = 8;  // walk 8 tile-rows at a time so B k-tiles are reused from L2
-  const int gsize = group * tiles_n;
-  const int g = t / gsize;
-  const int first_m = g * group;
-  const int gm = min(tiles_m - first_m, group);
-  const int tm = first_m + (t - g * gsize) % gm;
-  const int tn = (t - g * gsize) / gm;
-  const int m0 = tm * GBM, n0 = tn * GBN;
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2, wn = wave & 3;
-
-  // Buffer resources over this tile's row panels; the range ends with the
-  // last valid row's K elements.
-  const uint16_t* Ap = A + (int64_t)b * p.a_batch_stride + (int64_t)m0 * p.lda;
-  const uint16_t* Bp = B + (int64_t)b * p.b_batch_stride + (kBN ? (int64_t)n0 : (int64_t)n0 * p.ldb);
-  const int rows_a = min(GBM, p.M - m0), rows_b = min(GBN, p.N - n0);
-  const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(Ap), 0, (int)(((int64_t)(rows_a - 1) * p.lda + p.K) * 2), 0x00020000);
-  // N-contiguous B: the range ends with row K-1's last valid column, so k
-  // rows past K read as zero; columns past N are masked per load below.
-  const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(Bp), 0,
-      kBN ? (int)(((int64_t)(p.K - 1) * p.ldb + rows_b) * 2) : (int)(((int64_t)(rows_b - 1) * p.ldb + p.K) * 2),
-      0x00020000);
-  const int nk = (p.K + GBK - 1) / GBK;
-  const int ktail = p.K - (nk - 1) * GBK;  // valid elements of the last k-tile
-
-  // Load lanes: load i of load wave w fills stage rows (4 i + w) * 8 + L / 8,
-  // slot L % 8; its global chunk is (L % 8) ^ f(row), and f depends only on
-  // row % 16 = 8 (w % 2) + L / 8.
-  const int lrow = lane >> 3, lslot = lane & 7;
-  const int lchunk = lslot ^ ((((wave & 1) * 8 + lrow) >> 1) & 7);
-  const uint32_t tail_oob = lchunk * 8 >= ktail ? 0x80000000u : 0u;  // beyond the range of any resource
-  uint32_t aoff[kGemmLoadsPerWave / 2], boff[kGemmLoadsPerWave / 2];
-#pragma unroll
-  for (int i = 0; i < kGemmLoadsPerWave / 2; ++i) {
-    const int row = (i * kGemmLoadWaves + wave) * 8 + lrow;
-    aoff[i] = (uint32_t)(row * p.lda * 2 + lchunk * 16);
-    if constexpr (kBN) {
-      // Load i of load wave w fills k rows 2 (4 i + w) + L / 32, slot L % 32
-      // (global chunk (L % 32) ^ 4 (k & 3)); chunks past N get an offset
-      // beyond the range.
-      const int krow = (i * kGemmLoadWaves + wave) * 2 + (lane >> 5);
-      const int chunk = (lane & 31) ^ ((krow & 3) << 2);
-      boff[i] = (uint32_t)(krow * p.ldb * 2 + chunk * 16) | (chunk * 8 >= rows_b ? 0x80000000u : 0u);
-    } else {
-      boff[i] = (uint32_t)(row * p.ldb * 2 + lchunk * 16);
-    }
-  }
-  auto load_tile = [&](int kt, int stage) {
-    uint16_t* st = smem + stage * STAGE;
-    const uint32_t kb = (uint32_t)(kt * GBK * 2);
-    const uint32_t oob = kt == nk - 1 ? tail_oob : 0u;
-#pragma unroll
-    for (int i = 0; i < kGemmLoadsPerWave / 2; ++i) {
-      const int row = (i * kGemmLoadWaves + wave) * 8;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (gemm_lds_ptr)(st + row * GBK), 16, (aoff[i] + kb) | oob, 0, 0, 0);
-    }
-    if constexpr (kBN) {
-      const uint32_t kr = (uint32_t)(kt * GBK * p.ldb * 2);
-#pragma unroll
-      for (int i = 0; i < kGemmLoadsPerWave / 2; ++i) {
-        const int krow = (i * kGemmLoadWaves + wave) * 2;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (gemm_lds_ptr)(st + GBM * GBK + krow * GBN), 16, boff[i] + kr, 0,
-                                                 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kGemmLoadsPerWave / 2; ++i) {
-        const int row = (i * kGemmLoadWaves + wave) * 8;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (gemm_lds_ptr)(st + (GBM + row) * GBK), 16,
-                                                 (boff[i] + kb) | oob, 0, 0, 0);
-      }
-    }
-  };
-
-  // Fragments of v_mfma_f32_32x32x16: lane L holds row L % 32 of a 32-row
-  // block, k chunk 2 s + L / 32 of slab s; f(row) = f(L % 32).
-  const int fr = lane & 31, fh = lane >> 5;
-  int loff[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) loff[s] = gswz(fr, 2 * s + fh);
-  // N-contiguous B: lane L (16-lane group g = L / 16, e = (L % 16) / 4,
-  // c = L % 4) of transposing read h addresses k row 16 s + 8 (g / 2) + 4 h +
-  // e, columns wn 64 + 32 j + 16 (g % 2) + 4 c .. + 3.
-  int troff[4][2][2];
-  if constexpr (kBN) {
-    const int g4 = lane >> 4, e4 = (lane >> 2) & 3, c4 = lane & 3;
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int k = 16 * s + 8 * (g4 >> 1) + 4 * h + e4;
-          const int chunk = wn * 8 + 4 * j + 2 * (g4 & 1) + (c4 >> 1);
-          troff[s][h][j] = k * GBN + ((chunk ^ ((k & 3) << 2)) << 3) + 4 * (c4 & 1);
-        }
-  }
-  u32x4 fa[2][4], fb[2][2];
-  auto read_b = [&](const uint16_t* stb, int s, int j) -> u32x4 {
-    if constexpr (kBN) {
-      typedef short v4i16 __attribute__((ext_vector_type(4)));
-      typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-      typedef __attribute__((address_space(3))) uint16_t lds_u16;
-      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)((lds_u16*)(stb + troff[s][0][j])));
-      const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)((lds_u16*)(stb + troff[s][1][j])));
-      typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-      const u32x2_t l2 = __builtin_bit_cast(u32x2_t, lo), h2 = __builtin_bit_cast(u32x2_t, hi);
-      return u32x4{l2[0], l2[1], h2[0], h2[1]};
-    } else {
-      return *reinterpret_cast<const u32x4*>(stb + (wn * 64 + 32 * j) * GBK + loff[s]);
-    }
-  };
-  auto read_slab = [&](int stage, int s, int buf) {
-    const uint16_t* as = smem + stage * STAGE + (wm * 128) * GBK;
-    const uint16_t* stb = smem + stage * STAGE + GBM * GBK;
-    // In the order the MFMAs first use them.
-    fa[buf][0] = *reinterpret_cast<const u32x4*>(as + loff[s]);
-    fb[buf][0] = read_b(stb, s, 0);
-    fb[buf][1] = read_b(stb, s, 1);
-#pragma unroll
-    for (int i = 1; i < 4; ++i) fa[buf][i] = *reinterpret_cast<const u32x4*>(as + i * 32 * GBK + loff[s]);
-  };
-  f32x16 acc[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  auto mma = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma32<kF16>(fa[buf][i], fb[buf][j], acc[i][j]);
-  };
-  // One MFMA, then one fragment read, for each read of the slab; then the
-  // remaining MFMAs.
-  auto interleave_reads = [&]() {
-    constexpr int kReads = kBN ? 8 : 6;
-#pragma unroll
-    for (int q = 0; q < kReads; ++q) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    if constexpr (kReads < 8) __builtin_amdgcn_sched_group_barrier(0x008, 8 - kReads, 0);
-  };
-
-  // Tile kt: slabs 0..2 read the next slab's fragments while multiplying;
-  // then the barrier; then tile kt+1's first slab is read and tile kt+2's
-  // loads issued while the last slab multiplies. Tile indices past the last
-  // reload it into the free stage, so the load waves' counts stay uniform.
-  auto tile_body = [&](int kt, bool last, auto loader) {
-    constexpr bool kLoads = decltype(loader)::value;
-    const int cur = kt & 1;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      read_slab(cur, s + 1, (s + 1) & 1);
-      mma(s & 1);
-      interleave_reads();
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (!last) {
-      // Own loads of tile kt+1 landed and own reads of tile kt done, then
-      // everyone's.
-      __builtin_amdgcn_s_waitcnt(gemm_vmcnt0() & ~(15 << 8));
-      __builtin_amdgcn_s_barrier();
-      read_slab(cur ^ 1, 0, 0);
-      if constexpr (kLoads) load_tile(min(kt + 2, nk - 1), cur);
-    }
-    mma(1);
-    interleave_reads();
-    if constexpr (kLoads) {
-#pragma unroll
-      for (int q = 0; q < kGemmLoadsPerWave; ++q) {
-        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto run = [&](auto loader) {
-    constexpr bool kLoads = decltype(loader)::value;
-    if constexpr (kLoads) {
-      load_tile(0, 0);
-      load_tile(min(1, nk - 1), 1);
-      __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8) | (kGemmLoadsPerWave & 15) | ((kGemmLoadsPerWave >> 4) << 14));
-    }
-    __builtin_amdgcn_s_barrier();
-    read_slab(0, 0, 0);
-    for (int kt = 0; kt < nk - 1; ++kt) tile_body(kt, false, loader);
-    tile_body(nk - 1, true, loader);
-  };
-  if (wave < kGemmLoadWaves) run(std::true_type{});
-  else run(std::false_type{});
-  __builtin_amdgcn_s_waitcnt(gemm_vmcnt0());
-  __syncthreads();
-
-  // Epilogue: lane L holds rows 8 (r / 4) + 4 (L / 32) + r % 4, column L % 32
-  // of each 32 x 32 block.
-  const int wrow0 = m0 + wm * 128, wcol0 = n0 + wn * 64;
-  if constexpr (kOutBytes == 2) {
-    uint16_t* cs = smem + wave * 128 * GBK;  // this wave's 128 x 64 staging tile
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = i * 32 + (r >> 2) * 8 + fh * 4 + (r & 3);
-          const int col = j * 32 + fr;
-          const float v = acc[i][j][r];
-          cs[gswz(row, col >> 3) + (col & 7)] = kF16 ? f32_to_f16_bits(v) : f32_to_bf16_rne(v);
-        }
-    __syncthreads();
-    uint16_t* Cb = reinterpret_cast<uint16_t*>(C) + (int64_t)b * p.M * p.ldc;
-#pragma unroll
-    for (int tt = 0; tt < 16; ++tt) {
-      const int c = lane + 64 * tt;  // 1024 chunks of 8
-      const int row = c >> 3, ch = c & 7;
-      const int m = wrow0 + row, n = wcol0 + ch * 8;
-      if (m >= p.M || n >= p.N) continue;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(&cs[gswz(row, ch)]);
-      if (n + 8 <= p.N && p.ldc % 8 == 0) {
-        *reinterpret_cast<u32x4*>(Cb + (int64_t)m * p.ldc + n) = v;
-      } else {
-        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
-        for (int q = 0; q < 8 && n + q < p.N; ++q) Cb[(int64_t)m * p.ldc + n + q] = e[q];
-      }
-    }
-  } else {
-    float* Cb = reinterpret_cast<float*>(C) + (int64_t)b * p.M * p.ldc;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = wrow0 + i * 32 + (r >> 2) * 8 + fh * 4 + (r & 3);
-          const int n = wcol0 + j * 32 + fr;
-          if (m < p.M && n < p.N) Cb[(int64_t)m * p.ldc + n] = acc[i][j][r];
-        }
-  }
-}
-
-// out[b][c][r] = in[b][r][c] for 16-bit elements; 64 x 64 tiles through LDS.
-__global__ void __launch_bounds__(256) transpose16(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
-                                                   int64_t rows, int64_t cols, int64_t in_bs, int64_t out_bs) {
-  __shared__ uint16_t tile[64][66];
-  const int64_t b = blockIdx.z;
-  const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
-  const uint16_t* src = in + b * in_bs;
-  uint16_t* dst = out + b * out_bs;
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int c = tid + 256 * j;  // 512 chunks of 8
-    const int rr = c >> 3, cc = (c & 7) * 8;
-    const int64_t r = r0 + rr, col = c0 + cc;
-    uint16_t v[8];
-    if (r < rows && col + 8 <= cols && cols % 8 == 0) {
-      *reinterpret_cast<u32x4*>(v) = *reinterpret_cast<const u32x4*>(src + r * cols + col);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (r < rows && col + e < cols) ? src[r * cols + col + e] : (uint16_t)0;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) tile[rr][cc + e] = v[e];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int c = tid + 256 * j;
-    const int oc = c >> 3, orr = (c & 7) * 8;  // output row = input column
-    const int64_t orow = c0 + oc, ocol = r0 + orr;
-    if (orow >= cols) continue;
-    uint16_t v[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = tile[orr + e][oc];
-    if (ocol + 8 <= rows && rows % 8 == 0) {
-      *reinterpret_cast<u32x4*>(dst + orow * rows + ocol) = *reinterpret_cast<const u32x4*>(v);
-    } else {
-      for (int e = 0; e < 8 && ocol + e < rows; ++e) dst[orow * rows + ocol + e] = v[e];
-    }
   }
 }
 
@@ -889,50 +538,8 @@ void check(const char* what) {
 
 }  // namespace
 
-bool use_big_gemm(const GemmParams& p, bool b_kmajor) {
-  // Below one tile per CU the 128 x 128 kernel's 4x more tiles fill the GPU
-  // better (environment: PJRTX_BIG_GEMM_MIN_TILES).
-  const int64_t min_tiles = env_int("PJRTX_BIG_GEMM_MIN_TILES", 256);
-  const int64_t tiles = (int64_t)((p.M + GBM - 1) / GBM) * ((p.N + GBN - 1) / GBN) * p.batch;
-  // Every load offset (a 256-row panel of A, a panel or all K rows of B)
-  // must stay below 2^31 bytes.
-  const int64_t limit = int64_t(1) << 30;
-  const bool b_ok = b_kmajor ? (p.ldb >= p.K && (int64_t)GBN * p.ldb < limit)
-                             : (p.N % 8 == 0 && p.ldb >= p.N && (int64_t)p.K * p.ldb < limit);
-  return p.M >= GBM && p.N >= GBN && p.K > 0 && p.K % 8 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 &&
-         p.lda >= p.K && b_ok && p.a_batch_stride % 8 == 0 && p.b_batch_stride % 8 == 0 && tiles >= min_tiles &&
-         tiles < (int64_t(1) << 31) && (int64_t)GBM * p.lda < limit;
-}
-
-void launch_transpose16(hipStream_t s, const void* in, void* out, int64_t batch, int64_t rows, int64_t cols,
-                        int64_t in_bs, int64_t out_bs) {
-  if (batch == 0 || rows == 0 || cols == 0) return;
-  const dim3 grid(static_cast<unsigned>((cols + 63) / 64), static_cast<unsigned>((rows + 63) / 64),
-                  static_cast<unsigned>(batch));
-  hipLaunchKernelGGL(transpose16, grid, dim3(256), 0, s, static_cast<const uint16_t*>(in), static_cast<uint16_t*>(out),
-                     rows, cols, in_bs, out_bs);
-  check("transpose16");
-}
-
 void launch_mfma_gemm(hipStream_t s, const GemmParams& p, const void* A, const void* B, void* C, bool f16, bool b_kmajor,
                       int out_bytes) {
-  if (use_big_gemm(p, b_kmajor)) {
-    const int64_t tiles = (int64_t)((p.M + GBM - 1) / GBM) * ((p.N + GBN - 1) / GBN) * p.batch;
-    const dim3 grid(static_cast<unsigned>(tiles)), block(GTHREADS);
-    const uint16_t* a = static_cast<const uint16_t*>(A);
-    const uint16_t* b = static_cast<const uint16_t*>(B);
-#define PJRTX_BIG(F16, OB, BN) hipLaunchKernelGGL((gemm_nt_256<F16, OB, BN>), grid, block, 0, s, p, a, b, C)
-    if (out_bytes == 2) {
-      if (f16) { if (b_kmajor) PJRTX_BIG(true, 2, false); else PJRTX_BIG(true, 2, true); }
-      else { if (b_kmajor) PJRTX_BIG(false, 2, false); else PJRTX_BIG(false, 2, true); }
-    } else {
-      if (f16) { if (b_kmajor) PJRTX_BIG(true, 4, false); else PJRTX_BIG(true, 4, true); }
-      else { if (b_kmajor) PJRTX_BIG(false, 4, false); else PJRTX_BIG(false, 4, true); }
-    }
-#undef PJRTX_BIG
-    check("gemm_nt_256");
-    return;
-  }
   const int64_t tiles = (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * p.batch;
   if (tiles == 0 || p.K == 0) fail(Code::kInternal, "mfma_gemm: empty problem must be handled by the caller");
   PJRTX_CHECK(tiles < (int64_t(1) << 31), Code::kUnimplemented, "mfma_gemm: too many tiles");
