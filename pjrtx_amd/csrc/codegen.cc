@@ -807,7 +807,7 @@ void KernelGen::loop(Step& s) {
 
 void KernelGen::reduce(Step& s) {
   std::map<int, std::string> ptr_of;
-  const bool split = s.row_schedule && s.splits > 1;
+  const bool split = s.splits > 1;
   signature(s, &ptr_of, split);
   const std::string it = idx_type(s);
   out_ << "typedef " << it << " idx_t;\n";
@@ -843,11 +843,12 @@ void KernelGen::reduce(Step& s) {
   root.key = "R";
   root.shape = shape;
   root.lin = "lin";
-  root.identity = s.row_schedule;
+  root.identity = s.row_schedule || s.col_lanes > 0;
   root.multi.resize(rank);
   const int vec = s.vec;
 
   std::ostringstream head;  // before the element loop
+  std::string close_fold;              // closes what the column schedule's epilogue sits in
   bool epilogue_then_combine = false;  // fused combine: also emit the `_combine` fallback kernel
   std::string combine_fallback_body;
   if (s.row_schedule) {
@@ -884,17 +885,31 @@ void KernelGen::reduce(Step& s) {
       --k;
     }
   } else {
-    head << "const idx_t row = (idx_t)blockIdx.x * 256u + threadIdx.x;\n";
-    head << "if (row >= " << s.rows << "u) return;\n";
     std::string rest = "row";
+    if (s.col_lanes) {
+      const int64_t span = static_cast<int64_t>(s.col_lanes) * vec, blocks = (s.rows + span - 1) / span;
+      head << "const idx_t cb = (idx_t)blockIdx.x % " << blocks << "u, split = (idx_t)blockIdx.x / " << blocks << "u;\n";
+      head << "const uint32_t tx = threadIdx.x % " << s.col_lanes << "u, ty = threadIdx.x / " << s.col_lanes << "u;\n";
+      // Lanes past the last output walk no element (rows is a multiple of vec).
+      head << "const bool live = cb * " << span << "u + tx * " << vec << "u < " << s.rows << "u;\n";
+      head << "const idx_t row0 = live ? cb * " << span << "u + tx * " << vec << "u : 0u;\n";
+      head << "const idx_t c0 = split * " << s.chunk << "u;\n";
+      head << "const idx_t c1 = !live ? c0 : (c0 + " << s.chunk << "u < " << s.row_len << "u) ? c0 + " << s.chunk << "u : "
+           << s.row_len << "u;\n";
+      rest = "row0";
+    } else {
+      head << "const idx_t row = (idx_t)blockIdx.x * 256u + threadIdx.x;\n";
+      head << "if (row >= " << s.rows << "u) return;\n";
+    }
     for (int d = rank - 1, k = static_cast<int>(kept_dims.size()) - 1; d >= 0; --d) {
       if (is_red(d)) continue;
+      const std::string plus = s.col_lanes && d == rank - 1 ? " + j" : "";
       if (k == 0) {
-        root.multi[d] = rest;
+        root.multi[d] = "(" + rest + plus + ")";
       } else {
         head << "const idx_t kd" << d << " = " << rest << " % " << shape[d] << "u;\n";
         head << "const idx_t kq" << d << " = " << rest << " / " << shape[d] << "u;\n";
-        root.multi[d] = "kd" + std::to_string(d);
+        root.multi[d] = "(kd" + std::to_string(d) + plus + ")";
         rest = "kq" + std::to_string(d);
       }
       --k;
@@ -945,6 +960,16 @@ void KernelGen::reduce(Step& s) {
     }
     if (s.row_len % vec != 0 || s.chunk % vec != 0)
       fail(Code::kInternal, "reduce kernel: row length and chunk must be multiples of the vector width");
+  } else if (s.col_lanes) {
+    const int64_t n_all = num_elements(shape);
+    for (int v : s.inputs) {
+      if (prog_.type(v).elements() != n_all) continue;
+      const std::string name = "pre_" + ptr_of[v];
+      pre_decl << dtype_storage_ctype(prog_.type(v).dtype) << " " << name << "[" << unroll << "][" << vec << "];\n";
+      // The last dim and so every output group is a multiple of vec.
+      pre_load << ldv_of(v, vec, true) << "(" << name << "[u], " << ptr_of[v] << ", lin, 0u, true);\n";
+      w.preload[v] = "P_" + ptr_of[v];
+    }
   }
   // f32 sums of f16 values (JAX's f16 sum: convert f16->f32, add) fold each
   // element with one mixed-precision FMA on the f16 value (add_f16v), or, in
@@ -986,6 +1011,7 @@ void KernelGen::reduce(Step& s) {
 
   out_ << head.str();
   for (auto& a : accs) {
+    if (s.col_lanes) break;
     out_ << a.acc_t << " " << a.v << " = " << identity_of(a.kind, a.vt, a.acc_t) << ";\n";
     if (a.kind == ReducerKind::kArgMax || a.kind == ReducerKind::kArgMin)
       out_ << ait << " " << a.i << " = " << aimax << ";\n";
@@ -1453,6 +1479,112 @@ void KernelGen::reduce(Step& s) {
     } else {
       out_ << "if (threadIdx.x != 0) return;\n";
     }
+  } else if (s.col_lanes) {
+    // Column schedule, last dim kept: a thread owns vec neighbouring outputs
+    // (one 16-byte piece of every operand row it reads) and walks every
+    // lane-rows-th reduced element of its split, `unroll` loads in flight; the
+    // lane rows meet through LDS in lane-row order, the splits in a second
+    // launch in split order (deterministic). Bound by HBM: f32 sums over rows,
+    // [8192, 4096] 187 -> 26 us, [1048576, 16] 22.8 ms -> 27 us (one serial
+    // thread per output before).
+    const int lane_rows = 256 / s.col_lanes, span = s.col_lanes * vec;
+    const auto is_arg_kind = [](const Accum& a) { return a.kind == ReducerKind::kArgMax || a.kind == ReducerKind::kArgMin; };
+    std::string lin;
+    int64_t stride = 1;
+    for (int d = rank - 1; d >= 0; --d) {
+      if (shape[d] != 1) {
+        const std::string term =
+            stride == 1 ? "(" + root.multi[d] + ")" : "(" + root.multi[d] + ")*" + std::to_string(stride) + "u";
+        lin = lin.empty() ? term : term + " + " + lin;
+      }
+      stride *= shape[d];
+    }
+    if (lin.empty()) lin = "0";
+    for (auto& a : accs) {
+      out_ << a.acc_t << " ar_" << a.v << "[" << vec << "];\n";
+      if (is_arg_kind(a)) out_ << ait << " ar_" << a.i << "[" << vec << "];\n";
+      out_ << "#pragma unroll\nfor (int j = 0; j < " << vec << "; ++j) { ar_" << a.v << "[j] = "
+           << identity_of(a.kind, a.vt, a.acc_t) << ";";
+      if (is_arg_kind(a)) out_ << " ar_" << a.i << "[j] = " << aimax << ";";
+      out_ << " }\n";
+    }
+    out_ << pre_decl.str();
+    out_ << "for (idx_t c = c0 + ty; c < c1; c += " << lane_rows * unroll << "u) {\n";
+    // Unconditional loads: an element past the split re-reads its last one.
+    out_ << "#pragma unroll\nfor (int u = 0; u < " << unroll << "; ++u) {\n";
+    out_ << "const idx_t cu = c + (idx_t)u * " << lane_rows << "u;\nconst idx_t col = cu < c1 ? cu : c1 - 1u;\n";
+    out_ << "const int j = 0;\n" << col_digits.str() << "const idx_t lin = " << lin << ";\n" << pre_load.str() << "}\n";
+    out_ << "#pragma unroll\nfor (int u = 0; u < " << unroll << "; ++u) {\n";
+    out_ << "const idx_t col = c + (idx_t)u * " << lane_rows << "u;\n";
+    for (auto& [v, pname] : w.preload) out_ << "const auto& " << pname << " = pre_" << ptr_of[v] << "[u];\n";
+    out_ << "if (col < c1) {\n" << col_digits.str();
+    out_ << "#pragma unroll\nfor (int j = 0; j < " << vec << "; ++j) {\n";
+    for (auto& a : accs) {
+      out_ << a.acc_t << "& " << a.v << " = ar_" << a.v << "[j];\n";
+      if (is_arg_kind(a)) out_ << ait << "& " << a.i << " = ar_" << a.i << "[j];\n";
+    }
+    out_ << "const idx_t lin = " << lin << ";\n" << elem_body;
+    combine_elem(out_, 0);
+    out_ << "}\n}\n}\n}\n";
+    for (auto& a : accs) {
+      out_ << "__shared__ " << a.acc_t << " sm_" << a.v << "[" << lane_rows << "][" << span << "];\n";
+      if (is_arg_kind(a)) out_ << "__shared__ " << ait << " sm_" << a.i << "[" << lane_rows << "][" << span << "];\n";
+      out_ << "#pragma unroll\nfor (int j = 0; j < " << vec << "; ++j) { sm_" << a.v << "[ty][tx * " << vec << "u + j] = ar_"
+           << a.v << "[j];";
+      if (is_arg_kind(a)) out_ << " sm_" << a.i << "[ty][tx * " << vec << "u + j] = ar_" << a.i << "[j];";
+      out_ << " }\n";
+    }
+    out_ << "__syncthreads();\n";
+    out_ << "for (uint32_t o = threadIdx.x; o < " << span << "u; o += 256u) {\n";
+    out_ << "const idx_t row = cb * " << span << "u + o;\nif (row < " << s.rows << "u) {\n";
+    auto fold_one = [&](const Accum& a, const std::string& v, const std::string& i) {
+      if (is_arg_kind(a))
+        out_ << "if (" << arg_better(a.kind) << "(" << v << ", " << i << ", " << a.v << ", " << a.i << ")) { " << a.v << " = "
+             << v << "; " << a.i << " = " << i << "; }\n";
+      else
+        out_ << combine_stmt(a.kind, a.vt, a.v, v) << "\n";
+    };
+    for (auto& a : accs) {
+      out_ << a.acc_t << " " << a.v << " = sm_" << a.v << "[0][o];\n";
+      if (is_arg_kind(a)) out_ << ait << " " << a.i << " = sm_" << a.i << "[0][o];\n";
+      out_ << "#pragma unroll 4\nfor (int k = 1; k < " << lane_rows << "; ++k) {\n";
+      fold_one(a, "sm_" + a.v + "[k][o]", "sm_" + a.i + "[k][o]");
+      out_ << "}\n";
+    }
+    if (!split) {
+      close_fold = "}\n}\n";
+    } else {
+      // Partial slots, 8 bytes each: per reducer [splits][rows] (argmax:
+      // values, then indices).
+      const int64_t slots = s.rows * s.splits;
+      size_t off = 0;
+      std::ostringstream load;
+      for (auto& a : accs) {
+        out_ << "{ uint64_t* slot = reinterpret_cast<uint64_t*>(scratch + " << off << "u);\n";
+        out_ << "uint64_t bits = 0; __builtin_memcpy(&bits, &" << a.v << ", sizeof(" << a.v << "));\n";
+        out_ << "slot[split * " << s.rows << "u + row] = bits;\n";
+        if (is_arg_kind(a)) out_ << "slot[" << slots << "u + split * " << s.rows << "u + row] = (uint64_t)" << a.i << ";\n";
+        out_ << "}\n";
+        off += static_cast<size_t>(slots) * (is_arg_kind(a) ? 16 : 8);
+      }
+      out_ << "}\n}\n}\n\n";
+      signature(s, &ptr_of, true, "_combine");
+      out_ << "typedef " << it << " idx_t;\n";
+      out_ << "const idx_t row = (idx_t)blockIdx.x * 256u + threadIdx.x;\n";
+      out_ << "if (row >= " << s.rows << "u) return;\n";
+      off = 0;
+      for (auto& a : accs) {
+        out_ << a.acc_t << " " << a.v << " = " << identity_of(a.kind, a.vt, a.acc_t) << ";\n";
+        if (is_arg_kind(a)) out_ << ait << " " << a.i << " = " << aimax << ";\n";
+        out_ << "{ const uint64_t* slot = reinterpret_cast<const uint64_t*>(scratch + " << off << "u);\n";
+        out_ << "#pragma unroll 8\nfor (idx_t k = 0; k < " << s.splits << "u; ++k) {\n";
+        out_ << "const uint64_t bits = slot[k * " << s.rows << "u + row]; " << a.acc_t << " pv; __builtin_memcpy(&pv, &bits, sizeof(pv));\n";
+        if (is_arg_kind(a)) out_ << "const " << ait << " pi = (" << ait << ")slot[" << slots << "u + k * " << s.rows << "u + row];\n";
+        fold_one(a, "pv", "pi");
+        out_ << "}\n}\n";
+        off += static_cast<size_t>(slots) * (is_arg_kind(a) ? 16 : 8);
+      }
+    }
   } else {
     // Column schedule: one thread per output, serial walk of reduced elements.
     out_ << "for (idx_t col = 0; col < " << s.row_len << "u; ++col) {\n";
@@ -1523,7 +1655,7 @@ void KernelGen::reduce(Step& s) {
   epi << "{\n" << fin.str() << e.body.str();
   for (size_t o = 0; o < s.outputs.size(); ++o)
     epi << "out" << o << "[row] = " << to_storage(prog_.type(s.outputs[o]).dtype, outs[o]) << ";\n";
-  epi << "}\n}\n\n";
+  epi << "}\n" << close_fold << "}\n\n";
   out_ << epi.str();
   if (epilogue_then_combine) {
     // The `_combine` kernel of the fallback (fused_mode 0): one wavefront per

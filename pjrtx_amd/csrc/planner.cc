@@ -1178,11 +1178,54 @@ void Planner::shape_reduce(Step* s) {
   s->rows = rows;
   s->row_len = row_len;
   // Row schedule needs enough work per row to fill a workgroup; otherwise a
-  // thread per output walks its reduced elements serially.
+  // thread per output walks its reduced elements serially, or, when the last
+  // dim is kept, a workgroup's lanes span outputs and its lane rows and the
+  // splits share the reduced elements.
   s->row_schedule = trailing && row_len >= 64;
   if (!s->row_schedule) {
     s->vec = 1;
     s->splits = 1;
+    if (rank > 0 && nred > 0 && s->reduce_dims.back() != rank - 1 && rows > 0 && row_len >= 32) {
+      size_t min_size = 8, slot = 0;
+      for (int v : s->inputs)
+        if (prog_.type(v).elements() == num_elements(shape)) min_size = std::min(min_size, dtype_size(prog_.type(v).dtype));
+      for (const ReduceSpec& r : s->reduces) slot += (r.kind == ReducerKind::kArgMax || r.kind == ReducerKind::kArgMin) ? 16 : 8;
+      int vec = std::max(1, std::min(8, static_cast<int>(16 / min_size)));
+      while (vec > 1 && (shape[rank - 1] % vec != 0 || 256 * vec * slot > 48 * 1024)) vec /= 2;
+      int lanes = 1;
+      while (lanes < 64 && lanes * vec < rows) lanes *= 2;
+      const auto blocks_of = [&](int l) { return (rows + l * vec - 1) / (l * vec); };
+      const auto per_thread = [&](int l) { return (row_len + 256 / l - 1) / (256 / l); };
+      // One launch while a thread walks at most 32 elements (four batches of
+      // loads): a second one costs 2 us ([128, 4096] f32 6.4 us with splits,
+      // 4.3 in one launch). Eight lanes still read whole 128-byte lines;
+      // fewer lanes a row, more workgroups and fewer elements a thread.
+      // Longer columns take 1 KB row pieces and split.
+      int one = lanes;
+      while (one > 8 && (blocks_of(one) < 256 || per_thread(one) > 32)) one /= 2;
+      if (per_thread(one) <= 32) lanes = one;
+      if (256 * vec * slot <= 48 * 1024) {
+        const int64_t blocks = blocks_of(lanes);
+        int64_t splits = 1;
+        if (per_thread(lanes) > 32)
+          splits = std::max<int64_t>(1, std::min<int64_t>({(opts_.reduce_target_blocks + blocks - 1) / blocks,
+                                                           per_thread(lanes) / 4, 64}));
+        const int64_t chunk = (row_len + splits - 1) / splits;
+        splits = (row_len + chunk - 1) / chunk;
+        s->vec = vec;
+        s->col_lanes = lanes;
+        s->splits = splits;
+        s->chunk = chunk;
+        s->unroll = 8;
+        s->grid = static_cast<uint32_t>(blocks * splits);
+        s->block = 256;
+        if (splits > 1) {
+          s->scratch_bytes = static_cast<size_t>(rows * splits) * slot;
+          s->combine_grid = static_cast<uint32_t>((rows + 255) / 256);
+        }
+        return;
+      }
+    }
     s->grid = static_cast<uint32_t>(std::max<int64_t>(1, (rows + 255) / 256));
     s->block = 256;
     return;
