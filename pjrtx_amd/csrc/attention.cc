@@ -432,6 +432,7 @@ void rewrite_program(Program* prog) {
       if (m.try_rewrite(static_cast<int>(i))) changed = true;
     }
   }
+  changed |= fold_dot_transpose(prog);
   if (changed) remove_dead_ops(prog);
 }
 

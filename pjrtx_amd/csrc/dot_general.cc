@@ -6,6 +6,7 @@
 // [batch][K][cols] with uniform strides when its dimension groups can be
 // merged; otherwise it is first copied into that canonical layout.
 #include <algorithm>
+#include <map>
 
 #include "blaslt.h"
 #include "kernels/dot.h"
@@ -120,7 +121,10 @@ int single_wide_tiles(int64_t N) {
   return gemv_wide_tiles(one);
 }
 
-void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals) {
+// Writes the product to the dot's result, plus `add` (GemmMember::add, its
+// row stride add_ld) where the block tiles run it; returns whether they did.
+bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, const void* add,
+                     int64_t add_ld) {
   const TensorType& lt = prog.type(op.operands[0]);
   const TensorType& rt = prog.type(op.operands[1]);
   const TensorType& ot = prog.type(op.results[0]);
@@ -138,14 +142,14 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
   OperandView b = view_of(rt, op.rhs_batch, op.rhs_contract);
   const int64_t batch = a.batch, M = a.free, N = b.free, K = a.k;
   void* out = vals[op.results[0]]->ptr;
-  if (ot.elements() == 0) return;
+  if (ot.elements() == 0) return true;
   const void* A = vals[op.operands[0]]->ptr;
   const void* B = vals[op.operands[1]]->ptr;
   const bool low_precision = lt.dtype == DType::kBF16 || lt.dtype == DType::kF16;
   const bool out_ok = ot.dtype == lt.dtype || ot.dtype == DType::kF32;
   if (K == 0) {  // empty contraction: zeros
     launch_zero(dev->stream(), out, ot.elements() * static_cast<int64_t>(dtype_size(ot.dtype)));
-    return;
+    return false;
   }
   if (low_precision && out_ok) {
     const bool f16 = lt.dtype == DType::kF16;
@@ -209,7 +213,7 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
         g.m[0].ldw = b.ks ? b.ks : N;
         g.m[0].ldy = N;
         launch_gemv_wide(dev->stream(), g, A, f16);
-        return;
+        return false;
       }
       GemvParams g;
       g.batch = static_cast<int>(batch);
@@ -233,7 +237,7 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
       }
       if (room) {
         launch_gemv(dev->stream(), g, A, B, out, part ? static_cast<float*>(part->ptr) : nullptr, f16, b_kmajor);
-        return;
+        return false;
       }
     }
     if (ready && !aligned_rows(A, a, a_kmajor)) ready = pad(&A, &a, a_kmajor, &a_pad);
@@ -253,20 +257,34 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
       g.b_batch_stride = batch == 1 ? 0 : b.bs;
       if (a_kmajor && K % 8 == 0 && (b_kmajor || N % 8 == 0) && blaslt_wanted(g) &&
           blaslt_gemm(dev, g, A, B, out, f16, b_kmajor, out_kind == 2 ? 4 : 2))
-        return;
-      if (gemm_fits(g, a_kmajor, b_kmajor)) {
+        return false;
+      GemmGroup gg;
+      gg.batch = g.batch;
+      gg.M = g.M;
+      gg.K = g.K;
+      gg.lda = g.lda;
+      gg.a_batch_stride = g.a_batch_stride;
+      gg.m[0].B = B;
+      gg.m[0].C = out;
+      gg.m[0].N = g.N;
+      gg.m[0].ldb = g.ldb;
+      gg.m[0].b_batch_stride = g.b_batch_stride;
+      const bool fuse = add && out_kind != 2 && aligned16(add) && aligned16(out);
+      if (fuse) gg.m[0].add = add;
+      gg.m[0].add_ld = add_ld;
+      if (gemm_fits(gg, a_kmajor, b_kmajor)) {
         // Partials of a k-split: at most 64 MiB, and what a fixed block has left.
         const int64_t left = std::max<int64_t>(0, std::min<int64_t>(int64_t(64) << 20, scratch_left(dev) - 4096));
-        const GemmPlan plan = plan_gemm(g, left);
+        const GemmPlan plan = plan_gemm(gg, left);
         MemRef ws;
         if (plan.workspace) ws = dev->allocate(plan.workspace);
-        launch_gemm(dev->stream(), g, plan, A, a_kmajor, B, b_kmajor, out, f16, out_kind == 2 ? 4 : 2,
+        launch_gemm(dev->stream(), gg, plan, A, a_kmajor, b_kmajor, f16, out_kind == 2 ? 4 : 2,
                     ws ? static_cast<float*>(ws->ptr) : nullptr);
-        return;
+        return fuse;
       }
       if (a_kmajor && K % 8 == 0 && (b_kmajor || N % 8 == 0)) {
         launch_mfma_gemm(dev->stream(), g, A, B, out, f16, b_kmajor, out_kind == 2 ? 4 : 2);
-        return;
+        return false;
       }
     }
   }
@@ -295,18 +313,21 @@ void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
   f.b_ns = b.fs;
   f.b_ks = b.ks;
   launch_fma_gemm(dev->stream(), f, A, B, out, lt.dtype, ot.dtype);
+  return false;
 }
 
 // A dot whose result only feeds `add(dot, x)`: out = x + round(dot) as the
 // one-pass GEMV's epilogue, or, when that kernel does not apply to these
 // buffers, the dot into a temporary followed by the elementwise add.
-void run_dot_residual(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, int add, int out) {
+// `row`: x is one row added to every row of the product (a bias).
+void run_dot_residual(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, int add, int out,
+                      bool row) {
   const TensorType& lt = prog.type(op.operands[0]);
   const TensorType& rt = prog.type(op.operands[1]);
   const TensorType& ot = prog.type(op.results[0]);
   const void* A = vals[op.operands[0]]->ptr;
   const void* W = vals[op.operands[1]]->ptr;
-  const bool ok = lt.rank() == 2 && rt.rank() == 2 && op.lhs_batch.empty() && op.lhs_contract == Dims{1} &&
+  const bool ok = !row && lt.rank() == 2 && rt.rank() == 2 && op.lhs_batch.empty() && op.lhs_contract == Dims{1} &&
                   op.rhs_contract == Dims{0} && (lt.dtype == DType::kBF16 || lt.dtype == DType::kF16) &&
                   rt.dtype == lt.dtype && ot.dtype == lt.dtype && lt.dims[1] % 8 == 0 && rt.dims[1] % 8 == 0 &&
                   aligned16(W) && rt.dims[1] < (int64_t(1) << 30) &&
@@ -327,16 +348,68 @@ void run_dot_residual(Device* dev, const Program& prog, const Op& op, std::vecto
     launch_gemv_wide(dev->stream(), g, A, lt.dtype == DType::kF16);
     return;
   }
+  if (ot.dtype == DType::kBF16 || ot.dtype == DType::kF16) {
+    // The block tiles add in their epilogue; any other kernel's product is
+    // added to in place.
+    const int64_t n = row ? prog.type(add).elements() : ot.dims.empty() ? 1 : ot.dims.back();
+    vals[op.results[0]] = vals[out];
+    const bool added = run_dot_general(dev, prog, op, vals, vals[add]->ptr, row ? 0 : n);
+    vals[op.results[0]].reset();
+    if (!added && n > 0)
+      launch_add_rows16(dev->stream(), vals[out]->ptr, vals[add]->ptr, ot.elements() / n, n, row ? 0 : n,
+                        ot.dtype == DType::kF16);
+    return;
+  }
   vals[op.results[0]] = dev->allocate(ot.bytes());
-  run_dot_general(dev, prog, op, vals);
+  run_dot_general(dev, prog, op, vals, nullptr, 0);
   launch_add(dev->stream(), vals[add]->ptr, vals[op.results[0]]->ptr, vals[out]->ptr, ot.elements(), ot.dtype);
   vals[op.results[0]].reset();
+}
+
+// A group of more than 8 rows as one launch of the block tiles (the members'
+// tile columns side by side fill the GPU better than each alone); false when
+// they do not take some member's layout.
+static bool run_gemm_group(Device* dev, const Program& prog, const std::vector<int>& ops, std::vector<MemRef>& vals) {
+  const Op& first = prog.ops.at(ops.at(0));
+  const TensorType& lt = prog.type(first.operands[0]);
+  if (ops.size() > static_cast<size_t>(kMaxGemmMembers) || lt.rank() != 2 || lt.dims[0] <= 8 || lt.dims[1] == 0) return false;
+  const void* A = vals[first.operands[0]]->ptr;
+  const DType ot = prog.type(first.results[0]).dtype;
+  if ((lt.dtype != DType::kBF16 && lt.dtype != DType::kF16) || (ot != lt.dtype && ot != DType::kF32)) return false;
+  GemmGroup g;
+  g.M = static_cast<int>(lt.dims[0]);
+  g.K = static_cast<int>(lt.dims[1]);
+  g.lda = lt.dims[1];
+  g.count = static_cast<int>(ops.size());
+  if (!aligned16(A) || lt.dims[1] % 8 != 0) return false;
+  for (size_t i = 0; i < ops.size(); ++i) {
+    const Op& op = prog.ops.at(ops[i]);
+    const TensorType& rt = prog.type(op.operands[1]);
+    const void* B = vals[op.operands[1]]->ptr;
+    void* C = vals[op.results[0]]->ptr;
+    if (op.operands[0] != first.operands[0] || rt.rank() != 2 || op.lhs_contract != Dims{1} || op.rhs_contract != Dims{0} ||
+        rt.dtype != lt.dtype || prog.type(op.results[0]).dtype != ot || rt.dims[1] % 8 != 0 || !aligned16(B) || !aligned16(C))
+      return false;
+    g.m[i].B = B;
+    g.m[i].C = C;
+    g.m[i].N = static_cast<int>(rt.dims[1]);
+    g.m[i].ldb = rt.dims[1];
+  }
+  if (!gemm_fits(g, true, false)) return false;
+  const int64_t left = std::max<int64_t>(0, std::min<int64_t>(int64_t(64) << 20, scratch_left(dev) - 4096));
+  const GemmPlan plan = plan_gemm(g, left);
+  MemRef ws;
+  if (plan.workspace) ws = dev->allocate(plan.workspace);
+  launch_gemm(dev->stream(), g, plan, A, true, false, lt.dtype == DType::kF16, ot == DType::kF32 ? 4 : 2,
+              ws ? static_cast<float*>(ws->ptr) : nullptr);
+  return true;
 }
 
 // A dot group (planner: dots sharing one LHS): one gemv_wide launch when
 // every member is a decode-shaped product over the same X with an
 // N-contiguous weight; otherwise the members run one by one.
 void run_dot_group(Device* dev, const Program& prog, const std::vector<int>& ops, std::vector<MemRef>& vals) {
+  if (run_gemm_group(dev, prog, ops, vals)) return;
   GemvGroup g;
   bool ok = ops.size() >= 1 && ops.size() <= static_cast<size_t>(kMaxGemvMembers);
   const void* X = nullptr;
@@ -383,7 +456,51 @@ void run_dot_group(Device* dev, const Program& prog, const std::vector<int>& ops
     launch_gemv_wide(dev->stream(), g, X, in_t == DType::kF16);
     return;
   }
-  for (int oi : ops) run_dot_general(dev, prog, prog.ops.at(oi), vals);
+  for (int oi : ops) run_dot_general(dev, prog, prog.ops.at(oi), vals, nullptr, 0);
+}
+
+// transpose(dot_general(a, b)) that only moves b's free dims before a's is
+// dot_general(b, a) (the weight gradient as jax.vjp lowers it): the product is
+// written where the transpose would put it. Same sums, same rounding.
+// Decode-shaped products (8 rows or fewer on either side) keep their
+// orientation, which the GEMV kernels need.
+bool fold_dot_transpose(Program* prog) {
+  std::map<int, size_t> producer;
+  std::map<int, int> uses;
+  for (size_t i = 0; i < prog->ops.size(); ++i) {
+    for (int r : prog->ops[i].results) producer[r] = i;
+    for (int v : prog->ops[i].operands) uses[v]++;
+  }
+  for (int r : prog->results) uses[r]++;
+  bool changed = false;
+  for (Op& t : prog->ops) {
+    if (t.kind != OpKind::kTranspose) continue;
+    auto it = producer.find(t.operands[0]);
+    if (it == producer.end() || uses[t.operands[0]] != 1) continue;
+    const Op& d = prog->ops[it->second];
+    if (d.kind != OpKind::kDotGeneral || d.operands.size() != 2 || d.results.size() != 1) continue;
+    const TensorType& dt = prog->type(d.results[0]);
+    const int64_t nb = static_cast<int64_t>(d.lhs_batch.size());
+    const int64_t nl = prog->type(d.operands[0]).rank() - nb - static_cast<int64_t>(d.lhs_contract.size());
+    const int64_t nr = prog->type(d.operands[1]).rank() - nb - static_cast<int64_t>(d.rhs_contract.size());
+    if (nb + nl + nr != dt.rank() || static_cast<int64_t>(t.dims.size()) != dt.rank()) continue;
+    bool swaps = nl > 0 && nr > 0;
+    int64_t m = 1, n = 1;
+    for (int64_t i = 0; i < dt.rank() && swaps; ++i) {
+      const int64_t want = i < nb ? i : i < nb + nr ? i + nl : i - nr;
+      swaps = t.dims[i] == want;
+      if (i >= nb) (i < nb + nl ? m : n) *= dt.dims[i];
+    }
+    if (!swaps || m <= 8 || n <= 8) continue;
+    Op r = d;
+    std::swap(r.operands[0], r.operands[1]);
+    std::swap(r.lhs_batch, r.rhs_batch);
+    std::swap(r.lhs_contract, r.rhs_contract);
+    r.results = t.results;
+    t = std::move(r);
+    changed = true;
+  }
+  return changed;
 }
 
 }  // namespace pjrtx

@@ -17,11 +17,31 @@ struct GemmParams {
   int batch = 1, M = 0, N = 0, K = 0;
   int64_t lda = 0, ldb = 0, ldc = 0;
   int64_t a_batch_stride = 0, b_batch_stride = 0;
-  int split_tiles = 1 << 30;  // 64-deep k-tiles per k-split
 };
 
-// MFMA block tiles (kernels/gemm.hip). A K-contiguous operand whose K is no
-// multiple of 8 must be zero from K to its row stride.
+// Products of one A with up to four B's (MFMA block tiles, kernels/gemm.hip):
+// one launch. A member's C is [batch][M][N]; with `add`, C = add +
+// round(product), `add` shaped like C (add_ld = N) or one row of N added to
+// every row (add_ld = 0), in C's 16-bit type.
+// A K-contiguous operand whose K is no multiple of 8 must be zero from K to
+// its row stride.
+constexpr int kMaxGemmMembers = 4;
+struct GemmMember {
+  const void* B = nullptr;
+  void* C = nullptr;
+  const void* add = nullptr;
+  int N = 0;
+  int tile0 = 0;  // first tile column (set by the launcher)
+  int64_t ldb = 0, b_batch_stride = 0, add_ld = 0;
+};
+struct GemmGroup {
+  int batch = 1, M = 0, K = 0;
+  int count = 1;
+  int split_tiles = 1 << 30;  // 64-deep k-tiles per k-split (set by the launcher)
+  int tiles_n = 0;            // tile columns over the members (set by the launcher)
+  int64_t lda = 0, a_batch_stride = 0;
+  GemmMember m[kMaxGemmMembers];
+};
 constexpr int kGemmTiles = 6;
 struct GemmPlan {
   int cfg = 0;              // block tile
@@ -32,14 +52,16 @@ struct GemmPlan {
 // True when the tile kernels take the operands: 16-byte aligned rows and
 // lane offsets below 2^31 bytes (K-contiguous rows up to 4M elements,
 // otherwise up to 16M). The base addresses must be 16-byte aligned.
-bool gemm_fits(const GemmParams& p, bool a_kmajor, bool b_kmajor);
+bool gemm_fits(const GemmGroup& g, bool a_kmajor, bool b_kmajor);
 // Block tile and k-split with the least estimated time (environment:
 // PJRTX_GEMM_TILE forces a tile, PJRTX_BIG_GEMM_MIN_TILES=n takes 256 x 256
 // tiles for every product with at least n of them); the partials take at most
 // max_workspace bytes.
-GemmPlan plan_gemm(const GemmParams& p, int64_t max_workspace);
-void launch_gemm(hipStream_t s, GemmParams p, const GemmPlan& plan, const void* A, bool a_kmajor, const void* B,
-                 bool b_kmajor, void* C, bool f16, int out_bytes, float* workspace);
+GemmPlan plan_gemm(const GemmGroup& g, int64_t max_workspace);
+void launch_gemm(hipStream_t s, GemmGroup g, const GemmPlan& plan, const void* A, bool a_kmajor, bool b_kmajor, bool f16,
+                 int out_bytes, float* workspace);
+// C[i] = add[i] + C[i] over rows x n 16-bit elements (add_ld as above).
+void launch_add_rows16(hipStream_t s, void* C, const void* add, int64_t rows, int64_t n, int64_t add_ld, bool f16);
 // out[b][r][0, ldp) = in[b][r][0, cols) (batch stride bs, row stride rs),
 // then zeros, for 16-bit elements; ldp a multiple of 8.
 void launch_pad_rows16(hipStream_t s, const void* in, void* out, int64_t batch, int64_t bs, int64_t rows, int64_t rs,

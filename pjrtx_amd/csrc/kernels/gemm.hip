@@ -84,6 +84,25 @@ __device__ __forceinline__ uint16_t to_half(float f) {
 }
 
 template <bool kF16>
+__device__ __forceinline__ float from_half(uint16_t h) {
+  if constexpr (kF16) return (float)__builtin_bit_cast(_Float16, h);
+  return __builtin_bit_cast(float, (uint32_t)h << 16);
+}
+
+// Eight 16-bit sums a + v.
+template <bool kF16>
+__device__ __forceinline__ u32x4 add8(const u32x4& v, const u32x4& a) {
+  u32x4 o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float lo = from_half<kF16>((uint16_t)a[q]) + from_half<kF16>((uint16_t)v[q]);
+    const float hi = from_half<kF16>((uint16_t)(a[q] >> 16)) + from_half<kF16>((uint16_t)(v[q] >> 16));
+    o[q] = (uint32_t)to_half<kF16>(lo) | (uint32_t)to_half<kF16>(hi) << 16;
+  }
+  return o;
+}
+
+template <bool kF16>
 __device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f32x16& c) {
   if constexpr (kF16)
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
@@ -205,8 +224,7 @@ struct FragReader {
 // WM x WN x WK waves: WK waves share an output sub-tile, each multiplying
 // 4 / WK of a k-tile's slabs.
 template <bool kF16, int kOut, bool kAK, bool kBKc, int TM, int TN, int WM, int WN, int WK, int kStages, int kLW>
-__global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmParams p, const uint16_t* __restrict__ A,
-                                                               const uint16_t* __restrict__ B, void* __restrict__ C) {
+__global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmGroup p, const uint16_t* __restrict__ A) {
   constexpr int kWaves = WM * WN * WK, WTM = TM / WM, WTN = TN / WN, MI = WTM / 32, NJ = WTN / 32, KS = 4 / WK;
   // Fragments of a whole k-tile fit in registers twice over: they are read
   // while the tile before multiplies. Otherwise a slab at a time.
@@ -220,7 +238,7 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmParams p, con
   // Consecutive workgroup ids go to the 8 XCDs in turn: each XCD gets a
   // contiguous run of tiles, walked 8 tile rows at a time so that B k-tiles
   // are reused from its L2.
-  const int tiles_m = (p.M + TM - 1) / TM, tiles_n = (p.N + TN - 1) / TN;
+  const int tiles_m = (p.M + TM - 1) / TM, tiles_n = p.tiles_n;
   const int per_batch = tiles_m * tiles_n;
   const int total = gridDim.x;
   const int xcd = blockIdx.x & 7;
@@ -235,7 +253,13 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmParams p, con
   const int gm = min(tiles_m - first_m, 8);
   const int tm = first_m + (t - g * gsize) % gm;
   const int tn = (t - g * gsize) / gm;
-  const int m0 = tm * TM, n0 = tn * TN;
+  int mi = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxGemmMembers; ++i)
+    if (i < p.count && tn >= p.m[i].tile0) mi = i;
+  const GemmMember mb = p.m[mi];
+  const int N = mb.N;
+  const int m0 = tm * TM, n0 = (tn - mb.tile0) * TN;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -251,8 +275,8 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmParams p, con
   OpB ob;
   oa.init(A + (int64_t)b * p.a_batch_stride + (kAK ? (int64_t)m0 * p.lda : (int64_t)m0), p.lda, min(TM, p.M - m0), p.K,
           ktail, wave, lane);
-  ob.init(B + (int64_t)b * p.b_batch_stride + (kBKc ? (int64_t)n0 * p.ldb : (int64_t)n0), p.ldb, min(TN, p.N - n0), p.K,
-          ktail, wave, lane);
+  ob.init(static_cast<const uint16_t*>(mb.B) + (int64_t)b * mb.b_batch_stride + (kBKc ? (int64_t)n0 * mb.ldb : (int64_t)n0),
+          mb.ldb, min(TN, N - n0), p.K, ktail, wave, lane);
   const uint32_t lds0 = lds_offset(smem);
 
   FragReader<kAK, TM, KS> ra;
@@ -491,25 +515,31 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmParams p, con
       }
     }
     __syncthreads();
-    uint16_t* Cb = reinterpret_cast<uint16_t*>(C) + (int64_t)b * p.M * p.ldc;
-    const bool vec = p.ldc % 8 == 0;
+    uint16_t* Cb = static_cast<uint16_t*>(mb.C) + (int64_t)b * p.M * N;
+    const uint16_t* add = static_cast<const uint16_t*>(mb.add) + (mb.add_ld ? (int64_t)b * p.M * N : 0);
+    const bool vec = N % 8 == 0;
 #pragma unroll
     for (int tt = 0; tt < TM * kCh / (kWaves * 64); ++tt) {
       const int c = tid + kWaves * 64 * tt;
       const int row = c / kCh, ch = c % kCh;
       const int m = m0 + row, n = n0 + ch * 8;
-      if (m >= p.M || n >= p.N) continue;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(&smem[at(row, ch)]);
-      if (vec && n + 8 <= p.N) {
-        *reinterpret_cast<u32x4*>(Cb + (int64_t)m * p.ldc + n) = v;
+      if (m >= p.M || n >= N) continue;
+      u32x4 v = *reinterpret_cast<const u32x4*>(&smem[at(row, ch)]);
+      if (vec) {
+        if (mb.add) v = add8<kF16>(v, *reinterpret_cast<const u32x4*>(add + m * mb.add_ld + n));
+        *reinterpret_cast<u32x4*>(Cb + (int64_t)m * N + n) = v;
       } else {
 #pragma unroll
         for (int q = 0; q < 8; ++q)
-          if (n + q < p.N) Cb[(int64_t)m * p.ldc + n + q] = (uint16_t)(v[q >> 1] >> ((q & 1) * 16));
+          if (n + q < N) {
+            uint16_t x = (uint16_t)(v[q >> 1] >> ((q & 1) * 16));
+            if (mb.add) x = to_half<kF16>(from_half<kF16>(add[m * mb.add_ld + n + q]) + from_half<kF16>(x));
+            Cb[(int64_t)m * N + n + q] = x;
+          }
       }
     }
   } else {
-    float* Cb = reinterpret_cast<float*>(C) + ((int64_t)split * p.batch + b) * p.M * p.ldc;
+    float* Cb = static_cast<float*>(mb.C) + ((int64_t)split * p.batch + b) * p.M * N;
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       const int q = i * WK + wk, bi = q / NJ, bj = q % NJ;
@@ -517,38 +547,70 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm_tile(GemmParams p, con
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wrow0 + bi * 32 + (r >> 2) * 8 + fh * 4 + (r & 3);
         const int n = n0 + wcol0 + bj * 32 + fr;
-        if (m < p.M && n < p.N) Cb[(int64_t)m * p.ldc + n] = own[i][r];
+        if (m < p.M && n < N) Cb[(int64_t)m * N + n] = own[i][r];
       }
     }
   }
 }
 
-// C[i] = sum over the k-splits of their f32 partials, in split order.
+// C[i] = (add +) the sum over the k-splits of their f32 partials, in split
+// order; one grid row per member.
+struct SplitSum {
+  int splits = 1, count = 1;
+  struct {
+    const float* part = nullptr;
+    void* C = nullptr;
+    const void* add = nullptr;
+    int64_t n = 0, N = 1, add_ld = 0;
+  } m[kMaxGemmMembers];
+};
 template <int kOutKind>  // 0 bf16, 1 f16, 2 f32
-__global__ void __launch_bounds__(256) splitk_reduce(const float* __restrict__ part, int splits, int64_t n,
-                                                     void* __restrict__ C) {
+__global__ void __launch_bounds__(256) splitk_reduce(SplitSum p) {
+  constexpr bool f16 = kOutKind == 1;
+  const auto& mb = p.m[blockIdx.y];
+  const int64_t n = mb.n;
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= n) return;
-  if (i + 4 <= n && n % 4 == 0) {
+  const float* part = mb.part;
+  const uint16_t* add = static_cast<const uint16_t*>(mb.add);
+  if (mb.N % 4 == 0) {
     f32x4 s = *reinterpret_cast<const f32x4*>(part + i);
 #pragma unroll 4
-    for (int k = 1; k < splits; ++k) s += *reinterpret_cast<const f32x4*>(part + (int64_t)k * n + i);
+    for (int k = 1; k < p.splits; ++k) s += *reinterpret_cast<const f32x4*>(part + (int64_t)k * n + i);
     if constexpr (kOutKind == 2) {
-      *reinterpret_cast<f32x4*>(static_cast<float*>(C) + i) = s;
+      *reinterpret_cast<f32x4*>(static_cast<float*>(mb.C) + i) = s;
     } else {
-      constexpr bool f16 = kOutKind == 1;
-      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(C) + i) =
-          u32x2{(uint32_t)to_half<f16>(s[0]) | (uint32_t)to_half<f16>(s[1]) << 16,
-                (uint32_t)to_half<f16>(s[2]) | (uint32_t)to_half<f16>(s[3]) << 16};
+      uint16_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = to_half<f16>(s[e]);
+      if (add) {
+        const uint16_t* a = add + (mb.add_ld ? i : i % mb.N);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = to_half<f16>(from_half<f16>(a[e]) + from_half<f16>(h[e]));
+      }
+      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(mb.C) + i) =
+          u32x2{(uint32_t)h[0] | (uint32_t)h[1] << 16, (uint32_t)h[2] | (uint32_t)h[3] << 16};
     }
     return;
   }
   for (int64_t j = i; j < min(i + 4, n); ++j) {
     float s = part[j];
-    for (int k = 1; k < splits; ++k) s += part[(int64_t)k * n + j];
-    if constexpr (kOutKind == 2) static_cast<float*>(C)[j] = s;
-    else static_cast<uint16_t*>(C)[j] = to_half<kOutKind == 1>(s);
+    for (int k = 1; k < p.splits; ++k) s += part[(int64_t)k * n + j];
+    if constexpr (kOutKind == 2) {
+      static_cast<float*>(mb.C)[j] = s;
+    } else {
+      uint16_t h = to_half<f16>(s);
+      if (add) h = to_half<f16>(from_half<f16>(add[mb.add_ld ? j : j % mb.N]) + from_half<f16>(h));
+      static_cast<uint16_t*>(mb.C)[j] = h;
+    }
   }
+}
+
+template <bool kF16>
+__global__ void __launch_bounds__(256) add_rows16(uint16_t* __restrict__ C, const uint16_t* __restrict__ add, int64_t total,
+                                                  int64_t n, int64_t add_ld) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < total) C[i] = to_half<kF16>(from_half<kF16>(add[add_ld ? i : i % n]) + from_half<kF16>(C[i]));
 }
 
 // out[b][r] = in[b][r] (cols 16-bit elements, any alignment) in rows of ldp
@@ -591,16 +653,20 @@ constexpr Tile kTiles[kGemmTiles] = {
 constexpr int kCus = 256;
 constexpr int kMinSplitTiles = 4;  // k-tiles a split must have
 
-int64_t tiles_of(const GemmParams& p, const Tile& t) {
-  return (int64_t)((p.M + t.tm - 1) / t.tm) * ((p.N + t.tn - 1) / t.tn) * p.batch;
+int64_t tile_columns(const GemmGroup& g, const Tile& t) {
+  int64_t n = 0;
+  for (int i = 0; i < g.count; ++i) n += (g.m[i].N + t.tn - 1) / t.tn;
+  return n;
+}
+int64_t tiles_of(const GemmGroup& g, const Tile& t) {
+  return (int64_t)((g.M + t.tm - 1) / t.tm) * tile_columns(g, t) * g.batch;
 }
 
 template <bool kF16, int kOut, bool kAK, bool kBKc>
-void launch_cfg(hipStream_t s, int cfg, unsigned grid, const GemmParams& p, const uint16_t* A, const uint16_t* B,
-                void* C) {
+void launch_cfg(hipStream_t s, int cfg, unsigned grid, const GemmGroup& g, const uint16_t* A) {
 #define PJRTX_TILE(TM, TN, WM, WN, WK, ST, LW)                                                             \
   hipLaunchKernelGGL((gemm_tile<kF16, kOut, kAK, kBKc, TM, TN, WM, WN, WK, ST, LW>), dim3(grid),           \
-                     dim3(WM * WN * WK * 64), 0, s, p, A, B, C)
+                     dim3(WM * WN * WK * 64), 0, s, g, A)
   switch (cfg) {
     case 0: PJRTX_TILE(256, 256, 2, 4, 1, 2, 4); break;
     case 1: PJRTX_TILE(128, 256, 2, 4, 1, 3, 8); break;
@@ -613,55 +679,57 @@ void launch_cfg(hipStream_t s, int cfg, unsigned grid, const GemmParams& p, cons
 }
 
 template <bool kF16, int kOut>
-void launch_layout(hipStream_t s, int cfg, unsigned grid, const GemmParams& p, const void* A, bool a_kmajor,
-                   const void* B, bool b_kmajor, void* C) {
+void launch_layout(hipStream_t s, int cfg, unsigned grid, const GemmGroup& g, const void* A, bool a_kmajor, bool b_kmajor) {
   const uint16_t* a = static_cast<const uint16_t*>(A);
-  const uint16_t* b = static_cast<const uint16_t*>(B);
   if (a_kmajor) {
-    if (b_kmajor) launch_cfg<kF16, kOut, true, true>(s, cfg, grid, p, a, b, C);
-    else launch_cfg<kF16, kOut, true, false>(s, cfg, grid, p, a, b, C);
+    if (b_kmajor) launch_cfg<kF16, kOut, true, true>(s, cfg, grid, g, a);
+    else launch_cfg<kF16, kOut, true, false>(s, cfg, grid, g, a);
   } else {
-    if (b_kmajor) launch_cfg<kF16, kOut, false, true>(s, cfg, grid, p, a, b, C);
-    else launch_cfg<kF16, kOut, false, false>(s, cfg, grid, p, a, b, C);
+    if (b_kmajor) launch_cfg<kF16, kOut, false, true>(s, cfg, grid, g, a);
+    else launch_cfg<kF16, kOut, false, false>(s, cfg, grid, g, a);
   }
 }
 
 }  // namespace
 
-bool gemm_fits(const GemmParams& p, bool a_kmajor, bool b_kmajor) {
+bool gemm_fits(const GemmGroup& g, bool a_kmajor, bool b_kmajor) {
   // A load's lane offset (a block of K-contiguous rows, or 64 k rows) stays
   // below 2^31 bytes; 16-byte chunks are aligned.
   const int64_t limit = int64_t(1) << 30;
-  const auto ok = [&](int64_t ld, int64_t bs, bool kc) {
-    return ld % 8 == 0 && bs % 8 == 0 && (kc ? 256 : BK) * ld < limit;
+  const auto ok = [&](int64_t ld, int64_t bs, bool kc, int64_t len) {
+    return ld % 8 == 0 && bs % 8 == 0 && (kc ? 256 : BK) * ld < limit && ld >= len;
   };
-  return p.M > 0 && p.N > 0 && p.K > 0 && ok(p.lda, p.a_batch_stride, a_kmajor) &&
-         ok(p.ldb, p.b_batch_stride, b_kmajor) && p.lda >= (a_kmajor ? p.K : p.M) && p.ldb >= (b_kmajor ? p.K : p.N) &&
-         tiles_of(p, kTiles[kGemmTiles - 1]) < (int64_t(1) << 24);
+  bool fits = g.M > 0 && g.K > 0 && g.count >= 1 && g.count <= kMaxGemmMembers &&
+              ok(g.lda, g.a_batch_stride, a_kmajor, a_kmajor ? g.K : g.M);
+  for (int i = 0; i < g.count && fits; ++i)
+    fits = g.m[i].N > 0 && ok(g.m[i].ldb, g.m[i].b_batch_stride, b_kmajor, b_kmajor ? g.K : g.m[i].N);
+  return fits && tiles_of(g, kTiles[kGemmTiles - 1]) < (int64_t(1) << 24);
 }
 
-GemmPlan plan_gemm(const GemmParams& p, int64_t max_workspace) {
-  const int64_t nk = (p.K + BK - 1) / BK;
+GemmPlan plan_gemm(const GemmGroup& g, int64_t max_workspace) {
+  const int64_t nk = (g.K + BK - 1) / BK;
   const int64_t forced = env_int("PJRTX_GEMM_TILE", -1);
   const int64_t big_min = env_int("PJRTX_BIG_GEMM_MIN_TILES", 0);
-  const double out_bytes = 4.0 * p.batch * p.M * p.N;
+  int64_t n_all = 0;
+  for (int i = 0; i < g.count; ++i) n_all += g.m[i].N;
+  const int64_t out_bytes = int64_t(4) * g.batch * g.M * n_all;
   GemmPlan best;
   double best_us = 1e30;
   for (int c = 0; c < kGemmTiles; ++c) {
     const Tile& t = kTiles[c];
-    const int64_t tiles = tiles_of(p, t);
+    const int64_t tiles = tiles_of(g, t);
     if (forced >= 0 && forced < kGemmTiles && c != forced) continue;
-    if (forced < 0 && big_min > 0 && p.M >= 256 && p.N >= 256 && tiles_of(p, kTiles[0]) >= big_min && c != 0) continue;
+    if (forced < 0 && big_min > 0 && g.M >= 256 && n_all >= 256 && tiles_of(g, kTiles[0]) >= big_min && c != 0) continue;
     for (int64_t want = 1; want <= 64; want += want < 8 ? 1 : want / 4) {
       const int64_t per = (nk + want - 1) / want, splits = (nk + per - 1) / per;
       if (splits != want) continue;
-      if (splits > 1 && (per < kMinSplitTiles || splits * out_bytes > (double)max_workspace)) break;
+      if (splits > 1 && (per < kMinSplitTiles || splits * (double)out_bytes > (double)max_workspace)) break;
       // Every round of kCus workgroups multiplies its k-tiles; the splits'
       // partials are written, then read by a second launch (2.5 us and the
       // bytes at 6 TB/s).
       const int64_t rounds = (tiles * splits + kCus - 1) / kCus;
       double us = 2.0 + (double)rounds * per * t.us_tile + (double)((rounds + t.resident - 1) / t.resident) * t.us_edge;
-      if (splits > 1) us += 2.5 + 2.0 * splits * out_bytes / 6e6;
+      if (splits > 1) us += 2.5 + 2.0 * splits * (double)out_bytes / 6e6;
       if (us < best_us) {
         best_us = us;
         best.cfg = c;
@@ -671,33 +739,63 @@ GemmPlan plan_gemm(const GemmParams& p, int64_t max_workspace) {
       if (tiles * splits >= 2 * kCus) break;
     }
   }
-  best.workspace = best.splits > 1 ? (size_t)best.splits * p.batch * p.M * p.N * 4 : 0;
+  best.workspace = best.splits > 1 ? (size_t)best.splits * out_bytes : 0;
   return best;
 }
 
-void launch_gemm(hipStream_t s, GemmParams p, const GemmPlan& plan, const void* A, bool a_kmajor, const void* B,
-                 bool b_kmajor, void* C, bool f16, int out_bytes, float* workspace) {
-  const int64_t grid = tiles_of(p, kTiles[plan.cfg]) * plan.splits;
+void launch_gemm(hipStream_t s, GemmGroup g, const GemmPlan& plan, const void* A, bool a_kmajor, bool b_kmajor, bool f16,
+                 int out_bytes, float* workspace) {
+  const Tile& t = kTiles[plan.cfg];
+  const int64_t grid = tiles_of(g, t) * plan.splits;
   PJRTX_CHECK(grid > 0 && grid < (int64_t(1) << 31) && (plan.splits == 1 || workspace), Code::kInternal, "gemm: bad plan");
-  p.split_tiles = plan.split_tiles;
-  const unsigned g = static_cast<unsigned>(grid);
-  if (plan.splits == 1 && out_bytes == 2) {
-    if (f16) launch_layout<true, 2>(s, plan.cfg, g, p, A, a_kmajor, B, b_kmajor, C);
-    else launch_layout<false, 2>(s, plan.cfg, g, p, A, a_kmajor, B, b_kmajor, C);
-    check("gemm_tile");
-    return;
+  g.split_tiles = plan.split_tiles;
+  g.tiles_n = 0;
+  SplitSum sum;
+  sum.splits = plan.splits;
+  sum.count = g.count;
+  int64_t most = 0;
+  for (int i = 0; i < g.count; ++i) {
+    GemmMember& m = g.m[i];
+    PJRTX_CHECK(!m.add || out_bytes == 2, Code::kInternal, "gemm: an addend needs a 16-bit result");
+    m.tile0 = g.tiles_n;
+    g.tiles_n += (m.N + t.tn - 1) / t.tn;
+    if (plan.splits > 1) {
+      const int64_t n = (int64_t)g.batch * g.M * m.N;
+      sum.m[i] = {workspace, m.C, m.add, n, m.N, m.add_ld};
+      m.C = workspace;
+      m.add = nullptr;
+      workspace += n * plan.splits;
+      most = std::max(most, n);
+    }
   }
-  void* out = plan.splits == 1 ? C : workspace;
-  if (f16) launch_layout<true, 4>(s, plan.cfg, g, p, A, a_kmajor, B, b_kmajor, out);
-  else launch_layout<false, 4>(s, plan.cfg, g, p, A, a_kmajor, B, b_kmajor, out);
+  const unsigned gr = static_cast<unsigned>(grid);
+  const bool half_out = plan.splits == 1 && out_bytes == 2;
+  if (half_out) {
+    if (f16) launch_layout<true, 2>(s, plan.cfg, gr, g, A, a_kmajor, b_kmajor);
+    else launch_layout<false, 2>(s, plan.cfg, gr, g, A, a_kmajor, b_kmajor);
+  } else {
+    if (f16) launch_layout<true, 4>(s, plan.cfg, gr, g, A, a_kmajor, b_kmajor);
+    else launch_layout<false, 4>(s, plan.cfg, gr, g, A, a_kmajor, b_kmajor);
+  }
   if (plan.splits > 1) {
-    const int64_t n = (int64_t)p.batch * p.M * p.N;
-    const dim3 gr(static_cast<unsigned>((n + 1023) / 1024)), block(256);
-    if (out_bytes == 4) hipLaunchKernelGGL((splitk_reduce<2>), gr, block, 0, s, workspace, plan.splits, n, C);
-    else if (f16) hipLaunchKernelGGL((splitk_reduce<1>), gr, block, 0, s, workspace, plan.splits, n, C);
-    else hipLaunchKernelGGL((splitk_reduce<0>), gr, block, 0, s, workspace, plan.splits, n, C);
+    const dim3 sg(static_cast<unsigned>((most + 1023) / 1024), static_cast<unsigned>(g.count)), block(256);
+    if (out_bytes == 4) hipLaunchKernelGGL((splitk_reduce<2>), sg, block, 0, s, sum);
+    else if (f16) hipLaunchKernelGGL((splitk_reduce<1>), sg, block, 0, s, sum);
+    else hipLaunchKernelGGL((splitk_reduce<0>), sg, block, 0, s, sum);
   }
   check("gemm_tile");
+}
+
+void launch_add_rows16(hipStream_t s, void* C, const void* add, int64_t rows, int64_t n, int64_t add_ld, bool f16) {
+  const int64_t total = rows * n;
+  if (total == 0) return;
+  PJRTX_CHECK((total + 255) / 256 < (int64_t(1) << 31), Code::kInternal, "add_rows16: grid too large");
+  const dim3 grid(static_cast<unsigned>((total + 255) / 256)), block(256);
+  uint16_t* c = static_cast<uint16_t*>(C);
+  const uint16_t* a = static_cast<const uint16_t*>(add);
+  if (f16) hipLaunchKernelGGL((add_rows16<true>), grid, block, 0, s, c, a, total, n, add_ld);
+  else hipLaunchKernelGGL((add_rows16<false>), grid, block, 0, s, c, a, total, n, add_ld);
+  check("add_rows16");
 }
 
 void launch_pad_rows16(hipStream_t s, const void* in, void* out, int64_t batch, int64_t bs, int64_t rows, int64_t rs,

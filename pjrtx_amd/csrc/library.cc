@@ -286,11 +286,11 @@ GatherParams make_gather_params(const Program& prog, const Op& op) {
   return g;
 }
 
-void run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals);
+bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, const void* add, int64_t add_ld);
 void run_scatter(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals);
 void run_attention(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, bool partials_out);
 void run_dot_group(Device* dev, const Program& prog, const std::vector<int>& ops, std::vector<MemRef>& vals);
-void run_dot_residual(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, int add, int out);
+void run_dot_residual(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, int add, int out, bool row);
 
 // stablehlo.reduce_window (the planner checked the supported forms).
 // Replaces pjrtx_mlx_metal_buffer_reduce_window and
@@ -350,8 +350,8 @@ void run_library_step(Device* dev, const Program& prog, const Step& step, std::v
       return;
     }
     case LibKind::kDot:
-      if (step.dot_add >= 0) run_dot_residual(dev, prog, op, vals, step.dot_add, step.outputs[0]);
-      else run_dot_general(dev, prog, op, vals);
+      if (step.dot_add >= 0) run_dot_residual(dev, prog, op, vals, step.dot_add, step.outputs[0], step.dot_add_row);
+      else run_dot_general(dev, prog, op, vals, nullptr, 0);
       return;
     case LibKind::kScatter:
       run_scatter(dev, prog, op, vals);

@@ -513,13 +513,13 @@ int Planner::order_preserving_source(int v) const {
 
 // Decode-shaped dot (the reference's dot group candidates,
 // executable_metal_graph_lowering_fusion.zig:394-424): [M, K] x [K, N] with
-// M <= 4, 16-bit operands.
+// M <= 4, 16-bit operands; or M > 8, which the block tiles take in one launch.
 static bool group_candidate(const Program& prog, const Op& op) {
   if (op.kind != OpKind::kDotGeneral || op.operands.size() != 2) return false;
   const TensorType& l = prog.type(op.operands[0]);
   const TensorType& r = prog.type(op.operands[1]);
   return l.rank() == 2 && r.rank() == 2 && op.lhs_batch.empty() && op.rhs_batch.empty() &&
-         op.lhs_contract == Dims{1} && op.rhs_contract == Dims{0} && l.dims[0] <= 4 && l.dtype == r.dtype &&
+         op.lhs_contract == Dims{1} && op.rhs_contract == Dims{0} && (l.dims[0] <= 4 || l.dims[0] > 8) && l.dtype == r.dtype &&
          (l.dtype == DType::kBF16 || l.dtype == DType::kF16);
 }
 
@@ -732,9 +732,23 @@ void Planner::merge_sibling_loops(std::vector<Step>* steps) {
   }
 }
 
+// True for a product of 16-bit operands with more rows than the GEMV kernels
+// take and a result of the operands' type.
+static bool tile_gemm(const Program& prog, const Op& op) {
+  if (op.kind != OpKind::kDotGeneral || op.operands.size() != 2) return false;
+  const TensorType& l = prog.type(op.operands[0]);
+  const TensorType& r = prog.type(op.operands[1]);
+  const DType o = prog.type(op.results[0]).dtype;
+  int64_t m = l.elements();
+  for (int64_t d : op.lhs_batch) m = l.dims[d] ? m / l.dims[d] : 0;
+  for (int64_t d : op.lhs_contract) m = l.dims[d] ? m / l.dims[d] : 0;
+  return m > 8 && l.dtype == r.dtype && o == l.dtype && (o == DType::kBF16 || o == DType::kF16);
+}
+
 // add(dot, x) where the dot's only reader is that add: the dot step writes
-// x + round(dot) directly (the GEMV's epilogue), one launch and one buffer
-// fewer (a residual connection after an output or down projection).
+// x + round(dot) directly (the GEMV's or the block tiles' epilogue), one
+// launch and one buffer fewer (a residual connection after an output or down
+// projection); a bias row broadcast over the product's rows likewise.
 void Planner::merge_dot_residuals(std::vector<Step>* steps) {
   std::map<int, int> readers;
   for (const Step& s : *steps)
@@ -742,18 +756,33 @@ void Planner::merge_dot_residuals(std::vector<Step>* steps) {
   auto v2s = value_to_step(*steps);
   for (size_t g = 0; g < steps->size(); ++g) {
     Step& G = (*steps)[g];
-    if (G.kind != StepKind::kLoop || G.outputs.size() != 1 || G.ops.size() != 1 || G.inputs.size() != 2) continue;
-    const Op& add = prog_.ops[G.ops[0]];
+    if (G.kind != StepKind::kLoop || G.outputs.size() != 1 || G.ops.empty() || G.ops.size() > 2 || G.inputs.size() != 2)
+      continue;
+    const Op& add = prog_.ops[G.ops.back()];
     if (add.kind != OpKind::kAdd || add.results[0] != G.outputs[0]) continue;
+    // A second op is the broadcast of a bias row.
+    const Op* bias = G.ops.size() == 2 ? &prog_.ops[G.ops[0]] : nullptr;
+    if (bias && bias->kind != OpKind::kBroadcastInDim) continue;
     for (int side = 0; side < 2; ++side) {
-      const int d = add.operands[side], x = add.operands[1 - side];
+      const int d = add.operands[side];
+      int x = add.operands[1 - side];
       if (d == x || !v2s.count(d) || readers[d] != 1 || outputs_.count(d)) continue;
+      if (bias && x != bias->results[0]) continue;
       Step& D = (*steps)[v2s[d]];
       if (D.kind != StepKind::kLibrary || D.lib != LibKind::kDot || D.dot_add >= 0 || D.outputs.size() != 1) continue;
       const Op& dot = prog_.ops[D.lib_op];
-      if (!one_pass_gemv(prog_, dot) || prog_.type(x).dims != prog_.type(d).dims ||
+      const bool gemm = tile_gemm(prog_, dot);
+      if ((!gemm && (bias || !one_pass_gemv(prog_, dot))) || prog_.type(x).dims != prog_.type(d).dims ||
           prog_.type(x).dtype != prog_.type(d).dtype || prog_.type(G.outputs[0]).dtype != prog_.type(d).dtype)
         continue;
+      if (bias) {
+        x = bias->operands[0];
+        const TensorType& dt = prog_.type(d);
+        if (prog_.type(x).rank() != 1 || bias->dims != Dims{dt.rank() - 1} || prog_.type(x).dims[0] != dt.dims.back() ||
+            prog_.type(dot.operands[1]).rank() != static_cast<int>(dot.rhs_batch.size() + dot.rhs_contract.size()) + 1)
+          continue;
+        D.dot_add_row = true;
+      }
       D.dot_add = x;
       D.inputs.push_back(x);
       D.outputs = G.outputs;

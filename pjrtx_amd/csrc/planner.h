@@ -152,6 +152,7 @@ struct Step {
   // kDot: value added to the rounded product (a residual add merged into the
   // dot); the step's output is then the sum, not the dot's own result.
   int dot_add = -1;
+  bool dot_add_row = false;  // ... and it is one row, added to every row (a bias)
   // kWhile: the iteration count when constants fix it (a counter from a
   // constant start, compared with a constant bound, advanced by a constant
   // step), else -1 (the predicate is read every iteration).
@@ -252,6 +253,8 @@ void rewrite_program(Program* prog);
 // Folds JAX's negative-index normalization of gather indices into the
 // gathers (library.cc); true when a gather changed.
 bool fold_gather_index_wrap(Program* prog);
+// transpose(dot_general(a, b)) as dot_general(b, a) (dot_general.cc).
+bool fold_dot_transpose(Program* prog);
 
 // Turns decode-shaped dot and dot-group library steps into kGemv steps and
 // absorbs their row-fused prologues and elementwise epilogues
