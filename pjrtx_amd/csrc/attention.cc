@@ -433,6 +433,7 @@ void rewrite_program(Program* prog) {
     }
   }
   changed |= fold_dot_transpose(prog);
+  changed |= fold_sort_iota(prog);
   if (changed) remove_dead_ops(prog);
 }
 

@@ -103,16 +103,6 @@ MemRef canonicalize(Device* dev, const TensorType& t, const Dims& batch, const D
 
 }  // namespace
 
-namespace {
-// Bytes this thread may still allocate on the device: what the installed
-// fixed block has left, or no bound.
-int64_t scratch_left(Device* dev) {
-  const Arena* a = thread_arena();
-  if (!a || a->dev != dev) return int64_t(1) << 60;
-  return static_cast<int64_t>(a->cap - std::min(a->cap, (a->used + 255) & ~size_t(255)));
-}
-}  // namespace
-
 // Workgroups of the one-pass GEMV for a single product with N columns.
 int single_wide_tiles(int64_t N) {
   GemvGroup one;

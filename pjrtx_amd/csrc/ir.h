@@ -126,6 +126,10 @@ struct Op {
   // fold_gather_index_wrap. 0: indices are read as they are.
   int64_t index_wrap = 0;
 
+  // sort: results that are the sorted positions (their operand was an iota
+  // along the sorted dim, and is not in `operands`).
+  Dims iota_results;
+
   // constant literal: raw little-endian element bytes of the result type,
   // or one element when `splat`.
   std::vector<uint8_t> literal;

@@ -1,13 +1,12 @@
 // Row sorts for stablehlo.sort and chlo.top_k (launchers of kernels/sort.hip).
 //
-// Every element of a row becomes one 64-bit sort word: an order-preserving
-// 32-bit image of its key in the high half and its position in the row in
-// the low half. All words of a row are distinct, so sorting them ascending
-// gives the one order a stable sort gives (equal keys keep their positions'
-// order), whatever network sorts them. Bitonic networks do: in LDS for rows
-// up to kSortBlock words, with global compare-exchange passes between LDS
-// passes above that. A row's results are gathered from the operands by the
-// positions in the sorted words, so keys and payloads come back bit for bit.
+// Every element of a row becomes one sort word: an order-preserving 32-bit
+// image of its key over its position in the row. All words of a row are
+// distinct, so sorting them ascending gives the one order a stable sort gives
+// (equal keys keep their positions' order), however they are sorted. A row's
+// results are gathered from the operands by the positions in the sorted words
+// (the keys decoded from the image where it is invertible), so keys and
+// payloads come back bit for bit.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -16,7 +15,7 @@
 
 namespace pjrtx {
 
-constexpr int kSortBlock = 4096;       // words sorted per LDS pass (32 KiB)
+constexpr int kSortBlock = 4096;       // words a bitonic LDS pass sorts (32 KiB)
 constexpr int kSortMaxOperands = 8;    // operands gathered by one output launch
 
 // How operand 0's bits map to the ascending 32-bit image.
@@ -39,7 +38,9 @@ struct SortRows {
   uint32_t inf_bits = 0;  // float keys: the bits of +inf (a larger magnitude is a NaN)
 };
 
-// Results: out_j[outer, i, j] = operand_j[outer, pos_i, j] for i < out_n.
+// Results: out_j[outer, i, j] = operand_j[outer, pos_i, j] for i < out_n; a
+// null source is the position itself (an operand that was an iota along the
+// sorted dim). src[0] is the key operand.
 struct SortGather {
   int count = 0;
   const void* src[kSortMaxOperands] = {};
@@ -49,13 +50,15 @@ struct SortGather {
   void* index_dst = nullptr;  // optional s32 output of the positions (top_k indices)
 };
 
-// Bytes of device scratch sort_rows needs for these rows and out_n.
-size_t sort_scratch_bytes(const SortRows& r, int64_t out_n);
+// Bytes of device scratch sort_rows needs for these rows and out_n, at most
+// about max_bytes where a path with less exists (rows that merge take two
+// buffers of 8 bytes an element; a bitonic network one of padded rows).
+size_t sort_scratch_bytes(const SortRows& r, int64_t out_n, int64_t max_bytes);
 
 // Sorts every row of operand 0 (`keys`) and writes the first `g.out_n`
 // positions of each row's order through `g`. out_n == n is a full sort;
 // a smaller out_n keeps only the row's first out_n (top_k with
-// descending = 1). `scratch` holds sort_scratch_bytes bytes.
-void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGather& g, void* scratch);
+// descending = 1). `scratch` holds sort_scratch_bytes(..., max_bytes) bytes.
+void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGather& g, void* scratch, int64_t max_bytes);
 
 }  // namespace pjrtx

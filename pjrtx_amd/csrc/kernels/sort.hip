@@ -8,17 +8,15 @@
 // keys keep their positions' order in both directions (a stable sort, as
 // StableHLO's is_stable and XLA's TopK ask).
 //
-// Three kernels:
-//  * sort_local: one workgroup sorts up to kSortBlock words of a row in LDS
-//    (a bitonic network; 512 threads, each doing 4 compare-exchanges per
-//    stage) and either keeps the first `keep` words or writes the results.
-//  * bitonic_global: one compare-exchange stage with partner distance of
-//    at least kSortBlock, for rows longer than one LDS block.
-//  * sort_write: gathers the results of words held in HBM.
-// top_k with k <= kSortBlock / 2 reduces instead of sorting the whole row:
-// each block keeps its first k' = pow2 >= k words (every word of the row's
-// top k is among its block's top k'), and the survivors are sorted again
-// until one block holds them all. At [64, 128256] that is two LDS passes.
+// Kernels:
+//  * sort_block: one workgroup sorts up to kSortTile words of a row in LDS by
+//    merging: 16 words a thread by a register network, then runs of 16, 32,
+//    ... by merge path, and keeps the first `keep` words or writes the results.
+//  * merge_runs: merges neighbouring sorted runs of a row from HBM.
+//  * topk_select: the first k <= 256 words of a chunk, without sorting it.
+//  * sort_local, bitonic_global, sort_write: a bitonic network over padded
+//    rows in one buffer, for a caller whose fixed scratch block does not hold
+//    the two buffers merging needs, and for rows of 2^30 elements and more.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,17 +35,10 @@ struct LocalPass {
   const void* keys = nullptr;
   SortRows r;
   const uint64_t* list = nullptr;
-  int64_t list_len = 0, list_stride = 0;
-  int block = 0;              // words per workgroup, a power of two <= kSortBlock
+  int64_t row_len = 0;        // words of a padded row
   int64_t blocks_per_row = 1;
   int64_t k_first = 2, k_last = 2, j_first = 1;
-  int global_dir = 0;         // direction from the word's row position (global network) or block position
-  // Destination: the first `keep` words of each block, or the results.
   uint64_t* dst = nullptr;
-  int64_t keep = 0, dst_stride = 0;
-  int write_out = 0;
-  int filter = 0;             // sort only the words that can be among the first `keep` (or out_n)
-  SortGather g;
 };
 
 __device__ __forceinline__ uint32_t load_key(const void* keys, int64_t e, int bits) {
@@ -56,34 +47,33 @@ __device__ __forceinline__ uint32_t load_key(const void* keys, int64_t e, int bi
   return static_cast<const uint8_t*>(keys)[e];
 }
 
-// Order-preserving image of a key (ascending), inverted for descending.
-__device__ __forceinline__ uint32_t key_image(uint32_t raw, const SortRows& r) {
-  const uint32_t mask = r.key_bits == 32 ? 0xffffffffu : ((1u << r.key_bits) - 1u);
-  const uint32_t sign = 1u << (r.key_bits - 1);
-  uint32_t v = raw & mask, img;
-  if (r.key_class == kSortKeySigned) {
-    img = v ^ sign;
-  } else if (r.key_class == kSortKeyUnsigned) {
-    img = v;
-  } else {
-    const uint32_t mag = v & ~sign;
-    if (r.key_class == kSortKeyFloat && mag > r.inf_bits) {
-      img = mask;  // every NaN: one class, after +inf
-    } else {
-      if (r.key_class == kSortKeyFloat && mag == 0) v = 0;  // -0 == +0
-      img = (v & sign) ? (~v & mask) : (v | sign);
-    }
-  }
-  return r.descending ? (~img & mask) : img;
+// Order-preserving image of a key (ascending), inverted for descending: the
+// key XOR one mask where its top bit is set and another where it is not, and
+// for FLOAT compares one image for every NaN and one for both zeros. No branch
+// per element.
+struct KeyMap {
+  uint32_t mask = 0, neg = 0, pos = 0, nan_over = 0, zero_keep = 0, nan_image = 0;
+  int shift = 0;
+};
+__host__ __device__ __forceinline__ KeyMap key_map(const SortRows& r) {
+  KeyMap m;
+  m.mask = r.key_bits == 32 ? 0xffffffffu : ((1u << r.key_bits) - 1u);
+  const uint32_t sign = 1u << (r.key_bits - 1), flip = r.descending ? m.mask : 0u;
+  const bool fl = r.key_class == kSortKeyFloat, total = fl || r.key_class == kSortKeyTotal;
+  m.neg = (total ? m.mask : r.key_class == kSortKeySigned ? sign : 0u) ^ flip;
+  m.pos = (r.key_class == kSortKeyUnsigned ? 0u : sign) ^ flip;
+  m.nan_over = fl ? r.inf_bits : 0xffffffffu;  // larger magnitudes are NaNs, after +inf
+  m.zero_keep = fl ? 0u : 0xffffffffu;         // -0 == +0
+  m.nan_image = m.mask ^ flip;
+  m.shift = 32 - r.key_bits;
+  return m;
 }
-
-// Minimum over the wave's 64 lanes, in every lane (a butterfly of lane swaps).
-__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint64_t o = __shfl_xor(v, d, 64);
-    v = o < v ? o : v;
-  }
-  return v;
+__device__ __forceinline__ uint32_t key_image(uint32_t v, const KeyMap& m) {
+  const uint32_t mag = v & (m.mask >> 1);
+  v = mag == 0 ? v & m.zero_keep : v;
+  const uint32_t neg = (uint32_t)((int32_t)(v << m.shift) >> 31);
+  const uint32_t img = v ^ ((neg & m.neg) | (~neg & m.pos));
+  return mag > m.nan_over ? m.nan_image : img;
 }
 
 template <typename T>
@@ -98,6 +88,15 @@ __device__ __forceinline__ void gather_one(const SortGather& g, const SortRows& 
   const int64_t s = (outer * r.n + pos) * r.inner + j;
   const int64_t d = (outer * g.out_n + i) * r.inner + j;
   for (int o = 0; o < g.count; ++o) {
+    if (!g.src[o]) {
+      switch (g.elem_bytes[o]) {
+        case 1: static_cast<uint8_t*>(g.dst[o])[d] = (uint8_t)pos; break;
+        case 2: static_cast<uint16_t*>(g.dst[o])[d] = (uint16_t)pos; break;
+        case 4: static_cast<uint32_t*>(g.dst[o])[d] = (uint32_t)pos; break;
+        default: static_cast<uint64_t*>(g.dst[o])[d] = (uint64_t)pos; break;
+      }
+      continue;
+    }
     switch (g.elem_bytes[o]) {
       case 1: copy_elem<uint8_t>(g.src[o], g.dst[o], s, d); break;
       case 2: copy_elem<uint16_t>(g.src[o], g.dst[o], s, d); break;
@@ -112,116 +111,32 @@ __global__ void __launch_bounds__(kLocalThreads) sort_local_kernel(LocalPass p) 
   __shared__ uint64_t s[kSortBlock];
   const int64_t row = blockIdx.x / p.blocks_per_row;
   const int64_t blk = blockIdx.x - row * p.blocks_per_row;
-  const int B = p.block;
-  const int64_t base = blk * B;
-  // Loads in batches of kBatch per thread, all issued before any is used
-  // (one outstanding load per thread would leave the kernel latency-bound).
-  constexpr int kBatch = 8;
-  const int bd = static_cast<int>(blockDim.x);
-  if (p.list) {
-    const uint64_t* src = p.list + row * p.list_stride;
-    for (int i0 = 0; i0 < B; i0 += kBatch * bd) {
-      uint64_t w[kBatch];
+  const int64_t base = blk * kSortBlock;
+  const int64_t outer = row / p.r.inner, j0 = row - outer * p.r.inner;
+  const int64_t row0 = outer * p.r.n * p.r.inner + j0;
+  constexpr int kBatch = kSortBlock / kLocalThreads;
+  const KeyMap map = key_map(p.r);
+  uint64_t w[kBatch];
 #pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int i = i0 + q * bd + static_cast<int>(threadIdx.x);
-        const int64_t idx = base + i;
-        w[q] = (i < B && idx < p.list_len) ? src[idx] : kSentinel;
-      }
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int i = i0 + q * bd + static_cast<int>(threadIdx.x);
-        if (i < B) s[i] = w[q];
-      }
-    }
-  } else {
-    const int64_t outer = row / p.r.inner, j = row - outer * p.r.inner;
-    const int64_t row0 = outer * p.r.n * p.r.inner + j;
-    for (int i0 = 0; i0 < B; i0 += kBatch * bd) {
-      uint32_t raw[kBatch];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int i = i0 + q * bd + static_cast<int>(threadIdx.x);
-        const int64_t idx = base + i;
-        raw[q] = (i < B && idx < p.r.n) ? load_key(p.keys, row0 + idx * p.r.inner, p.r.key_bits) : 0u;
-      }
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int i = i0 + q * bd + static_cast<int>(threadIdx.x);
-        const int64_t idx = base + i;
-        if (i < B)
-          s[i] = idx < p.r.n ? ((static_cast<uint64_t>(key_image(raw[q], p.r)) << 32) | static_cast<uint64_t>(idx))
-                             : kSentinel;
-      }
-    }
+  for (int q = 0; q < kBatch; ++q) {
+    const int64_t idx = base + q * kLocalThreads + (int)threadIdx.x;
+    if (p.list) w[q] = p.list[row * p.row_len + idx];
+    else if (idx < p.r.n)
+      w[q] = (static_cast<uint64_t>(key_image(load_key(p.keys, row0 + idx * p.r.inner, p.r.key_bits), map)) << 32) |
+             static_cast<uint64_t>(idx);
+    else w[q] = kSentinel;
   }
+#pragma unroll
+  for (int q = 0; q < kBatch; ++q) s[q * kLocalThreads + (int)threadIdx.x] = w[q];
   __syncthreads();
-  int M = B;  // words the network sorts
-  if (p.filter) {
-    // Only the first `need` words are wanted. Each wave takes the r-th
-    // smallest of its lanes' minima (r = need / waves, rounded up): the wave
-    // then holds r distinct words at or below it, so the largest of the
-    // waves' values, T, has at least `need` words at or below it, and every
-    // word below the need-th is <= T. Only the words <= T are sorted.
-    __shared__ uint64_t wave_t[kLocalThreads / 64];
-    __shared__ uint32_t cnt;
-    const int need = static_cast<int>(p.write_out ? p.g.out_n : p.keep);
-    const int waves = bd / 64, wv = static_cast<int>(threadIdx.x) / 64;
-    const int r = (need + waves - 1) / waves;
-    // B is a multiple of the workgroup size (both powers of two, B >= 256),
-    // so `q < nm` is uniform across the workgroup.
-    constexpr int kMine = kSortBlock / kLocalThreads;
-    const int nm = B / bd;
-    uint64_t mine[kMine];
-    uint64_t lo = kSentinel;
-#pragma unroll
-    for (int q = 0; q < kMine; ++q) {
-      if (q < nm) {
-        mine[q] = s[threadIdx.x + q * bd];
-        lo = mine[q] < lo ? mine[q] : lo;
-      }
-    }
-    if (threadIdx.x == 0) cnt = 0;
-    uint64_t t = kSentinel, v = lo;
-    for (int round = 0; round < r; ++round) {
-      t = wave_min_u64(v);
-      const uint64_t owner = __ballot(v == t);  // words are distinct: one lane, or none once all are sentinels
-      if (static_cast<int>(__lane_id()) == __ffsll(static_cast<unsigned long long>(owner)) - 1) v = kSentinel;
-    }
-    if (__lane_id() == 0) wave_t[wv] = t;
-    __syncthreads();
-    uint64_t T = 0;
-    for (int w = 0; w < waves; ++w) T = wave_t[w] > T ? wave_t[w] : T;
-#pragma unroll
-    for (int q = 0; q < kMine; ++q) {
-      if (q >= nm) break;
-      // One LDS atomic per wave: the wave's slots, then each lane's rank.
-      const bool take = mine[q] <= T;
-      const uint64_t mask = __ballot(take);
-      if (mask) {
-        uint32_t base = 0;
-        if (__lane_id() == 0) base = atomicAdd(&cnt, static_cast<uint32_t>(__popcll(mask)));
-        base = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(base)));
-        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
-        if (take) s[base + rank] = mine[q];
-      }
-    }
-    __syncthreads();
-    const int m = static_cast<int>(cnt);
-    M = 2;
-    while (M < m) M <<= 1;
-    for (int i = m + threadIdx.x; i < M; i += bd) s[i] = kSentinel;
-    __syncthreads();
-  }
-  for (int64_t k = p.k_first; k <= (p.filter ? M : p.k_last); k <<= 1) {
+  for (int64_t k = p.k_first; k <= p.k_last; k <<= 1) {
     // Within a block only bit log2(k) of the row position matters: it is the
-    // block's (base & k) when k >= B, else the position's own bit.
-    const bool block_up = !p.global_dir || k < B || (base & k) == 0;
-    const int kb = k < B ? static_cast<int>(k) : 0;
+    // block's (base & k) when k >= kSortBlock, else the position's own bit.
+    const bool block_up = k < kSortBlock || (base & k) == 0;
+    const int kb = k < kSortBlock ? static_cast<int>(k) : 0;
     for (int64_t jj = (k == p.k_first ? p.j_first : k >> 1); jj > 0; jj >>= 1) {
       const int j = static_cast<int>(jj);
-      for (int t = threadIdx.x; t < M / 2; t += blockDim.x) {
+      for (int t = threadIdx.x; t < kSortBlock / 2; t += kLocalThreads) {
         const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
         const int l = i | j;
         const bool up = block_up == ((i & kb) == 0);
@@ -234,13 +149,9 @@ __global__ void __launch_bounds__(kLocalThreads) sort_local_kernel(LocalPass p) 
       __syncthreads();
     }
   }
-  if (p.write_out) {
-    for (int i = threadIdx.x; i < p.g.out_n; i += blockDim.x)
-      gather_one(p.g, p.r, row, i, static_cast<int64_t>(s[i] & 0xffffffffu));
-  } else {
-    uint64_t* dst = p.dst + row * p.dst_stride + blk * p.keep;
-    for (int i = threadIdx.x; i < p.keep; i += blockDim.x) dst[i] = s[i];
-  }
+#pragma unroll
+  for (int q = 0; q < kBatch; ++q)
+    p.dst[row * p.row_len + base + q * kLocalThreads + (int)threadIdx.x] = s[q * kLocalThreads + (int)threadIdx.x];
 }
 
 __global__ void bitonic_global_kernel(uint64_t* a, int64_t rows, int64_t p, int64_t k, int64_t j) {
@@ -266,6 +177,578 @@ __global__ void sort_write_kernel(const uint64_t* list, int64_t list_stride, Sor
   gather_one(g, r, row, i, static_cast<int64_t>(list[row * list_stride + i] & 0xffffffffu));
 }
 
+// ------------------------------------------------------------ merge sort
+// A word is the 32-bit key image over 30 bits of position, 62 bits, held as a
+// double: with the top two bits zero it is a finite non-negative double whose
+// order is the word's, so a compare-exchange is one v_min_f64 and one
+// v_max_f64 (a 64-bit integer one is a compare and four selects).
+constexpr int kGroup = 8;           // words loaded together
+constexpr int kSortThreads = 512;   // sort_block's largest workgroup, 16 words a thread
+constexpr int kSortTile = 16 * kSortThreads;
+constexpr int kMergeThreads = 512;
+constexpr int kMergeItems = 8;
+constexpr int kMergeTile = kMergeItems * kMergeThreads;
+constexpr int64_t kWordRows = int64_t{1} << 30;  // positions a word holds
+constexpr uint64_t kWordEnd = (uint64_t{1} << 62) - 1;  // after every word
+
+__device__ __forceinline__ double as_word(uint64_t u) { return __builtin_bit_cast(double, u); }
+__device__ __forceinline__ uint64_t word_bits(double w) { return __builtin_bit_cast(uint64_t, w); }
+__device__ __forceinline__ double make_word(uint32_t image, int64_t pos) {
+  return as_word(((uint64_t)image << 30) | (uint64_t)pos);
+}
+__device__ __forceinline__ int64_t word_pos(double w) { return (int64_t)(word_bits(w) & (uint64_t)(kWordRows - 1)); }
+__device__ __forceinline__ uint32_t word_image(double w) { return (uint32_t)(word_bits(w) >> 30); }
+
+__device__ __forceinline__ void order2(double& a, double& b) {
+  double lo, hi;
+  asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+  asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+  a = lo;
+  b = hi;
+}
+// The words in ascending order (Batcher's odd-even merge sort, 1968: 19 / 63
+// compare-exchanges for 8 / 16 words).
+template <int N>
+__device__ __forceinline__ void sort_words(double (&w)[N]) {
+#pragma unroll
+  for (int p = 1; p < N; p *= 2)
+#pragma unroll
+    for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+      for (int j = k % p; j + k < N; j += 2 * k)
+#pragma unroll
+        for (int i = 0; i < k; ++i)
+          if (i + j + k < N && (i + j) / (2 * p) == (i + j + k) / (2 * p)) order2(w[i + j], w[i + j + k]);
+}
+// An ascending then descending sequence of N words in ascending order.
+template <int N>
+__device__ __forceinline__ void merge_words(double (&w)[N]) {
+#pragma unroll
+  for (int d = N / 2; d > 0; d >>= 1)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (!(i & d)) order2(w[i], w[i | d]);
+}
+
+// LDS slot of word i: one word of padding per eight, so that threads storing
+// eight neighbouring words each hit different banks.
+__device__ __forceinline__ int slot(int i) { return i + (i >> 3); }
+constexpr size_t words_lds(int n) { return (size_t)(n + n / 8) * 8; }
+
+// Words of A[0, la) among the first d of A and B[0, lb) merged (A first on
+// ties); a and b are the runs' first LDS word indices.
+__device__ __forceinline__ int merge_split(const double* s, int a, int la, int b, int lb, int d) {
+  int lo = max(0, d - lb), hi = min(d, la);
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (s[slot(a + mid)] <= s[slot(b + d - 1 - mid)]) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// The thread's N merged words from diagonal d: na from A at a0, the rest from
+// B at b0, read as one ascending and descending sequence.
+template <int N>
+__device__ __forceinline__ void merge_take(const double* s, int a0, int na, int b0, double (&w)[N]) {
+  const int b1 = b0 + N - 1;
+#pragma unroll
+  for (int i = 0; i < N; ++i) w[i] = s[slot(i < na ? a0 + i : b1 - i)];
+  merge_words(w);
+}
+
+// Raw key of an image (images are invertible except for kSortKeyFloat).
+__device__ __forceinline__ uint32_t key_of_image(uint32_t img, const SortRows& r) {
+  const uint32_t mask = r.key_bits == 32 ? 0xffffffffu : ((1u << r.key_bits) - 1u);
+  const uint32_t sign = 1u << (r.key_bits - 1);
+  if (r.descending) img = ~img & mask;
+  if (r.key_class == kSortKeySigned) return img ^ sign;
+  if (r.key_class == kSortKeyUnsigned) return img;
+  return (img & sign) ? img ^ sign : ~img & mask;
+}
+
+// Result i of `row` from a sorted word.
+__device__ __forceinline__ void write_result(const SortGather& g, const SortRows& r, int64_t row, int64_t i, double w) {
+  const int64_t pos = word_pos(w);
+  const int64_t outer = r.inner == 1 ? row : row / r.inner, j = row - outer * r.inner;
+  const int64_t from = (outer * r.n + pos) * r.inner + j;
+  const int64_t d = (outer * g.out_n + i) * r.inner + j;
+  for (int o = 0; o < g.count; ++o) {
+    uint64_t v = 0;
+    if (!g.src[o]) {
+      v = (uint64_t)pos;
+    } else if (o == 0 && r.key_class != kSortKeyFloat) {
+      v = key_of_image(word_image(w), r);
+    } else {
+      switch (g.elem_bytes[o]) {
+        case 1: v = static_cast<const uint8_t*>(g.src[o])[from]; break;
+        case 2: v = static_cast<const uint16_t*>(g.src[o])[from]; break;
+        case 4: v = static_cast<const uint32_t*>(g.src[o])[from]; break;
+        default: v = static_cast<const uint64_t*>(g.src[o])[from]; break;
+      }
+    }
+    switch (g.elem_bytes[o]) {
+      case 1: static_cast<uint8_t*>(g.dst[o])[d] = (uint8_t)v; break;
+      case 2: static_cast<uint16_t*>(g.dst[o])[d] = (uint16_t)v; break;
+      case 4: static_cast<uint32_t*>(g.dst[o])[d] = (uint32_t)v; break;
+      default: static_cast<uint64_t*>(g.dst[o])[d] = v; break;
+    }
+  }
+  if (g.index_dst) static_cast<int32_t*>(g.index_dst)[d] = static_cast<int32_t>(pos);
+}
+
+// Where a pass reads a row's words: the raw keys, or a list of words.
+struct WordSource {
+  const void* keys = nullptr;
+  const double* list = nullptr;
+  int64_t len = 0;      // words of a row
+  int64_t stride = 0;   // list: words from one row to the next
+  int vec = 0;          // keys: 16-byte loads (inner == 1, rows 16-byte aligned)
+};
+
+// The images of the thread's eight of keys [base, base + 8 threads) of a row
+// (any of them, since a word carries its position): key e is at position
+// base + key_at(src, tid, threads, e), past the row when that is >= src.len.
+__device__ __forceinline__ int key_at(const WordSource& src, int tid, int threads, int e) {
+  return src.vec ? tid * kGroup + e : tid + e * threads;
+}
+__device__ __forceinline__ void load_images(const WordSource& src, const SortRows& r, const KeyMap& map, int64_t row,
+                                            int64_t base, int tid, int threads, uint32_t (&img)[kGroup]) {
+  const int64_t end = src.len;
+  uint32_t raw[kGroup];
+  if (src.vec) {
+    // Eight neighbouring keys: one 16-byte load of 16-bit keys, two of 32-bit.
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    const int64_t pos = base + (int64_t)tid * kGroup;
+    const char* from = static_cast<const char*>(src.keys) + (row * r.n + pos) * (r.key_bits / 8);
+    // n is a multiple of the load: a load lies inside the row or past it.
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    const u32x4 v0 = pos < end ? *reinterpret_cast<const u32x4*>(from) : zero;
+    if (r.key_bits == 32) {
+      const u32x4 v1 = pos + 4 < end ? *reinterpret_cast<const u32x4*>(from + 16) : zero;
+#pragma unroll
+      for (int e = 0; e < kGroup; ++e) raw[e] = e < 4 ? v0[e & 3] : v1[e & 3];
+    } else {
+#pragma unroll
+      for (int e = 0; e < kGroup; ++e) raw[e] = (v0[e >> 1] >> ((e & 1) * 16)) & 0xffffu;
+    }
+  } else {
+    const int64_t outer = row / r.inner, j = row - outer * r.inner;
+    const int64_t row0 = outer * r.n * r.inner + j;
+#pragma unroll
+    for (int e = 0; e < kGroup; ++e) {
+      const int64_t i = base + tid + (int64_t)e * threads;
+      raw[e] = i < end ? load_key(src.keys, row0 + i * r.inner, r.key_bits) : 0u;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < kGroup; ++e) img[e] = key_image(raw[e], map);
+}
+
+// The thread's eight of words [base, base + 8 threads) of a row.
+__device__ __forceinline__ void load_words(const WordSource& src, const SortRows& r, int64_t row, int64_t base, int tid,
+                                           int threads, double (&w)[kGroup]) {
+  if (src.list) {
+    const double* p = src.list + row * src.stride;
+#pragma unroll
+    for (int e = 0; e < kGroup; ++e) {
+      const int64_t i = base + e * threads + tid;
+      w[e] = i < src.len ? p[i] : as_word(kWordEnd);
+    }
+    return;
+  }
+  uint32_t img[kGroup];
+  load_images(src, r, key_map(r), row, base, tid, threads, img);
+#pragma unroll
+  for (int e = 0; e < kGroup; ++e) {
+    const int64_t i = base + key_at(src, tid, threads, e);
+    w[e] = i < src.len ? make_word(img[e], i) : as_word(kWordEnd);
+  }
+}
+
+// Orders the wave's own LDS writes before its reads (a wave's LDS operations
+// run in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+struct BlockPass {
+  SortRows r;
+  WordSource src;
+  int64_t blocks_per_row = 1;
+  double* dst = nullptr;      // the first `keep` words of each block; null: the results
+  int64_t keep = 0, dst_stride = 0;
+  SortGather g;
+};
+
+// One block of N blockDim words. A merge round finds each thread's split of
+// the pair's two runs (a binary search), then reads its N words in one LDS
+// latency and merges them in registers. Rounds within a wave's words need no
+// barrier. Bound by instruction issue, most of it the searches (which is why
+// a thread holds 16 words and not 8, unless rows are short). Whole sorts with
+// positions, bitonic blocks and passes before -> now: [4096, 1024] 101 -> 45 us,
+// [64, 32000] 187 -> 57, [64, 128256] bf16 735 -> 212, [1, 2^20] 329 -> 116.
+template <int N>
+__global__ void __launch_bounds__(kSortThreads) sort_block_kernel(BlockPass p) {
+  extern __shared__ double sw[];
+  __shared__ int part[kSortThreads + 1];
+  const int64_t row = blockIdx.x / p.blocks_per_row;
+  const int64_t blk = blockIdx.x - row * p.blocks_per_row;
+  const int threads = (int)blockDim.x, tid = (int)threadIdx.x;
+  const int64_t base = blk * (threads * N);
+  double w[N];
+#pragma unroll
+  for (int q = 0; q < N / kGroup; ++q) {
+    double g[kGroup];
+    load_words(p.src, p.r, row, base + q * threads * kGroup, tid, threads, g);
+#pragma unroll
+    for (int e = 0; e < kGroup; ++e) w[q * kGroup + e] = g[e];
+  }
+  sort_words(w);
+  const int mine = tid * N;
+#pragma unroll
+  for (int e = 0; e < N; ++e) sw[slot(mine + e)] = w[e];
+  for (int run = N; run < threads * N; run *= 2) {
+    const bool wave = 2 * run <= 64 * N;
+    if (wave) wave_sync();
+    else __syncthreads();
+    const int pair = mine & ~(2 * run - 1), d = mine - pair;
+    const int a = merge_split(sw, pair, run, pair + run, run, d);
+    int a1;
+    if (wave) {
+      a1 = __shfl_down(a, 1, 64);
+    } else {
+      part[tid] = a;
+      __syncthreads();
+      a1 = part[tid + 1];
+    }
+    if (d + N == 2 * run) a1 = run;
+    merge_take(sw, pair + a, a1 - a, pair + run + d - a, w);
+    if (wave) wave_sync();
+    else __syncthreads();
+#pragma unroll
+    for (int e = 0; e < N; ++e) sw[slot(mine + e)] = w[e];
+  }
+  __syncthreads();
+  if (p.dst) {
+    double* dst = p.dst + row * p.dst_stride + blk * p.keep;
+    const int64_t n = min(p.keep, p.dst_stride - blk * p.keep);
+    for (int i = tid; i < n; i += threads) dst[i] = sw[slot(i)];
+  } else {
+    for (int i = tid; i < p.g.out_n; i += threads) write_result(p.g, p.r, row, i, sw[slot(i)]);
+  }
+}
+
+struct MergePass {
+  SortRows r;
+  const double* src = nullptr;
+  double* dst = nullptr;       // null: the results (one pair a row)
+  int64_t len = 0, run = 0;    // words of a row (the rows' stride), sorted run length
+  int64_t tiles_per_row = 1;
+  SortGather g;
+};
+
+// Words of A[0, la) among the first d merged, in HBM: the wave's lanes probe
+// 64 points of the range at a time.
+__device__ int64_t merge_split_wave(const double* A, int64_t la, const double* B, int64_t lb, int64_t d) {
+  int64_t lo = max((int64_t)0, d - lb), hi = min(d, la);
+  const int lane = (int)__lane_id();
+  while (lo < hi) {
+    const int64_t step = (hi - lo + 63) / 64, mid = lo + lane * step;
+    const bool take = mid < hi && A[mid] <= B[d - 1 - mid];
+    const int n = __popcll(__ballot(take));  // true up to the split, then false
+    const int64_t from = lo;
+    if (n == 0) hi = lo;
+    else {
+      lo = from + (n - 1) * step + 1;
+      hi = min(from + n * step, hi);
+    }
+  }
+  return lo;
+}
+
+// Output words [tile, tile + kMergeTile) of a pair of runs: the tile's parts
+// of both runs are staged in LDS and merged as in sort_block.
+__global__ void __launch_bounds__(kMergeThreads) merge_runs_kernel(MergePass p) {
+  __shared__ double sw[kMergeTile + kMergeTile / 8];
+  __shared__ int part[kMergeThreads + 1];
+  __shared__ int64_t ends[2];
+  const int64_t row = blockIdx.x / p.tiles_per_row;
+  const int64_t t0 = (blockIdx.x - row * p.tiles_per_row) * kMergeTile;
+  // Runs are multiples of the tile: a tile lies in one pair.
+  const int64_t pair = t0 / (2 * p.run) * (2 * p.run);
+  const double* A = p.src + row * p.len + pair;
+  const double* B = A + p.run;
+  const int64_t la = min(p.run, p.len - pair), lb = max((int64_t)0, min(p.run, p.len - pair - p.run));
+  const int64_t d0 = t0 - pair, d1 = min(d0 + kMergeTile, la + lb);
+  const int tid = (int)threadIdx.x, wave = tid >> 6;
+  if (wave < 2) {
+    const int64_t e = merge_split_wave(A, la, B, lb, wave == 0 ? d0 : d1);
+    if ((tid & 63) == 0) ends[wave] = e;
+  }
+  __syncthreads();
+  const int64_t a0 = ends[0], b0 = d0 - a0;
+  const int na = (int)(ends[1] - a0), n = (int)(d1 - d0), nb = n - na;
+#pragma unroll
+  for (int e = 0; e < kMergeItems; ++e) {
+    const int i = e * kMergeThreads + tid;
+    if (i < n) sw[slot(i)] = i < na ? A[a0 + i] : B[b0 + i - na];
+  }
+  __syncthreads();
+  const int d = min(tid * kMergeItems, n);
+  const int a = merge_split(sw, 0, na, na, nb, d);
+  part[tid] = a;
+  __syncthreads();
+  const int d_end = min(d + kMergeItems, n), a1 = d_end == n ? na : part[tid + 1];
+  // The last thread with words may have fewer than its share: its B part then
+  // starts later in the sequence, behind ends of the order.
+  double w[kMergeItems];
+  const int take_a = a1 - a, take_b = d_end - d - take_a;
+#pragma unroll
+  for (int i = 0; i < kMergeItems; ++i) {
+    const int k = kMergeItems - 1 - i;
+    w[i] = i < take_a ? sw[slot(a + i)] : k < take_b ? sw[slot(na + d - a + k)] : as_word(kWordEnd);
+  }
+  merge_words(w);
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kMergeItems; ++e)
+    if (d + e < d_end) sw[slot(d + e)] = w[e];
+  __syncthreads();
+  if (p.dst) {
+    double* dst = p.dst + row * p.len + t0;
+    for (int i = tid; i < n; i += kMergeThreads) dst[i] = sw[slot(i)];
+  } else {
+    for (int i = tid; i < n && t0 + i < p.g.out_n; i += kMergeThreads) write_result(p.g, p.r, row, t0 + i, sw[slot(i)]);
+  }
+}
+
+// ---------------------------------------------------------------- top-k
+// The first `need` <= 256 words of a chunk of 256 * kShare * 8 words. Threads
+// (or, for 16-bit keys, groups of one, two or four) take the least of their
+// words; the need-th smallest of these, T, has at least `need` words at or
+// below it, and usually little more: only those are ranked, by counting, which
+// also orders them. No network over the chunk, no histogram: one pass over the
+// keys in registers. Larger groups give fewer values to rank (64 for need <= 56)
+// and a few more candidates.
+constexpr int kTopkThreads = 256;
+constexpr int kTopkMax = 256;
+struct TopkPass {
+  SortRows r;
+  WordSource src;
+  int64_t blocks_per_row = 1;
+  int need = 0;
+  int group = 1;           // topk_half: threads per group, at least `need` groups
+  double* dst = nullptr;   // `need` words of each block; null: the results
+  SortGather g;
+};
+struct TopkLds {
+  double least[kTopkThreads];
+  double bound;
+  uint32_t bound_image;
+  int count;
+};
+
+// The candidates' ranks (distinct words): rank k is result k. The threads of a
+// candidate count over a segment of the list each, eight words at a time; the
+// list holds kTopkPad more words than candidates, filled with ends.
+constexpr int kTopkPad = 64;
+__device__ __forceinline__ void topk_rank(const TopkPass& p, int64_t row, int64_t blk, int tid, int m, double* cand) {
+  double* dst = p.dst ? p.dst + (row * p.blocks_per_row + blk) * p.need : nullptr;
+  const int lg = m <= 32 ? 3 : m <= 64 ? 2 : m <= 128 ? 1 : 0;
+  const int seg = (((m + (1 << lg) - 1) >> lg) + 7) & ~7;  // at most 63 words past m in all
+  if (tid < (seg << lg) - m) cand[m + tid] = as_word(kWordEnd);
+  __syncthreads();
+  const int sub = tid & ((1 << lg) - 1);
+  for (int c = tid >> lg; c < m; c += kTopkThreads >> lg) {
+    const double x = cand[c];
+    const double* part = cand + sub * seg;
+    int k = 0;
+    for (int i = 0; i < seg; i += 8) {
+      double z[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) z[e] = part[i + e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) k += z[e] < x ? 1 : 0;
+    }
+    if (lg > 0) k += __shfl_xor(k, 1, 64);
+    if (lg > 1) k += __shfl_xor(k, 2, 64);
+    if (lg > 2) k += __shfl_xor(k, 4, 64);
+    if (sub == 0 && k < p.need) {
+      if (dst) dst[k] = x;
+      else write_result(p.g, p.r, row, k, x);
+    }
+  }
+  if (dst)
+    for (int i = m + tid; i < p.need; i += kTopkThreads) dst[i] = as_word(kWordEnd);
+}
+
+// The words at or below T of 256 threads' kShare * 8 words each: T is the
+// need-th smallest of the threads' own least words, so at most need * 8 *
+// kShare words go to `cand`. Returns how many.
+template <int kShare>
+__device__ __forceinline__ int topk_bound(const double (&w)[kShare][kGroup], int need, int tid, TopkLds& lds, double* cand) {
+  const double end = as_word(kWordEnd);
+  double lo = end;
+#pragma unroll
+  for (int q = 0; q < kShare; ++q)
+#pragma unroll
+    for (int e = 0; e < kGroup; ++e) asm("v_min_f64 %0, %0, %1" : "+v"(lo) : "v"(w[q][e]));
+  lds.least[tid] = lo;
+  if (tid == 0) {
+    lds.bound = as_word(kWordEnd - 1);  // fewer than `need` threads hold words: all of them
+    lds.count = 0;
+  }
+  __syncthreads();
+  int rank = 0;
+#pragma unroll 8
+  for (int i = 0; i < kTopkThreads; ++i) rank += lds.least[i] < lo ? 1 : 0;
+  if (rank == need - 1 && lo < end) lds.bound = lo;
+  __syncthreads();
+  const double T = lds.bound;
+  if (lo <= T) {
+#pragma unroll
+    for (int q = 0; q < kShare; ++q)
+#pragma unroll
+      for (int e = 0; e < kGroup; ++e)
+        if (w[q][e] <= T) cand[atomicAdd(&lds.count, 1)] = w[q][e];
+  }
+  __syncthreads();
+  return lds.count;
+}
+
+// Any source.
+template <int kShare>
+__device__ __forceinline__ int topk_words(const TopkPass& p, int64_t row, int64_t blk, int tid, TopkLds& lds, double* cand) {
+  double w[kShare][kGroup];
+#pragma unroll
+  for (int q = 0; q < kShare; ++q)
+    load_words(p.src, p.r, row, (blk * kShare + q) * (kTopkThreads * kGroup), tid, kTopkThreads, w[q]);
+  return topk_bound<kShare>(w, p.need, tid, lds, cand);
+}
+
+template <int kShare>
+__global__ void __launch_bounds__(kTopkThreads) topk_select_kernel(TopkPass p) {
+  extern __shared__ double cand[];  // need * kShare * kGroup + kTopkPad words
+  __shared__ TopkLds lds;
+  const int64_t row = blockIdx.x / p.blocks_per_row;
+  const int64_t blk = blockIdx.x - row * p.blocks_per_row;
+  const int m = topk_words<kShare>(p, row, blk, (int)threadIdx.x, lds, cand);
+  topk_rank(p, row, blk, (int)threadIdx.x, m, cand);
+}
+
+// 16-bit keys (not FLOAT-compared) in 16-byte aligned rows: the images, the
+// least of them and the test against T two keys an instruction, on packed
+// 16-bit integers. T is the least image with `need` groups at or below it, so
+// every key of T's image is a candidate; the few candidates are read again and
+// made words. Many candidates (ties, or neighbouring keys that are all large)
+// are bounded again as words.
+// [64, 128256] bf16, k = 50: 69 us with bitonic blocks, 25 on words, 20 now
+// (both launches).
+template <int kShare>
+__global__ void __launch_bounds__(kTopkThreads) topk_half_kernel(TopkPass p) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  typedef short ss2 __attribute__((ext_vector_type(2)));
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int kPairs = 4 * kShare;  // packed registers a thread
+  constexpr int kChunk = kTopkThreads * kShare * kGroup;
+  extern __shared__ double cand[];  // need * kShare * kGroup + kTopkPad words
+  __shared__ TopkLds lds;
+  const int64_t row = blockIdx.x / p.blocks_per_row;
+  const int64_t blk = blockIdx.x - row * p.blocks_per_row;
+  const int tid = (int)threadIdx.x;
+  const int64_t base = blk * kChunk;
+  const int keys = (int)min((int64_t)kChunk, p.src.len - base);  // a multiple of 8
+  const uint16_t* from = static_cast<const uint16_t*>(p.src.keys) + row * p.r.n + base;
+  const KeyMap map = key_map(p.r);
+  const uint32_t neg2 = map.neg * 0x10001u, pos2 = map.pos * 0x10001u;
+  u32x4 v[kShare];
+#pragma unroll
+  for (int q = 0; q < kShare; ++q) {
+    const int at = q * (kTopkThreads * kGroup) + tid * kGroup;
+    v[q] = *reinterpret_cast<const u32x4*>(from + (at < keys ? at : 0));
+  }
+  uint32_t img[kPairs];
+  us2 least2 = {0xffff, 0xffff};
+#pragma unroll
+  for (int j = 0; j < kPairs; ++j) {
+    const bool in = (j / 4) * (kTopkThreads * kGroup) + tid * kGroup < keys;
+    const uint32_t raw = v[j / 4][j % 4];
+    const uint32_t sign = __builtin_bit_cast(uint32_t, (ss2)(__builtin_bit_cast(ss2, raw) >> 15));
+    img[j] = in ? raw ^ ((sign & neg2) | (~sign & pos2)) : 0xffffffffu;
+    least2 = __builtin_elementwise_min(least2, __builtin_bit_cast(us2, img[j]));
+  }
+  uint32_t lo = min((uint32_t)least2[0], (uint32_t)least2[1]);
+  for (int d = 1; d < p.group; d *= 2) lo = min(lo, (uint32_t)__shfl_xor((int)lo, d, 64));
+  uint32_t* least = reinterpret_cast<uint32_t*>(lds.least);
+  if (tid % p.group == 0) least[tid / p.group] = lo;
+  if (tid == 0) {
+    lds.bound_image = 0xffffu;
+    lds.count = 0;
+  }
+  __syncthreads();
+  int le = 0;
+#pragma unroll 4
+  for (int i = 0; i < kTopkThreads / p.group; i += 4) {
+    const u32x4 x = *reinterpret_cast<const u32x4*>(least + i);
+    le += (x[0] <= lo ? 1 : 0) + (x[1] <= lo ? 1 : 0) + (x[2] <= lo ? 1 : 0) + (x[3] <= lo ? 1 : 0);
+  }
+  if (le >= p.need) atomicMin(&lds.bound_image, lo);
+  __syncthreads();
+  const uint32_t T = lds.bound_image;
+  const us2 T2 = {(unsigned short)T, (unsigned short)T}, one = {1, 1};
+  // Bit kPairs - 1 - j of the low half: pair j's low key is above T; of the
+  // high half, its high key.
+  uint32_t above = 0;
+#pragma unroll
+  for (int j = 0; j < kPairs; ++j) {
+    const us2 over = __builtin_elementwise_sub_sat(__builtin_bit_cast(us2, img[j]), T2);
+    above = (above << 1) | __builtin_bit_cast(uint32_t, (us2)__builtin_elementwise_min(over, one));
+  }
+  uint32_t bits = ~above & (((1u << kPairs) - 1u) * 0x10001u);
+#pragma unroll
+  for (int q = 0; q < kShare; ++q)
+    if (q * (kTopkThreads * kGroup) + tid * kGroup >= keys) bits &= ~((0xfu << (kPairs - 4 - 4 * q)) * 0x10001u);
+  const int room = p.need * kShare * kGroup;
+  int to = bits ? atomicAdd(&lds.count, __popc(bits)) : 0;
+  while (bits) {
+    const int k = __ffs(bits) - 1;
+    bits &= bits - 1;
+    const int j = kPairs - 1 - (k & 15);
+    const int at = (j >> 2) * (kTopkThreads * kGroup) + tid * kGroup + (j & 3) * 2 + (k >> 4);
+    if (to < room) reinterpret_cast<int*>(cand + to)[0] = at;
+    ++to;
+  }
+  __syncthreads();
+  int m = lds.count;
+  if (m > room) {
+    __syncthreads();
+    m = topk_words<kShare>(p, row, blk, tid, lds, cand);
+  } else {
+    // Every candidate's key in one round of loads.
+    for (int c = tid; c < m; c += kTopkThreads) {
+      const int at = reinterpret_cast<const int*>(cand + c)[0];
+      cand[c] = make_word(key_image(from[at], map), base + at);
+    }
+    __syncthreads();
+    if (m > 2 * p.need + kTopkThreads / 2) {
+      double w[kShare][kGroup];
+#pragma unroll
+      for (int q = 0; q < kShare; ++q)
+#pragma unroll
+        for (int e = 0; e < kGroup; ++e) {
+          const int c = (q * kGroup + e) * kTopkThreads + tid;  // room <= 256 * 8 * kShare
+          w[q][e] = c < m ? cand[c] : as_word(kWordEnd);
+        }
+      __syncthreads();
+      m = topk_bound<kShare>(w, p.need, tid, lds, cand);
+    }
+  }
+  topk_rank(p, row, blk, tid, m, cand);
+}
+
 int64_t pow2_at_least(int64_t v) {
   int64_t p = 1;
   while (p < v) p <<= 1;
@@ -280,105 +763,187 @@ void check_launch(const char* what) {
 void local(hipStream_t s, const LocalPass& p, int64_t rows) {
   const int64_t grid = rows * p.blocks_per_row;
   PJRTX_CHECK(grid > 0 && grid < (int64_t{1} << 31), Code::kUnimplemented, "sort: too many rows");
-  const int threads = static_cast<int>(std::min<int64_t>(kLocalThreads, std::max<int64_t>(64, p.block / 2)));
-  hipLaunchKernelGGL(sort_local_kernel, dim3(static_cast<unsigned>(grid)), dim3(threads), 0, s, p);
+  hipLaunchKernelGGL(sort_local_kernel, dim3(static_cast<unsigned>(grid)), dim3(kLocalThreads), 0, s, p);
   check_launch("sort_local");
 }
 
-// Words of scratch for each path (0 when one LDS block holds a row).
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The kernels a row's sort takes and their scratch.
+enum SortPath {
+  kPathTopk,    // topk_select rounds
+  kPathKeep,    // sort_block rounds that keep the first out_n words of a block
+  kPathMerge,   // sort_block, then merge_runs
+  kPathBitonic  // padded rows in one buffer
+};
 struct Layout {
-  int path = 0;                // 0: one block; 1: top-k reduction; 2: full bitonic
-  int64_t kp = 0, len1 = 0;    // top-k: words kept per block, list length after round one
-  int64_t p = 0;               // full: padded row length
+  SortPath path = kPathMerge;
+  int share = 1;               // topk: eight-word groups a thread
+  int64_t len1 = 0;            // topk / keep: list length after round one
+  int64_t p = 0;               // bitonic: padded row length
+  size_t bytes = 0;
 };
 
-Layout layout_of(const SortRows& r, int64_t out_n) {
+// Words a topk thread holds (in eights): a row that one chunk holds goes to
+// one launch; else enough workgroups for the GPU (1024), then long chunks,
+// whose lists are shorter.
+int topk_share(const SortRows& r, int64_t len) {
+  for (int one = 1; one <= 4; one *= 2)
+    if (len <= kTopkThreads * kGroup * one) return one;
+  int share = 4;
+  while (share > 1 && r.rows * ceil_div(len, kTopkThreads * kGroup * share) < 1024) share /= 2;
+  return share;
+}
+int64_t topk_blocks(int share, int64_t len) { return ceil_div(len, kTopkThreads * kGroup * share); }
+
+Layout layout_of(const SortRows& r, int64_t out_n, int64_t max_bytes) {
   Layout L;
-  if (r.n <= kSortBlock) return L;
-  L.kp = pow2_at_least(std::max<int64_t>(out_n, 1));
-  if (out_n < r.n && L.kp <= kSortBlock / 2) {
-    L.path = 1;
-    L.len1 = (r.n + kSortBlock - 1) / kSortBlock * L.kp;
+  const auto bitonic = [&] {
+    L.path = kPathBitonic;
+    L.p = std::max<int64_t>(pow2_at_least(r.n), kSortBlock);
+    L.bytes = static_cast<size_t>(r.rows * L.p) * 8;
+    return L;
+  };
+  if (r.n >= kWordRows) return bitonic();
+  if (out_n < r.n && out_n <= kTopkMax) {
+    L.path = kPathTopk;
+    L.share = topk_share(r, r.n);
+    const int64_t blocks = topk_blocks(L.share, r.n);
+    L.len1 = blocks * out_n;
+    L.bytes = blocks > 1 ? static_cast<size_t>(2 * r.rows * L.len1) * 8 : 0;
+  } else if (r.n > kSortTile && out_n <= kSortTile / 2) {
+    L.path = kPathKeep;
+    L.len1 = ceil_div(r.n, kSortTile) * out_n;
+    L.bytes = static_cast<size_t>(2 * r.rows * L.len1) * 8;
   } else {
-    L.path = 2;
-    L.p = pow2_at_least(r.n);
+    // One buffer per side of a merge round; the last round writes the results.
+    L.bytes = r.n <= kSortTile ? 0 : static_cast<size_t>((r.n <= 2 * kSortTile ? 1 : 2) * r.rows * r.n) * 8;
+    if (static_cast<int64_t>(L.bytes) > max_bytes) return bitonic();
   }
   return L;
 }
 
-}  // namespace
-
-size_t sort_scratch_bytes(const SortRows& r, int64_t out_n) {
-  const Layout L = layout_of(r, out_n);
-  if (L.path == 1) return static_cast<size_t>(2 * r.rows * L.len1) * 8;
-  if (L.path == 2) return static_cast<size_t>(r.rows * L.p) * 8;
-  return 0;
+unsigned grid_of(int64_t rows, int64_t per_row) {
+  const int64_t grid = rows * per_row;
+  PJRTX_CHECK(grid > 0 && grid < (int64_t{1} << 31), Code::kUnimplemented, "sort: too many rows");
+  return static_cast<unsigned>(grid);
 }
 
-void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGather& g, void* scratch) {
+// Blocks of `words` <= kSortTile words.
+void sort_blocks(hipStream_t s, const BlockPass& p, int64_t words) {
+  const int n = words <= 64 * kGroup ? kGroup : 16;
+  const int threads = static_cast<int>(std::max<int64_t>(64, pow2_at_least(ceil_div(words, n))));
+  const dim3 grid(grid_of(p.r.rows, p.blocks_per_row));
+  if (n == kGroup) hipLaunchKernelGGL((sort_block_kernel<kGroup>), grid, dim3(threads), words_lds(threads * n), s, p);
+  else hipLaunchKernelGGL((sort_block_kernel<16>), grid, dim3(threads), words_lds(threads * n), s, p);
+  check_launch("sort_block");
+}
+
+void topk_blocks_launch(hipStream_t s, TopkPass p, int share) {
+  const dim3 grid(grid_of(p.r.rows, p.blocks_per_row)), block(kTopkThreads);
+  const size_t lds = static_cast<size_t>(p.need * share * kGroup + kTopkPad) * 8;
+  p.group = p.need <= 56 ? 4 : p.need <= 112 ? 2 : 1;
+  const bool half = !p.src.list && p.src.vec && p.r.key_bits == 16 && p.r.key_class != kSortKeyFloat;
+#define PJRTX_TOPK(SHARE)                                                                  \
+  if (half) hipLaunchKernelGGL((topk_half_kernel<SHARE>), grid, block, lds, s, p);         \
+  else hipLaunchKernelGGL((topk_select_kernel<SHARE>), grid, block, lds, s, p)
+  if (share == 1) { PJRTX_TOPK(1); }
+  else if (share == 2) { PJRTX_TOPK(2); }
+  else { PJRTX_TOPK(4); }
+#undef PJRTX_TOPK
+  check_launch("topk_select");
+}
+
+}  // namespace
+
+size_t sort_scratch_bytes(const SortRows& r, int64_t out_n, int64_t max_bytes) {
+  return layout_of(r, out_n, max_bytes).bytes;
+}
+
+void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGather& g, void* scratch, int64_t max_bytes) {
   if (r.rows == 0 || r.n == 0 || g.out_n == 0) return;
   PJRTX_CHECK(r.n < (int64_t{1} << 31) && g.out_n <= r.n, Code::kInvalidArgument, "sort: row length out of range");
   PJRTX_CHECK(r.key_bits == 8 || r.key_bits == 16 || r.key_bits == 32, Code::kUnimplemented,
               "sort: keys wider than 32 bits are not supported");
-  const Layout L = layout_of(r, g.out_n);
+  const Layout L = layout_of(r, g.out_n, max_bytes);
+  WordSource src;
+  src.keys = keys;
+  src.len = r.n;
+  src.vec = r.inner == 1 && r.key_bits >= 16 && (r.n * r.key_bits / 8) % 16 == 0 && reinterpret_cast<uintptr_t>(keys) % 16 == 0;
+  double* a = static_cast<double*>(scratch);
+  double* b = a + r.rows * (L.path == kPathMerge ? r.n : L.len1);
+  if (L.path == kPathTopk) {
+    TopkPass p;
+    p.r = r;
+    p.src = src;
+    p.need = static_cast<int>(g.out_n);
+    p.g = g;
+    int share = L.share;
+    for (;;) {
+      p.blocks_per_row = topk_blocks(share, p.src.len);
+      p.dst = p.blocks_per_row == 1 ? nullptr : a;
+      topk_blocks_launch(s, p, share);
+      if (!p.dst) return;
+      p.src.list = a;
+      p.src.len = p.src.stride = p.blocks_per_row * p.need;
+      share = topk_share(r, p.src.len);
+      std::swap(a, b);
+    }
+  }
+  if (L.path == kPathKeep || L.path == kPathMerge) {
+    BlockPass p;
+    p.r = r;
+    p.src = src;
+    p.g = g;
+    if (r.n <= kSortTile) {
+      sort_blocks(s, p, r.n);
+      return;
+    }
+    p.blocks_per_row = ceil_div(r.n, kSortTile);
+    p.dst = a;
+    p.keep = L.path == kPathKeep ? g.out_n : kSortTile;
+    p.dst_stride = L.path == kPathKeep ? p.blocks_per_row * p.keep : r.n;
+    sort_blocks(s, p, kSortTile);
+    if (L.path == kPathKeep) {
+      for (;;) {
+        p.src.list = a;
+        p.src.len = p.src.stride = p.dst_stride;
+        if (p.src.len <= kSortTile) break;
+        p.blocks_per_row = ceil_div(p.src.len, kSortTile);
+        p.dst_stride = p.blocks_per_row * p.keep;
+        p.dst = b;
+        sort_blocks(s, p, kSortTile);
+        std::swap(a, b);
+      }
+      p.blocks_per_row = 1;
+      p.dst = nullptr;
+      sort_blocks(s, p, p.src.len);
+      return;
+    }
+    MergePass m;
+    m.r = r;
+    m.g = g;
+    m.len = r.n;
+    m.tiles_per_row = ceil_div(r.n, kMergeTile);
+    for (m.run = kSortTile; m.run < r.n; m.run *= 2) {
+      m.src = a;
+      m.dst = 2 * m.run >= r.n ? nullptr : b;
+      hipLaunchKernelGGL(merge_runs_kernel, dim3(grid_of(r.rows, m.tiles_per_row)), dim3(kMergeThreads), 0, s, m);
+      check_launch("merge_runs");
+      std::swap(a, b);
+    }
+    return;
+  }
+  // Bitonic network over L.p words per row: LDS passes for partner distances
+  // below kSortBlock, global passes for the rest.
+  uint64_t* buf = static_cast<uint64_t*>(scratch);
   LocalPass p;
   p.keys = keys;
   p.r = r;
-  p.g = g;
-  if (L.path == 0) {
-    p.block = static_cast<int>(pow2_at_least(std::max<int64_t>(r.n, 2)));
-    p.k_first = 2, p.k_last = p.block, p.j_first = 1;
-    p.write_out = 1;
-    p.filter = 8 * g.out_n <= p.block && p.block >= 256;
-    local(s, p, r.rows);
-    return;
-  }
-  uint64_t* buf = static_cast<uint64_t*>(scratch);
-  if (L.path == 1) {
-    // Round one from the keys, then rounds over the kept words.
-    uint64_t* a = buf;
-    uint64_t* b = buf + r.rows * L.len1;
-    p.block = kSortBlock;
-    p.blocks_per_row = (r.n + kSortBlock - 1) / kSortBlock;
-    p.k_first = 2, p.k_last = kSortBlock, p.j_first = 1;
-    p.keep = L.kp;
-    p.filter = 8 * L.kp <= kSortBlock;
-    p.dst = a;
-    p.dst_stride = L.len1;
-    local(s, p, r.rows);
-    int64_t len = L.len1, stride = L.len1;
-    while (len > kSortBlock) {
-      LocalPass q = p;
-      q.keys = nullptr;
-      q.list = a, q.list_len = len, q.list_stride = stride;
-      q.blocks_per_row = (len + kSortBlock - 1) / kSortBlock;
-      q.dst = b;
-      q.dst_stride = q.blocks_per_row * L.kp;
-      local(s, q, r.rows);
-      len = q.dst_stride, stride = q.dst_stride;
-      std::swap(a, b);
-    }
-    LocalPass f = p;
-    f.keys = nullptr;
-    f.list = a, f.list_len = len, f.list_stride = stride;
-    f.block = static_cast<int>(pow2_at_least(std::max<int64_t>(len, 2)));
-    f.blocks_per_row = 1;
-    f.k_first = 2, f.k_last = f.block, f.j_first = 1;
-    f.dst = nullptr;
-    f.write_out = 1;
-    f.filter = 8 * g.out_n <= f.block && f.block >= 256;
-    local(s, f, r.rows);
-    return;
-  }
-  // Full bitonic network over p words per row: LDS passes for partner
-  // distances below kSortBlock, global passes for the rest.
-  p.block = kSortBlock;
+  p.row_len = L.p;
   p.blocks_per_row = L.p / kSortBlock;
   p.k_first = 2, p.k_last = kSortBlock, p.j_first = 1;
-  p.global_dir = 1;
-  p.keep = kSortBlock;
   p.dst = buf;
-  p.dst_stride = L.p;
   local(s, p, r.rows);
   const int64_t pairs = r.rows * (L.p / 2);
   PJRTX_CHECK((pairs + 255) / 256 < (int64_t{1} << 31), Code::kUnimplemented, "sort: too large");
@@ -389,8 +954,7 @@ void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGat
       check_launch("bitonic_global");
     }
     LocalPass m = p;
-    m.keys = nullptr;
-    m.list = buf, m.list_len = L.p, m.list_stride = L.p;
+    m.list = buf;
     m.k_first = k, m.k_last = k, m.j_first = kSortBlock / 2;
     local(s, m, r.rows);
   }

@@ -253,6 +253,8 @@ void rewrite_program(Program* prog);
 // Folds JAX's negative-index normalization of gather indices into the
 // gathers (library.cc); true when a gather changed.
 bool fold_gather_index_wrap(Program* prog);
+// Sort operands that are the positions (sort.cc).
+bool fold_sort_iota(Program* prog);
 // transpose(dot_general(a, b)) as dot_general(b, a) (dot_general.cc).
 bool fold_dot_transpose(Program* prog);
 

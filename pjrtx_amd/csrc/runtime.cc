@@ -7,6 +7,7 @@
 #include <sys/stat.h>
 #include <unistd.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -37,6 +38,11 @@ thread_local Arena* t_arena = nullptr;
 }  // namespace
 
 Arena* thread_arena() { return t_arena; }
+int64_t scratch_left(const Device* dev) {
+  const Arena* a = t_arena;
+  if (!a || a->dev != dev) return int64_t(1) << 60;
+  return static_cast<int64_t>(a->cap - std::min(a->cap, (a->used + 255) & ~size_t(255)));
+}
 ArenaScope::ArenaScope(Arena* a) : prev_(t_arena) { t_arena = a; }
 ArenaScope::~ArenaScope() { t_arena = prev_; }
 

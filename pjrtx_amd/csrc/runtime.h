@@ -59,6 +59,9 @@ struct Arena {
   size_t peak = 0;
 };
 Arena* thread_arena();
+// Bytes this thread may still allocate on the device: what an installed arena
+// has left, or no bound.
+int64_t scratch_left(const Device* dev);
 class ArenaScope {
  public:
   explicit ArenaScope(Arena* a);

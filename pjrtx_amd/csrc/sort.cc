@@ -11,6 +11,9 @@
 // equal values by position (XLA's TopK).
 #include "sort_op.h"
 
+#include <algorithm>
+#include <map>
+
 #include "kernels/sort.h"
 #include "runtime.h"
 
@@ -59,10 +62,10 @@ SortSpec spec_of(const Program& prog, const Op& op) {
     sp.out_n = k;
     return sp;
   }
-  const size_t n_ops = op.operands.size();
+  const size_t n_ops = op.operands.size() + op.iota_results.size();
   PJRTX_CHECK(n_ops >= 1 && n_ops <= static_cast<size_t>(kSortMaxOperands) && op.results.size() == n_ops,
               Code::kUnimplemented, strformat("sort: %zu operands (1 to %d supported)", n_ops, kSortMaxOperands));
-  for (size_t i = 1; i < n_ops; ++i)
+  for (size_t i = 1; i < op.operands.size(); ++i)
     PJRTX_CHECK(prog.type(op.operands[i]).dims == x.dims, Code::kInvalidArgument, "sort: operand shapes differ");
   const int64_t dim = op.dim < 0 ? x.rank() - 1 : op.dim;
   PJRTX_CHECK(dim >= 0 && dim < x.rank(), Code::kInvalidArgument, "sort: dimension out of range");
@@ -108,6 +111,33 @@ SortSpec spec_of(const Program& prog, const Op& op) {
 
 }  // namespace
 
+// A sort operand that is an integer iota along the sorted dim (the positions
+// of an argsort) is not read: the sorted positions are its result.
+bool fold_sort_iota(Program* prog) {
+  std::map<int, const Op*> producer;
+  for (const Op& op : prog->ops)
+    for (int r : op.results) producer[r] = &op;
+  bool changed = false;
+  for (Op& op : prog->ops) {
+    if (op.kind != OpKind::kSort || op.operands.size() != op.results.size()) continue;
+    const int rank = prog->type(op.operands.at(0)).rank();
+    const int64_t dim = op.dim < 0 ? rank - 1 : op.dim;
+    std::vector<int> keep;
+    for (size_t i = 0; i < op.operands.size(); ++i) {
+      auto it = producer.find(op.operands[i]);
+      const TensorType& t = prog->type(op.operands[i]);
+      const bool iota = i > 0 && it != producer.end() && it->second->kind == OpKind::kIota && it->second->dim == dim &&
+                        t.dims == prog->type(op.operands[0]).dims && t.dtype != DType::kPred &&
+                        (dtype_is_signed_int(t.dtype) || dtype_is_unsigned_int(t.dtype));
+      if (iota) op.iota_results.push_back(static_cast<int64_t>(i));
+      else keep.push_back(op.operands[i]);
+    }
+    changed |= keep.size() != op.operands.size();
+    op.operands = keep;
+  }
+  return changed;
+}
+
 void check_sort_supported(const Program& prog, const Op& op) { (void)spec_of(prog, op); }
 
 void run_sort(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals) {
@@ -121,16 +151,19 @@ void run_sort(Device* dev, const Program& prog, const Op& op, std::vector<MemRef
     g.elem_bytes[0] = static_cast<int>(dtype_size(prog.type(op.operands[0]).dtype));
     g.index_dst = vals[op.results[1]]->ptr;
   } else {
-    g.count = static_cast<int>(op.operands.size());
+    g.count = static_cast<int>(op.results.size());
+    size_t operand = 0;
     for (int i = 0; i < g.count; ++i) {
-      g.src[i] = vals[op.operands[i]]->ptr;
+      const bool iota = std::find(op.iota_results.begin(), op.iota_results.end(), i) != op.iota_results.end();
+      g.src[i] = iota ? nullptr : vals[op.operands.at(operand++)]->ptr;
       g.dst[i] = vals[op.results[i]]->ptr;
-      g.elem_bytes[i] = static_cast<int>(dtype_size(prog.type(op.operands[i]).dtype));
+      g.elem_bytes[i] = static_cast<int>(dtype_size(prog.type(op.results[i]).dtype));
     }
   }
-  const size_t scratch_bytes = sort_scratch_bytes(sp.rows, sp.out_n);
+  const int64_t left = std::max<int64_t>(0, scratch_left(dev) - 4096);
+  const size_t scratch_bytes = sort_scratch_bytes(sp.rows, sp.out_n, left);
   MemRef scratch = scratch_bytes ? dev->allocate(scratch_bytes) : MemRef();
-  sort_rows(dev->stream(), sp.rows, vals[op.operands[0]]->ptr, g, scratch ? scratch->ptr : nullptr);
+  sort_rows(dev->stream(), sp.rows, vals[op.operands[0]]->ptr, g, scratch ? scratch->ptr : nullptr, left);
 }
 
 }  // namespace pjrtx
