@@ -332,3 +332,46 @@ def test_gather_index_wrap_needs_the_row_count(plugin):
     # normalization and stays an elementwise kernel
     p = plan(plugin, _wrapped_gather(1000, 64, 16, add_value=999))
     assert [st["kind"] for st in p["steps"]] == ["loop", "library"]
+
+
+def _dot_steps(plugin, make):
+    b = Builder()
+    return plan(plugin, b.build(make(b)))["steps"]
+
+
+def test_transposed_product_swaps_its_operands(plugin):
+    def make(perm, shape=(40, 24), other=(24, 56), read_twice=False):
+        def f(b):
+            batch = tuple(range(len(shape) - 2))
+            d = b.dot_general(b.param(shape, "bf16"), b.param(other, "bf16"), batch=(batch, batch),
+                              contract=((len(shape) - 1,), (len(shape) - 2,)))
+            return [b.transpose(d, perm)] + ([d] if read_twice else [])
+        return f
+    assert len(_dot_steps(plugin, make([1, 0]))) == 1
+    assert len(_dot_steps(plugin, make([0, 2, 1], (2, 40, 24), (2, 24, 56)))) == 1
+    assert len(_dot_steps(plugin, make([1, 0], read_twice=True))) == 2
+    assert len(_dot_steps(plugin, make([2, 1, 0], (2, 40, 24), (2, 24, 56)))) == 2  # moves the batch too
+    assert len(_dot_steps(plugin, make([1, 0], (4, 24)))) == 2                      # GEMV rows stay as they are
+
+
+def test_bias_row_merges_into_the_product(plugin):
+    def make(bias_shape, dims, dt="bf16"):
+        def f(b):
+            d = b.dot_general(b.param((40, 24), "bf16"), b.param((24, 40), "bf16"), contract=((1,), (0,)), out_dtype=dt)
+            return [b.add(d, b.broadcast_in_dim(b.param(bias_shape, dt), (40, 40), dims))]
+        return f
+    assert len(_dot_steps(plugin, make((40,), [1]))) == 1
+    assert len(_dot_steps(plugin, make((40,), [0]))) == 2        # a column
+    assert len(_dot_steps(plugin, make((1, 40), [0, 1]))) == 2
+    assert len(_dot_steps(plugin, make((40,), [1], "f32"))) == 2
+
+
+def test_sort_writes_positions_itself(plugin):
+    def make(iota_dim, first=False):
+        def f(b):
+            ops = [b.param((8, 64), "f32"), b.iota((8, 64), iota_dim)]
+            return b.sort(ops[::-1] if first else ops, 1)
+        return f
+    assert [s["kind"] for s in _dot_steps(plugin, make(1))] == ["library"]
+    assert len(_dot_steps(plugin, make(0))) == 2               # not the position
+    assert len(_dot_steps(plugin, make(1, first=True))) == 2   # the key itself
