@@ -13,9 +13,10 @@
 //    the whole walk. Workgroups take the heaviest (latest) query tiles first;
 //    when B*H is a multiple of 8, one head's query tiles run on one XCD so
 //    its K and V are served from that XCD's L2.
-//  * attn_pipe (head dim 128, the default for it): the same work split with
-//    K and V loaded straight into LDS, V^T fragments from transposing LDS
-//    reads and a leaner softmax (see its comment below).
+//  * attn_pipe (the default for both): the same work split, or a finer one
+//    for small launches, with K and V loaded straight into LDS, V^T fragments
+//    from transposing LDS reads and a leaner softmax (see its comment below).
+//    attn_tiles keeps heads whose K or V spans 2 GiB or more.
 //  * attn_rows (any element type, head dim <= 512): one workgroup per query
 //    row, its 4 waves splitting the keys in blocks of 64 (one key per lane
 //    for the scores, then lanes across the head dim for P.V), combined at the
@@ -339,10 +340,12 @@ __global__ void __launch_bounds__(256, 2) attn_tiles(AttnParams p, const uint16_
 }
 
 // ------------------------------------------------------ DMA tiles
-// attn_pipe (head dim 128): the tile kernel's work split (128 queries per
-// workgroup, 32 per wave, 64-key blocks, S^T = K.Q^T so a lane holds 16
-// scores of one query) with the memory and the VALU work laid out for
-// gfx950:
+// attn_pipe: the tile kernel's work split (128 queries per workgroup, 32 per
+// wave, 64-key blocks, S^T = K.Q^T so a lane holds 16 scores of one query; 64
+// or 32 queries in small launches) with the memory and the VALU work laid out
+// for gfx950. Bound by the MFMA and VALU issue of two or three waves a SIMD
+// that overlap in part ([8,32,2048] causal bf16, head dim 128: matrix cores
+// 40%, VALU issue 58% busy at 347 us; 332 us with the softmax below).
 //  * K and V blocks go from global memory straight into LDS (buffer loads
 //    with the LDS destination, 16 bytes a lane), two LDS stages each, one
 //    barrier per block; no register staging. The loads are lds_dma16: with
@@ -356,37 +359,78 @@ __global__ void __launch_bounds__(256, 2) attn_tiles(AttnParams p, const uint16_
 //    canonicalization), the max taken on the unrounded scores (rounding is
 //    monotone), one packed convert per two scores for the rounding, the row
 //    sums from the P.V MFMAs (a row of ones beside V^T), and the running max
-//    raised only when it grows by more than 2^8 in the exponential, so most
-//    blocks skip the output rescale.
-// LDS: K stage [64 keys][128] with 16-byte chunk c of row r at c ^ (r & 15)
-// (the 16 rows of a fragment read fall in distinct banks); V stage [64][128]
-// with chunk c of row r at c ^ 2 (r & 7) (the 8 rows a half-wave of
-// transposing reads touches fall in distinct banks). The buffer loads place
-// lane L's 16 bytes at slot L of the wave's 1 KB, so the swizzle is applied
-// on the global side: the lane filling slot (r, s) fetches chunk s ^ f(r).
-typedef __attribute__((address_space(3))) void* attn_lds_ptr;
+//    raised only when it grows by more than 2^8 in the exponential: one test
+//    a block, and the output is rescaled only where it holds (a rescale
+//    factor recomputed each block is 1 but for rounding, and half of the
+//    blocks rescaled for that). With the stage a constant of the unrolled
+//    block loop and the row max without LDS round trips: 347 -> 332 us.
+//  * Query tiles of a causal launch run latest first and one to a workgroup:
+//    pairing late with early ones, which leveled the workgroups, cost 8 us.
+//  * Head dim 64 in the same form: [8,32,2048,64] causal bf16 344 -> 182 us
+//    against attn_tiles.
+// LDS: K stage [64 keys][D] with 16-byte chunk c of row r at c ^ (r & 15), or
+// (r >> 1) & 7 at head dim 64 (the 16 rows of a fragment read fall in distinct
+// banks); V stage [64][D] with chunk c of row r at c ^ 2 (r & 7), or
+// 2 ((r >> 1) & 3) (the 8 rows a half-wave of transposing reads touches fall
+// in distinct banks). The buffer loads place lane L's 16 bytes at slot L of
+// the wave's 1 KB, so the swizzle is applied on the global side: the lane
+// filling slot (r, s) fetches chunk s ^ f(r).
 typedef short attn_v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) attn_v4i16 attn_lds_v4i16;
 
-constexpr int PK = 64;          // keys per block
-constexpr int PSTAGE = PK * 128;  // elements per K or V stage
+constexpr int PK = 64;  // keys per block
 
-__device__ __forceinline__ int pk_swz(int row, int ch) { return row * 128 + ((ch ^ (row & 15)) << 3); }
-__device__ __forceinline__ int pv_swz(int row, int ch) { return row * 128 + ((ch ^ ((row & 7) << 1)) << 3); }
+template <int D>
+__device__ __forceinline__ int pk_xor(int row) { return D == 128 ? row & 15 : (row >> 1) & 7; }
+template <int D>
+__device__ __forceinline__ int pv_xor(int row) { return (D == 128 ? row & 7 : (row >> 1) & 3) << 1; }
+template <int D>
+__device__ __forceinline__ int pk_swz(int row, int ch) { return row * D + ((ch ^ pk_xor<D>(row)) << 3); }
+template <int D>
+__device__ __forceinline__ int pv_swz(int row, int ch) { return row * D + ((ch ^ pv_xor<D>(row)) << 3); }
 constexpr int attn_vmcnt0() { return (7 << 4) | (15 << 8); }  // s_waitcnt vmcnt(0) alone
 
-template <bool kF16, bool kRound>
-__global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t* __restrict__ Q,
-                                                    const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
-                                                    uint16_t* __restrict__ O, int order, int pair, int prio) {
-  constexpr int D = 128, NDS = 4, NDT = 8;
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[2 * PSTAGE];
-  __shared__ __attribute__((aligned(16))) uint16_t Vs[2 * PSTAGE];
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
+}
+
+// The max over the 4 16-lane groups of a wave, on every lane: swapped halves
+// and rows (v_permlane32_swap, v_permlane16_swap) rather than LDS shuffles,
+// whose two round trips each block waited for.
+__device__ __forceinline__ float max_of_groups(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float y = __builtin_elementwise_maximum(__builtin_bit_cast(float, (uint32_t)h[0]), __builtin_bit_cast(float, (uint32_t)h[1]));
+  const uint32_t v = __builtin_bit_cast(uint32_t, y);
+  const auto w = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return __builtin_elementwise_maximum(__builtin_bit_cast(float, (uint32_t)w[0]), __builtin_bit_cast(float, (uint32_t)w[1]));
+}
+
+// A workgroup's 4 waves hold NQT tiles of 16 queries each; KW waves share the
+// queries and take every KW-th key block.
+template <int D, int NQT, int KW>
+struct PipeShape {
+  static constexpr int kQueries = 4 / KW * NQT * 16;  // per workgroup
+  static constexpr int kStage = KW * PK * D;          // elements per K or V stage
+  static constexpr int kLds = 4 * kStage * 2;         // bytes
+  // Workgroups per CU (and waves per SIMD): what the LDS and registers hold.
+  static constexpr int kFit = 160 * 1024 / kLds, kMost = NQT == 1 ? 4 : D == 64 ? 3 : 2;
+  static constexpr int kPerCu = kFit < kMost ? kFit : kMost;
+};
+constexpr int kPipeCus = 256;
+
+template <int D, int NQT, int KW, bool kF16, bool kRound>
+__global__ void __launch_bounds__(256, (PipeShape<D, NQT, KW>::kPerCu))
+    attn_pipe(AttnParams p, const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+              const uint16_t* __restrict__ V, uint16_t* __restrict__ O, int order, int prio) {
+  typedef PipeShape<D, NQT, KW> Shape;
+  constexpr int FQ = Shape::kQueries, PSTAGE = Shape::kStage;
+  constexpr int NDS = D / 32, NDT = D / 16;
+  extern __shared__ __attribute__((aligned(16))) uint16_t pipe_lds[];
+  uint16_t* const Ks = pipe_lds;
+  uint16_t* const Vs = pipe_lds + 2 * PSTAGE;
 
   const int nq = (p.Sq + FQ - 1) / FQ;
-  // pair: a workgroup takes query tiles nq-1-j and j (the heaviest with the
-  // lightest), so every workgroup has the same number of key blocks.
-  const int nslots = pair ? (nq + 1) / 2 : nq;
   const int BH = p.B * p.Hq;
   const int bid = blockIdx.x;
   int bh, slot;
@@ -400,43 +444,38 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
     if (order > 0) {
       const int hx = BH / 8;
       const int gsz = std::min(order, hx);
-      const int span = gsz * nslots;
+      const int span = gsz * nq;
       const int grp = n / span, w = n - grp * span;
       const int gfirst = grp * gsz, gcount = std::min(gsz, hx - gfirst);
       slot = w / gcount;
       bh = (gfirst + w % gcount) * 8 + x;
     } else {
-      bh = (n / nslots) * 8 + x;
-      slot = n % nslots;
+      bh = (n / nq) * 8 + x;
+      slot = n % nq;
     }
   } else {
     bh = bid % BH;
     slot = bid / BH;
   }
-  const int tile0 = nq - 1 - slot;
-  const int tile1 = pair && slot < tile0 ? slot : -1;
   const int b = bh / p.Hq, h = bh - b * p.Hq;
   const int hk = h / (p.Hq / p.Hkv);
   const uint16_t* Qp = Q + (int64_t)b * p.q_b + (int64_t)h * p.q_h;
   const uint16_t* Kp = K + (int64_t)b * p.k_b + (int64_t)hk * p.k_h;
   const uint16_t* Vp = V + (int64_t)b * p.v_b + (int64_t)hk * p.v_h;
   uint16_t* Op = O + (int64_t)b * p.o_b + (int64_t)h * p.o_h;
-  for (int ti = 0; ti < 2; ++ti) {
-  const int qtile = ti == 0 ? tile0 : tile1;
-  if (qtile < 0) break;
-  if (ti > 0) __syncthreads();  // the first tile's last LDS reads are done
-  const int q0 = qtile * FQ;
+  const int q0 = (nq - 1 - slot) * FQ;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, c16 = lane & 15;
   const u32x4 zero = {0u, 0u, 0u, 0u};
 
-  u32x4 qf[2][NDS];
-  int lim[2];
+  const int qw = wave / KW, kg = wave - qw * KW;  // the wave's queries, and its block of a step's KW
+  u32x4 qf[NQT][NDS];
+  int lim[NQT];
   const int64_t off = read_offset(p);
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const int q = q0 + wave * 32 + qt * 16 + c16;
+  for (int qt = 0; qt < NQT; ++qt) {
+    const int q = q0 + (qw * NQT + qt) * 16 + c16;
 #pragma unroll
     for (int ds = 0; ds < NDS; ++ds)
       qf[qt][ds] = q < p.Sq ? *reinterpret_cast<const u32x4*>(Qp + (int64_t)q * p.q_s + ds * 32 + g * 8) : zero;
@@ -451,54 +490,63 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
   const uint32_t v_bytes = (uint32_t)(((int64_t)(p.Skv - 1) * p.v_s + D) * 2);
   const lds_rsrc krs = make_lds_rsrc(Kp, p.Skv > 0 ? k_bytes : 0);
   const lds_rsrc vrs = make_lds_rsrc(Vp, p.Skv > 0 ? v_bytes : 0);
-  // Wave w fills rows 16w .. 16w+15 of a stage, four rows per load; the
-  // lane part of each load's offset is fixed, the block part is scalar.
+  // Each wave fills its share of a stage's rows, 1 KB per load; the lane part
+  // of each load's offset is fixed, the block part is scalar.
+  constexpr int kWaveRows = KW * PK / 4, kLoadRows = 512 / D, NL = kWaveRows / kLoadRows;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int lrow = lane >> 4, lslot = lane & 15;
-  uint32_t koff[4], voff[4];
+  const int lrow = lane / (D / 8), lslot = lane % (D / 8);
+  uint32_t koff[NL], voff[NL];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = wave_u * 16 + i * 4 + lrow;
-    koff[i] = (uint32_t)(((int64_t)row * p.k_s + ((lslot ^ (row & 15)) * 8)) * 2);
-    voff[i] = (uint32_t)(((int64_t)row * p.v_s + ((lslot ^ ((row & 7) << 1)) * 8)) * 2);
+  for (int i = 0; i < NL; ++i) {
+    const int row = wave_u * kWaveRows + i * kLoadRows + lrow;
+    koff[i] = (uint32_t)(((int64_t)row * p.k_s + ((lslot ^ pk_xor<D>(row)) * 8)) * 2);
+    voff[i] = (uint32_t)(((int64_t)row * p.v_s + ((lslot ^ pv_xor<D>(row)) * 8)) * 2);
   }
-  const uint32_t klds = lds_offset(Ks + wave_u * 16 * 128), vlds = lds_offset(Vs + wave_u * 16 * 128);
-  auto dma_k = [&](int kb, int stage) {
-    const uint32_t sblk = (uint32_t)((int64_t)kb * PK * p.k_s * 2);
+  const uint32_t klds = lds_offset(Ks + wave_u * kWaveRows * D), vlds = lds_offset(Vs + wave_u * kWaveRows * D);
+  auto dma_k = [&](int step, int stage) {
+    const uint32_t sblk = (uint32_t)((int64_t)step * (KW * PK) * p.k_s * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      lds_dma16(krs, koff[i], sblk, klds + (uint32_t)(stage * PSTAGE + i * 4 * 128) * 2);
+    for (int i = 0; i < NL; ++i)
+      lds_dma16(krs, koff[i], sblk, klds + (uint32_t)(stage * PSTAGE + i * kLoadRows * D) * 2);
   };
-  auto dma_v = [&](int kb, int stage) {
-    const uint32_t sblk = (uint32_t)((int64_t)kb * PK * p.v_s * 2);
+  auto dma_v = [&](int step, int stage) {
+    const uint32_t sblk = (uint32_t)((int64_t)step * (KW * PK) * p.v_s * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      lds_dma16(vrs, voff[i], sblk, vlds + (uint32_t)(stage * PSTAGE + i * 4 * 128) * 2);
+    for (int i = 0; i < NL; ++i)
+      lds_dma16(vrs, voff[i], sblk, vlds + (uint32_t)(stage * PSTAGE + i * kLoadRows * D) * 2);
   };
 
   const float c2 = p.scale * 1.44269504088896340736f;
-  float m[2] = {-INFINITY, -INFINITY};
-  f32x4 oacc[NDT][2];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) oacc[dt][0] = oacc[dt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float mc[NQT], limit[NQT];
+  f32x4 oacc[NDT][NQT];
   // Row sums: O^T rows of an all-ones V^T tile (every element of a lane's
   // accumulator holds its query's sum).
-  f32x4 lacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  f32x4 lacc[NQT];
+#pragma unroll
+  for (int qt = 0; qt < NQT; ++qt) {
+    mc[qt] = 0.f;
+    limit[qt] = -INFINITY;
+    lacc[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) oacc[dt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   const uint32_t one2 = kF16 ? 0x3c003c00u : 0x3f803f80u;
   const u32x4 ones = {one2, one2, one2, one2};
 
-  // S^T[key][query] of block kb for the wave's 32 queries, from K stage `stage`.
-  auto scores = [&](int stage, f32x4 (&sacc)[4][2]) {
-    const uint16_t* ks = Ks + stage * PSTAGE;
+  // S^T[key][query] of the wave's block and queries, from K stage `stage`.
+  auto scores = [&](int stage, f32x4 (&sacc)[4][NQT]) {
+    const uint16_t* ks = Ks + stage * PSTAGE + kg * (PK * D);
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) sacc[kt][0] = sacc[kt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int qt = 0; qt < NQT; ++qt) sacc[kt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ds = 0; ds < NDS; ++ds) {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(&ks[pk_swz(kt * 16 + c16, ds * 4 + g)]);
-        sacc[kt][0] = mfma16<kF16>(a, qf[0][ds], sacc[kt][0]);
-        sacc[kt][1] = mfma16<kF16>(a, qf[1][ds], sacc[kt][1]);
+        const u32x4 a = *reinterpret_cast<const u32x4*>(&ks[pk_swz<D>(kt * 16 + c16, ds * 4 + g)]);
+#pragma unroll
+        for (int qt = 0; qt < NQT; ++qt) sacc[kt][qt] = mfma16<kF16>(a, qf[qt][ds], sacc[kt][qt]);
       }
     }
   };
@@ -507,10 +555,10 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
   // Keys past a query's limit: only blocks that reach past the first
   // query's limit have any (a branch of its own, so unmasked blocks pay
   // nothing per score).
-  auto mask = [&](int kb, f32x4 (&sacc)[4][2]) {
+  auto mask = [&](int kb, f32x4 (&sacc)[4][NQT]) {
     if (kb * PK + PK <= free_end) return;
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt)
+    for (int qt = 0; qt < NQT; ++qt)
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
@@ -521,36 +569,46 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
   // 2^8 in the exponential (then the output and sum are rescaled), so the
   // exponentials stay below 2^8 and most blocks skip the rescale. The row
   // sums come from the P.V products (a row of ones beside V), so the softmax
-  // itself is max, round, exponential and pack.
-  auto softmax = [&](int kb, f32x4 (&sacc)[4][2], u32x4 (&pf)[2][2]) {
-    (void)kb;
-    float alpha[2];
+  // itself is max, round, exponential and pack. mc is the max times c2, limit
+  // what a block's max must pass.
+  auto softmax = [&](f32x4 (&sacc)[4][NQT], u32x4 (&pf)[NQT][2]) {
+    float mx[NQT];
+    bool raise = false;
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
+    for (int qt = 0; qt < NQT; ++qt) {
+      float t[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f32x4 x = sacc[2 * h][qt], y = sacc[2 * h + 1][qt];
+        t[h] = max3(max3(max3(x[0], x[1], x[2]), x[3], y[0]), y[1], y[2]);
+        t[h] = h ? max3(t[0], t[h], y[3]) : __builtin_elementwise_maximum(t[h], y[3]);
+      }
+      mx[qt] = max_of_groups(t[1]);
+      raise |= mx[qt] * c2 > limit[qt];
+    }
+    if (__any(raise)) {
+#pragma unroll
+      for (int qt = 0; qt < NQT; ++qt) {
+        float r = mx[qt];
+        if constexpr (kRound) r = round16<kF16>(r);
+        const bool up = mx[qt] * c2 > limit[qt];
+        const float mnew = up ? r * c2 : mc[qt];
+        const float alpha = limit[qt] == -INFINITY ? (up ? 0.f : 1.f) : __builtin_amdgcn_exp2f(mc[qt] - mnew);
+        mc[qt] = mnew;
+        if (up) limit[qt] = mnew + 8.f;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) oacc[dt][qt] *= alpha;
+        lacc[qt][0] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int qt = 0; qt < NQT; ++qt) {
       float s[4][4];
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[kt][r] = sacc[kt][qt][r];
-      float mx = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-        mx = __builtin_elementwise_maximum(
-            mx, __builtin_elementwise_maximum(__builtin_elementwise_maximum(s[kt][0], s[kt][1]),
-                                              __builtin_elementwise_maximum(s[kt][2], s[kt][3])));
-      mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 16));
-      mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32));
-      if constexpr (kRound) mx = round16<kF16>(mx);
-      const bool raise = mx * c2 > m[qt] * c2 + 8.f;
-      const float mnew = raise ? mx : m[qt];
-      const float mc = (mnew == -INFINITY ? 0.f : mnew) * c2;
-      alpha[qt] = __builtin_amdgcn_exp2f(m[qt] * c2 - mc);
-      m[qt] = mnew;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
         for (int r = 0; r < 4; r += 2) {
-          float x0 = s[kt][r], x1 = s[kt][r + 1];
+          float x0 = sacc[kt][qt][r], x1 = sacc[kt][qt][r + 1];
           if constexpr (kRound) {
             const uint32_t pk = pack2<kF16>(x0, x1);
             if constexpr (kF16) {
@@ -561,8 +619,8 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
               x1 = __builtin_bit_cast(float, pk & 0xffff0000u);
             }
           }
-          s[kt][r] = __builtin_amdgcn_exp2f(fmaf(x0, c2, -mc));
-          s[kt][r + 1] = __builtin_amdgcn_exp2f(fmaf(x1, c2, -mc));
+          s[kt][r] = __builtin_amdgcn_exp2f(fmaf(x0, c2, -mc[qt]));
+          s[kt][r + 1] = __builtin_amdgcn_exp2f(fmaf(x1, c2, -mc[qt]));
         }
 #pragma unroll
       for (int st = 0; st < 2; ++st)
@@ -570,18 +628,10 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
                            pack2<kF16>(s[2 * st + 1][0], s[2 * st + 1][1]),
                            pack2<kF16>(s[2 * st + 1][2], s[2 * st + 1][3])};
     }
-    if (!__all(alpha[0] == 1.f && alpha[1] == 1.f)) {
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) oacc[dt][qt] *= alpha[qt];
-        lacc[qt][0] *= alpha[qt];
-      }
-    }
   };
   // O^T[d][query] += V^T[d][key] . P^T[key][query] from V stage `stage`.
-  auto pv = [&](int stage, const u32x4 (&pf)[2][2]) {
-    const uint16_t* vs = Vs + stage * PSTAGE;
+  auto pv = [&](int stage, const u32x4 (&pf)[NQT][2]) {
+    const uint16_t* vs = Vs + stage * PSTAGE + kg * (PK * D);
     const int i = lane & 15;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -590,66 +640,112 @@ __global__ void __launch_bounds__(256, 2) attn_pipe(AttnParams p, const uint16_t
         const int r0 = st * 32 + 4 * g + (i >> 2), r1 = r0 + 16;
         const int ch = 2 * dt + ((i & 3) >> 1), sub = 4 * (i & 1);
         const attn_v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (attn_lds_v4i16*)((__attribute__((address_space(3))) uint16_t*)(vs + pv_swz(r0, ch) + sub)));
+            (attn_lds_v4i16*)((__attribute__((address_space(3))) uint16_t*)(vs + pv_swz<D>(r0, ch) + sub)));
         const attn_v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (attn_lds_v4i16*)((__attribute__((address_space(3))) uint16_t*)(vs + pv_swz(r1, ch) + sub)));
+            (attn_lds_v4i16*)((__attribute__((address_space(3))) uint16_t*)(vs + pv_swz<D>(r1, ch) + sub)));
         const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
         const u32x4 a = u32x4{l2[0], l2[1], h2[0], h2[1]};
-        oacc[dt][0] = mfma16<kF16>(a, pf[0][st], oacc[dt][0]);
-        oacc[dt][1] = mfma16<kF16>(a, pf[1][st], oacc[dt][1]);
+#pragma unroll
+        for (int qt = 0; qt < NQT; ++qt) oacc[dt][qt] = mfma16<kF16>(a, pf[qt][st], oacc[dt][qt]);
       }
-      lacc[0] = mfma16<kF16>(ones, pf[0][st], lacc[0]);
-      lacc[1] = mfma16<kF16>(ones, pf[1][st], lacc[1]);
+#pragma unroll
+      for (int qt = 0; qt < NQT; ++qt) lacc[qt] = mfma16<kF16>(ones, pf[qt][st], lacc[qt]);
     }
   };
 
-  f32x4 sA[4][2];
-  u32x4 pf[2][2];
-  // Block kb from stage kb & 1 while block kb + 1 loads into the other
-  // (read in the step before); two workgroups per CU overlap one's MFMAs
-  // with the other's softmax. A wave whose 32 queries allow none of a
-  // block's keys (the diagonal blocks past its last query) only takes part
-  // in the loads and barriers.
-  const int wave_last = key_limit(p, off, std::min(q0 + wave * 32 + 31, p.Sq - 1));
-  if (nblocks > 0) {
+  f32x4 sA[4][NQT];
+  u32x4 pf[NQT][2];
+  // A step's KW blocks from stage step & 1 while the next step's load into the
+  // other (read in the step before); the waves of a SIMD overlap one's MFMAs
+  // with another's softmax. A wave whose queries allow none of its block's
+  // keys (the diagonal blocks past its last query) only takes part in the
+  // loads and barriers.
+  const int wave_last = key_limit(p, off, std::min(q0 + (qw + 1) * (NQT * 16) - 1, p.Sq - 1));
+  const int steps = (nblocks + KW - 1) / KW;
+  if (steps > 0) {
     dma_k(0, 0);
     dma_v(0, 0);
   }
-  for (int kb = 0; kb < nblocks; ++kb) {
+  auto block = [&](int step, auto parity) {
+    constexpr int st = decltype(parity)::value;  // a constant, so that LDS addresses are immediates
     __builtin_amdgcn_s_waitcnt(attn_vmcnt0());
     __syncthreads();
-    if (kb + 1 < nblocks) {
-      dma_k(kb + 1, (kb + 1) & 1);
-      dma_v(kb + 1, (kb + 1) & 1);
+    if (step + 1 < steps) {
+      dma_k(step + 1, st ^ 1);
+      dma_v(step + 1, st ^ 1);
     }
-    if (kb * PK > wave_last) continue;
+    const int kb = step * KW + kg;
+    if (kb * PK > wave_last) return;
     // With `prio`, the matrix-core phases run at raised wave priority: on a
     // SIMD whose other wave is in its softmax, the MFMAs issue first
     // (environment: PJRTX_ATTN_PRIO=0 disables; 360-365 vs 368-370 us on
     // [8,32,2048,128] causal bf16).
     if (prio) __builtin_amdgcn_s_setprio(1);
-    scores(kb & 1, sA);
+    scores(st, sA);
     if (prio) __builtin_amdgcn_s_setprio(0);
     mask(kb, sA);
-    softmax(kb, sA, pf);
+    softmax(sA, pf);
     if (prio) __builtin_amdgcn_s_setprio(1);
-    pv(kb & 1, pf);
+    pv(st, pf);
     if (prio) __builtin_amdgcn_s_setprio(0);
+  };
+  for (int step = 0; step < steps; step += 2) {
+    block(step, std::integral_constant<int, 0>());
+    if (step + 1 < steps) block(step + 1, std::integral_constant<int, 1>());
   }
 
+  if constexpr (KW > 1) {
+    // The key ways' (max, sum, output) meet in LDS; way 0 merges them. A way
+    // with no allowed key has sum 0 and adds nothing.
+    constexpr int kWay = (NDT + 1) * NQT * 256;  // floats a wave leaves
+    float* const xs = reinterpret_cast<float*>(pipe_lds);
+    __syncthreads();
+    if (kg > 0) {
+      float* x = xs + (qw * (KW - 1) + kg - 1) * kWay + lane * 4;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const int q = q0 + wave * 32 + qt * 16 + c16;
-    if (q >= p.Sq) continue;
-    uint16_t* orow = Op + (int64_t)q * p.o_s;
+      for (int qt = 0; qt < NQT; ++qt) {
+        *reinterpret_cast<f32x4*>(x + qt * 256) = f32x4{mc[qt], lacc[qt][0], 0.f, 0.f};
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const f32x4 o = oacc[dt][qt];
-      const float lq = lacc[qt][0];
-      *reinterpret_cast<u32x2*>(orow + dt * 16 + g * 4) =
-          u32x2{pack2<kF16>(o[0] / lq, o[1] / lq), pack2<kF16>(o[2] / lq, o[3] / lq)};
+        for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f32x4*>(x + ((dt + 1) * NQT + qt) * 256) = oacc[dt][qt];
+      }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int qt = 0; qt < NQT; ++qt) {
+      for (int w = 0; w < KW - 1; ++w) {
+        const float* x = xs + (qw * (KW - 1) + w) * kWay + lane * 4;
+        const f32x4 ml = *reinterpret_cast<const f32x4*>(x + qt * 256);
+        if (ml[1] == 0.f) continue;
+        const bool none = lacc[qt][0] == 0.f;
+        const float a0 = none ? 0.f : __builtin_amdgcn_exp2f(std::min(mc[qt] - ml[0], 0.f));
+        const float a1 = none ? 1.f : __builtin_amdgcn_exp2f(std::min(ml[0] - mc[qt], 0.f));
+        mc[qt] = none ? ml[0] : std::max(mc[qt], ml[0]);
+        lacc[qt][0] = lacc[qt][0] * a0 + ml[1] * a1;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+          oacc[dt][qt] = oacc[dt][qt] * a0 + *reinterpret_cast<const f32x4*>(x + ((dt + 1) * NQT + qt) * 256) * a1;
+      }
     }
   }
+#pragma unroll
+  for (int qt = 0; qt < NQT; ++qt) {
+    const int q = q0 + (qw * NQT + qt) * 16 + c16;
+    if (q >= p.Sq) continue;
+    uint16_t* orow = Op + (int64_t)q * p.o_s;
+    // o / l by the rounded reciprocal and one correction of the quotient
+    // (Markstein), with the quotient's special cases put right.
+    const float lq = lacc[qt][0], r = 1.f / lq;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+      f32x4 o = oacc[dt][qt];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float y = o[e] * r;
+        o[e] = __builtin_amdgcn_div_fixupf(fmaf(fmaf(-y, lq, o[e]), r, y), lq, o[e]);
+      }
+      *reinterpret_cast<u32x2*>(orow + dt * 16 + g * 4) = u32x2{pack2<kF16>(o[0], o[1]), pack2<kF16>(o[2], o[3])};
+    }
   }
 }
 
@@ -1104,6 +1200,28 @@ void launch_decode(hipStream_t s, const AttnParams& p, const T* q, const T* k, c
                        nsplit, keys_per_split, o);
 }
 
+// 128 queries a workgroup, unless 64 or 32 of them leave no workgroup waiting
+// for a CU: then the launch takes as long as its longest workgroup, and that
+// is shorter with fewer queries (and two key ways). us at 128 / 64 / 32
+// queries, causal bf16, head dim 128: [1,16,512] 15.3 / 13.0 / 10.6, [1,32,512]
+// 16.0 / 13.6 / 15.3, [1,32,1024] 27.8 / 24.9 / 39.3, [4,32,1024] 52 / 64 /
+// 146; head dim 64: [1,16,1024] 18.8 / 14.1 / 10.8, [2,32,1024] 21.4 / 17.9 /
+// 27.2, [2,32,2048] 47 / 54 / 78.
+template <int D, bool kF16, bool kRound>
+void launch_pipe(hipStream_t s, const AttnParams& p, const uint16_t* q, const uint16_t* k, const uint16_t* v,
+                 uint16_t* o, int order, int prio) {
+  const auto workgroups = [&](int queries) {
+    return static_cast<int64_t>(p.B) * p.Hq * ((p.Sq + queries - 1) / queries);
+  };
+#define PJRTX_PIPE_AS(NQT, KW)                                                                                   \
+  hipLaunchKernelGGL((attn_pipe<D, NQT, KW, kF16, kRound>), dim3(static_cast<uint32_t>(workgroups(PipeShape<D, NQT, KW>::kQueries))), \
+                     dim3(256), (PipeShape<D, NQT, KW>::kLds), s, p, q, k, v, o, order, prio)
+  if (workgroups(PipeShape<D, 1, 2>::kQueries) <= kPipeCus * PipeShape<D, 1, 2>::kPerCu) PJRTX_PIPE_AS(1, 2);
+  else if (workgroups(PipeShape<D, 1, 1>::kQueries) <= kPipeCus * PipeShape<D, 1, 1>::kPerCu) PJRTX_PIPE_AS(1, 1);
+  else PJRTX_PIPE_AS(2, 1);
+#undef PJRTX_PIPE_AS
+}
+
 template <typename T>
 void launch_rows(hipStream_t s, const AttnParams& p, const void* Q, const void* K, const void* V, void* out) {
   const dim3 grid(static_cast<uint32_t>(static_cast<int64_t>(p.B) * p.Hq * p.Sq)), block(256);
@@ -1204,16 +1322,15 @@ void launch_attention(hipStream_t s, const AttnParams& p, DType t, const void* Q
     const dim3 g(static_cast<uint32_t>(grid)), block(256);
 #define PJRTX_ATTN(F16, DIM, RND) hipLaunchKernelGGL((attn_tiles<F16, DIM, RND>), g, block, 0, s, p, q, k, v, o)
     const int order = static_cast<int>(env_int("PJRTX_ATTN_ORDER", 8));
-    const int pair = p.causal && env_int("PJRTX_ATTN_PAIR", 1) != 0 ? 1 : 0;
-    const dim3 gp(static_cast<uint32_t>(static_cast<int64_t>(p.B) * p.Hq *
-                                        (pair ? ((p.Sq + FQ - 1) / FQ + 1) / 2 : (p.Sq + FQ - 1) / FQ)));
     const int prio = static_cast<int>(env_int("PJRTX_ATTN_PRIO", 1));
-#define PJRTX_PIPE(F16, RND) hipLaunchKernelGGL((attn_pipe<F16, RND>), gp, block, 0, s, p, q, k, v, o, order, pair, prio)
+#define PJRTX_PIPE(F16, RND)                                                 \
+  (p.D == 128 ? launch_pipe<128, F16, RND>(s, p, q, k, v, o, order, prio)    \
+              : launch_pipe<64, F16, RND>(s, p, q, k, v, o, order, prio))
     const bool rnd = p.round_scores != 0;
     // The DMA kernel addresses K and V through 32-bit buffer offsets;
     // PJRTX_ATTN_PIPE=0 keeps the register-staged tile kernel.
-    const bool dma = p.D == 128 && env_int("PJRTX_ATTN_PIPE", 1) != 0 &&
-                     ((int64_t)std::max(p.Skv, 1) + PK) * std::max(p.k_s, p.v_s) * 2 < (int64_t(1) << 31);
+    const bool dma = env_int("PJRTX_ATTN_PIPE", 1) != 0 &&
+                     ((int64_t)std::max(p.Skv, 1) + 2 * PK) * std::max(p.k_s, p.v_s) * 2 < (int64_t(1) << 31);
     if (dma && f16 && rnd) PJRTX_PIPE(true, true);
     else if (dma && f16) PJRTX_PIPE(true, false);
     else if (dma && rnd) PJRTX_PIPE(false, true);

@@ -1,0 +1,69 @@
+"""attn_pipe's workgroup shapes (32, 64 and 128 queries, one and two key ways)
+at both head dims: ragged lengths, grouped heads, cached prefixes, queries
+with no allowed key and inputs that are not finite, against the float64
+oracle. The bar is test_gpu_attention's: probabilities are rounded to the
+input type before the division by their sum."""
+import numpy as np
+import pytest
+
+from oracle import attention as A
+from tests.test_gpu_attention import assert_close16, from_bits, sdpa_exe, to_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(client, dt, d, sizes, spoil=None):
+    b, sq, hq, skv, hkv, tok = sizes
+    rng = np.random.default_rng(sq * 7 + skv + d)
+    qs, kvs = (b, sq, hq, d), (b, skv, hkv, d)
+    q, k, v = (to_bits(rng.standard_normal(s), dt) for s in (qs, kvs, kvs))
+    if spoil:
+        spoil(q, k, v)
+    (out,) = sdpa_exe(client, dt, qs, kvs)(q, k, v, np.array(tok, np.int32), dtypes=[dt, dt, dt, None])
+    with np.errstate(invalid="ignore"):
+        want = A.sdpa_f64(from_bits(q, dt), from_bits(k, dt), from_bits(v, dt), np.int32(tok))
+    return from_bits(out, dt), want, out, v
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sizes", [
+    (1, 17, 1, 17, 1, 0),        # 32 queries, two key ways
+    (1, 200, 8, 333, 2, 100),
+    (2, 64, 3, 700, 3, 636),
+    (1, 32, 4, 64, 4, 32),       # the second way's only block is masked for most queries
+    (4, 300, 16, 300, 4, 0),     # 64 queries
+    (4, 330, 15, 470, 5, 139),   # batch * heads not a multiple of 8
+    (8, 140, 48, 140, 6, 0),     # 128 queries
+    (7, 130, 53, 195, 53, 64),
+])
+def test_workgroup_shapes(client, dt, d, sizes):
+    got, want, out, v = _run(client, dt, d, sizes)
+    assert_close16(got, want)
+    b, sq, hq, skv, hkv, tok = sizes
+    if tok == 0:  # query 0 sees key 0 alone: its value row exactly
+        np.testing.assert_array_equal(np.asarray(out)[:, 0], np.repeat(np.asarray(v)[:, 0], hq // hkv, axis=1))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sizes", [(1, 40, 2, 150, 1, -3), (4, 300, 16, 300, 4, -1), (8, 140, 48, 140, 48, -2)])
+def test_queries_with_no_allowed_key(client, d, sizes):
+    got, want, _, _ = _run(client, "bf16", d, sizes)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    assert np.isnan(want).any()
+    assert_close16(np.nan_to_num(got), np.nan_to_num(want))
+
+
+@pytest.mark.parametrize("sizes", [(1, 96, 4, 200, 4, 104), (4, 300, 16, 300, 16, 0), (8, 140, 48, 140, 48, 0)])
+def test_values_that_are_not_finite(client, sizes):
+    """An infinite value passes through (a quotient's special case), a NaN key
+    poisons the queries that may see it and no other."""
+    def spoil(q, k, v):
+        v[0, 0, 0, 5] = 0x7f80
+        k[0, 70, 1, 3] = 0x7fc0
+    got, want, _, _ = _run(client, "bf16", 128, sizes, spoil)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.isposinf(want).any() and np.isnan(want).any()
+    keep = np.isfinite(want)
+    assert_close16(np.where(keep, got, 0), np.where(keep, want, 0))
