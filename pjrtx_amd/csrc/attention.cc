@@ -415,6 +415,36 @@ void remove_dead_ops(Program* prog) {
 
 }  // namespace
 
+// transpose(attention, [0, 2, 1, 3]), the attention's only reader: the
+// attention writes [B, S, H, D] itself (its rows are D elements either way).
+// 512 queries of 16 heads, head dim 128: a 7 us copy and a launch less a
+// layer. Few queries keep the transpose, which moves nothing at one query and
+// whose result the decode GEMV's split merge looks for.
+static bool fold_attention_transpose(Program* prog) {
+  std::map<int, size_t> producer;
+  std::map<int, int> uses;
+  for (size_t i = 0; i < prog->ops.size(); ++i) {
+    for (int r : prog->ops[i].results) producer[r] = i;
+    for (int v : prog->ops[i].operands) uses[v]++;
+  }
+  for (int r : prog->results) uses[r]++;
+  bool changed = false;
+  for (Op& t : prog->ops) {
+    if (t.kind != OpKind::kTranspose || t.dims != Dims{0, 2, 1, 3}) continue;
+    auto it = producer.find(t.operands[0]);
+    if (it == producer.end() || uses[t.operands[0]] != 1) continue;
+    const Op& a = prog->ops[it->second];
+    if (a.kind != OpKind::kAttention || a.attn.layout != 0 || a.attn.out_bshd || prog->type(a.results[0]).dims[2] < 16)
+      continue;
+    Op r = a;
+    r.results = t.results;
+    r.attn.out_bshd = true;
+    t = std::move(r);
+    changed = true;
+  }
+  return changed;
+}
+
 void rewrite_program(Program* prog) {
   bool changed = false;
   for (Op& op : prog->ops) {
@@ -432,6 +462,7 @@ void rewrite_program(Program* prog) {
       if (m.try_rewrite(static_cast<int>(i))) changed = true;
     }
   }
+  changed |= fold_attention_transpose(prog);
   changed |= fold_dot_transpose(prog);
   changed |= fold_sort_iota(prog);
   if (changed) remove_dead_ops(prog);
@@ -477,7 +508,9 @@ AttnParams attention_params(const Program& prog, const Op& op) {
   strides_of(a, q, &p.q_b, &p.q_h, &p.q_s);
   strides_of(a, k, &p.k_b, &p.k_h, &p.k_s);
   strides_of(a, prog.type(op.operands[2]).dims, &p.v_b, &p.v_h, &p.v_s);
-  strides_of(a, prog.type(op.results[0]).dims, &p.o_b, &p.o_h, &p.o_s);
+  AttentionAttrs out = a;
+  if (a.out_bshd) out.layout = 1;
+  strides_of(out, prog.type(op.results[0]).dims, &p.o_b, &p.o_h, &p.o_s);
   p.scale = static_cast<float>(a.scale);
   p.causal = a.causal ? 1 : 0;
   p.q_coef = a.q_coef;

@@ -76,6 +76,7 @@ struct AttentionAttrs {
   // Operand layouts: 0 = [B, H, S, D] (the unfused dot_general form),
   // 1 = [B, S, H, D], 2 = [S, H, D] (the custom call's rank 4 / rank 3).
   int layout = 0;
+  bool out_bshd = false;  // layout 0: the result is written as [B, S, H, D]
   double scale = 1.0;
   bool causal = false;
   int q_coef = 1;

@@ -7,7 +7,9 @@ import numpy as np
 import pytest
 
 from oracle import attention as A
-from tests.test_gpu_attention import assert_close16, from_bits, sdpa_exe, to_bits
+from pjrtx_amd import programs
+from test_planner import attention_then_transpose
+from test_gpu_attention import assert_close16, from_bits, sdpa_exe, to_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +69,14 @@ def test_values_that_are_not_finite(client, sizes):
     assert np.isposinf(want).any() and np.isnan(want).any()
     keep = np.isfinite(want)
     assert_close16(np.where(keep, got, 0), np.where(keep, want, 0))
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shape", [(1, 16, 100, 128), (3, 5, 33, 64), (2, 3, 17, 40), (2, 130, 160, 128)])
+def test_result_written_transposed(client, shape, dt):
+    rng = np.random.default_rng(shape[2])
+    args = [rng.standard_normal(shape).astype(np.float32) for _ in range(3)]
+    args = args if dt == "f32" else [to_bits(a, dt) for a in args]
+    (plain,) = client.compile(programs.c3_attention(*shape, True, dtype=dt))(*args, dtypes=[dt] * 3)
+    (got,) = client.compile(attention_then_transpose(shape, [0, 2, 1, 3], dt))(*args, dtypes=[dt] * 3)
+    np.testing.assert_array_equal(np.asarray(got).view(np.uint8), np.ascontiguousarray(np.asarray(plain).transpose(0, 2, 1, 3)).view(np.uint8))

@@ -375,3 +375,24 @@ def test_sort_writes_positions_itself(plugin):
     assert [s["kind"] for s in _dot_steps(plugin, make(1))] == ["library"]
     assert len(_dot_steps(plugin, make(0))) == 2               # not the position
     assert len(_dot_steps(plugin, make(1, first=True))) == 2   # the key itself
+
+
+def attention_then_transpose(shape, perm, dt="bf16", twice=False):
+    """c3_attention whose result is transposed (and also returned, `twice`)."""
+    mlir = lambda d: "tensor<" + "x".join(map(str, d)) + f"x{dt}>"  # noqa: E731
+    src, dst = mlir(shape), mlir([shape[p] for p in perm])
+    text = programs.c3_attention(*shape, True, dtype=dt)
+    head = next(ln for ln in text.splitlines() if "func.func" in ln)
+    ret = next(ln for ln in text.splitlines() if ln.strip().split(" ")[0] in ("return", "func.return", "stablehlo.return"))
+    name = ret.split()[1]
+    both = (f"%tr, {name} : {dst}, {src}", f"({dst}, {src})") if twice else (f"%tr : {dst}", dst)
+    text = text.replace(ret, f"    %tr = stablehlo.transpose {name}, dims = {list(perm)} : ({src}) -> {dst}\n    return {both[0]}")
+    return text.replace(head, head[:head.index("->")] + f"-> {both[1]} {{")
+
+
+def test_attention_writes_its_transposed_result(plugin):
+    kinds = lambda *a, **k: [s.get("library", s["kind"]) for s in plan(plugin, attention_then_transpose(*a, **k))["steps"]]  # noqa: E731
+    assert kinds((2, 4, 128, 64), [0, 2, 1, 3]) == ["attention"]
+    assert kinds((2, 4, 128, 64), [0, 2, 1, 3], twice=True) == ["attention", "loop"]
+    assert kinds((2, 4, 128, 64), [0, 1, 3, 2]) == ["attention", "loop"]
+    assert kinds((2, 4, 8, 64), [0, 2, 1, 3]) == ["attention", "loop"]  # few queries
