@@ -1,5 +1,5 @@
 // MFMA GEMM for bf16 / f16 with f32 accumulation, either layout of either
-// operand, in block tiles from 32 x 128 to 256 x 256.
+// operand, in block tiles from 32 x 64 to 256 x 256.
 //
 // gemm_tile: C[b] = A[b] * B[b], A K-contiguous ([M][K]) or M-contiguous
 // ([K][M]), B K-contiguous ([N][K]) or N-contiguous ([K][N]).
