@@ -26,7 +26,9 @@
 namespace pjrtx {
 namespace {
 
-constexpr int kItems = 32;              // elements per lane per sort tile
+// Elements per lane per sort tile. 16 (twice the waves, twice the strided
+// histogram columns) took 9.2 + 19.3 us a pass against 6.7 + 19.6.
+constexpr int kItems = 32;
 constexpr int kTile = 64 * kItems;      // elements per sort workgroup (one wave)
 constexpr int kScanTile = 2048;         // elements per scan workgroup (256 x 8)
 
@@ -115,11 +117,12 @@ __global__ void __launch_bounds__(64) radix_hist(const uint32_t* __restrict__ ke
   for (uint32_t i = lane; i < BINS; i += 64) h[i] = 0;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * kTile;
-#pragma unroll 4
-  for (int j = 0; j < kItems; ++j) {
-    const int64_t e = base + j * 64 + lane;
-    if (e < n) atomicAdd(&h[(keys[e] >> shift) & (BINS - 1)], 1u);
-  }
+  uint32_t k[kItems];
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) k[j] = keys[min(base + j * 64 + lane, n - 1)];
+#pragma unroll
+  for (int j = 0; j < kItems; ++j)
+    if (base + j * 64 + lane < n) atomicAdd(&h[(k[j] >> shift) & (BINS - 1)], 1u);
   __syncthreads();
   for (uint32_t i = lane; i < BINS; i += 64) hist[(int64_t)i * nblocks + blockIdx.x] = h[i];
 }
@@ -131,15 +134,25 @@ __global__ void __launch_bounds__(64) radix_scatter(const uint32_t* __restrict__
   constexpr uint32_t BINS = 1u << BITS;
   __shared__ uint32_t cnt[BINS];
   const int lane = threadIdx.x;
+  // The whole tile's keys and values are requested first: one memory latency
+  // a tile, not one for each 64 of its elements (here and in radix_hist; 2^20
+  // updates, whole call: s32 384 -> 354 us, f32 579 -> 552).
+  const int64_t base = (int64_t)blockIdx.x * kTile;
+  uint32_t ks[kItems], vs[kItems];
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const int64_t e = min(base + j * 64 + lane, n - 1);
+    ks[j] = kin[e];
+    vs[j] = vin[e];
+  }
   for (uint32_t i = lane; i < BINS; i += 64) cnt[i] = offsets[(int64_t)i * nblocks + blockIdx.x];
   __syncthreads();
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  const int64_t base = (int64_t)blockIdx.x * kTile;
+#pragma unroll
   for (int j = 0; j < kItems; ++j) {
-    const int64_t e = base + j * 64 + lane;
-    const bool valid = e < n;
-    const uint32_t k = valid ? kin[e] : 0u;
-    const uint32_t v = valid ? vin[e] : 0u;
+    const bool valid = base + j * 64 + lane < n;
+    const uint32_t k = ks[j];
+    const uint32_t v = vs[j];
     const uint32_t d = (k >> shift) & (BINS - 1);
     // Lanes holding the same digit: intersect the per-bit ballots.
     uint64_t peers = __ballot(valid);
