@@ -111,6 +111,13 @@ int single_wide_tiles(int64_t N) {
   return gemv_wide_tiles(one);
 }
 
+// Row stride of a product's addend (GemmMember::add_ld). The product is
+// [batch][M][N] with N all of the right operand's free dims, whatever their
+// number, and so is an addend of the result's shape; a bias is one row for all.
+int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row) {
+  return row ? 0 : view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract).free;
+}
+
 // Writes the product to the dot's result, plus `add` (GemmMember::add, its
 // row stride add_ld) where the block tiles run it; returns whether they did.
 bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, const void* add,
@@ -341,13 +348,14 @@ void run_dot_residual(Device* dev, const Program& prog, const Op& op, std::vecto
   if (ot.dtype == DType::kBF16 || ot.dtype == DType::kF16) {
     // The block tiles add in their epilogue; any other kernel's product is
     // added to in place.
-    const int64_t n = row ? prog.type(add).elements() : ot.dims.empty() ? 1 : ot.dims.back();
+    const int64_t ld = dot_addend_stride(prog, op, row), n = dot_addend_stride(prog, op, false);
+    PJRTX_CHECK(prog.type(add).elements() == (row ? n : ot.elements()), Code::kInternal,
+                "dot_general: an addend of another size than the product's");
     vals[op.results[0]] = vals[out];
-    const bool added = run_dot_general(dev, prog, op, vals, vals[add]->ptr, row ? 0 : n);
+    const bool added = run_dot_general(dev, prog, op, vals, vals[add]->ptr, ld);
     vals[op.results[0]].reset();
     if (!added && n > 0)
-      launch_add_rows16(dev->stream(), vals[out]->ptr, vals[add]->ptr, ot.elements() / n, n, row ? 0 : n,
-                        ot.dtype == DType::kF16);
+      launch_add_rows16(dev->stream(), vals[out]->ptr, vals[add]->ptr, ot.elements() / n, n, ld, ot.dtype == DType::kF16);
     return;
   }
   vals[op.results[0]] = dev->allocate(ot.bytes());

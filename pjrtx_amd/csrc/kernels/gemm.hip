@@ -757,6 +757,7 @@ void launch_gemm(hipStream_t s, GemmGroup g, const GemmPlan& plan, const void* A
   for (int i = 0; i < g.count; ++i) {
     GemmMember& m = g.m[i];
     PJRTX_CHECK(!m.add || out_bytes == 2, Code::kInternal, "gemm: an addend needs a 16-bit result");
+    PJRTX_CHECK(!m.add || m.add_ld == 0 || m.add_ld == m.N, Code::kInternal, "gemm: an addend's rows are not the product's");
     m.tile0 = g.tiles_n;
     g.tiles_n += (m.N + t.tn - 1) / t.tn;
     if (plan.splits > 1) {

@@ -1450,7 +1450,9 @@ std::string Plan::describe(const Program& prog) const {
         }
         o << ",\"flops\":" << flops;
         if (s.lib == LibKind::kDotGroup) o << ",\"group_size\":" << s.group_ops.size();
-        if (s.dot_add >= 0) o << ",\"residual_add\":" << s.dot_add;
+        if (s.dot_add >= 0)
+          o << ",\"residual_add\":" << s.dot_add
+            << ",\"residual_stride\":" << dot_addend_stride(prog, prog.ops[s.lib_op], s.dot_add_row);
       }
       if (s.lib == LibKind::kWhile) o << ",\"while_trips\":" << s.while_trips;
       if (s.lib == LibKind::kAttention) {  // q.k and p.v over every (query, key) pair

@@ -257,6 +257,8 @@ bool fold_gather_index_wrap(Program* prog);
 bool fold_sort_iota(Program* prog);
 // transpose(dot_general(a, b)) as dot_general(b, a) (dot_general.cc).
 bool fold_dot_transpose(Program* prog);
+// Elements from one row of a merged addend to the next (dot_general.cc).
+int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row);
 
 // Turns decode-shaped dot and dot-group library steps into kGemv steps and
 // absorbs their row-fused prologues and elementwise epilogues

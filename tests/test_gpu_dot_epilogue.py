@@ -56,6 +56,29 @@ def test_added_row_and_residual(client, m, n, k, add, dt):
     _check_sum(got, av @ wv, xv, k, dt)
 
 
+# Right operands with no, two and three free dims; batched; contracted last.
+# 72 elements are summed in one launch of the block tiles, 8200 in k-splits.
+FREE_DIMS = [("mk", "k", "m"), ("mk", "kgh", "mgh"), ("mk", "ghk", "mgh"), ("km", "kgh", "mgh"), ("mk", "kfgh", "mfgh"),
+             ("amk", "kgh", "amgh"), ("bmk", "bk", "bm"), ("bmk", "bkgh", "bmgh"), ("bkm", "bghk", "bmgh")]
+
+
+@pytest.mark.parametrize("k", [72, 8200])
+@pytest.mark.parametrize("lhs,rhs,out", FREE_DIMS)
+@pytest.mark.parametrize("g,h", [(4, 32), (3, 7)])
+def test_residual_of_any_free_dims(client, lhs, rhs, out, g, h, k):
+    size = dict(a=2, b=3, f=2, g=g, h=h, k=k, m=130)
+    shape = lambda s: tuple(size[c] for c in s)  # noqa: E731
+    (a, av), (w, wv), (x, xv) = (_draw(shape(s), "bf16", i) for i, s in enumerate((lhs, rhs, out)))
+    b = Builder()
+    pa, pw, px = (b.param(shape(s), "bf16") for s in (lhs, rhs, out))
+    y = b.dot_general(pa, pw, batch=((0,), (0,)) if "b" in lhs else ((), ()),
+                      contract=((lhs.index("k"),), (rhs.index("k"),)))
+    exe = client.compile(b.build([b.add(px, y)]))
+    assert len(_steps(exe)) == 1
+    (got,) = exe(a, w, x, dtypes=["bf16"] * 3)
+    _check_sum(got, np.einsum(f"{lhs},{rhs}->{out}", av, wv), xv, k, "bf16")
+
+
 def test_batched_residual_and_bias(client):
     (a, av), (w, wv) = _draw((3, 40, 72), "bf16", 1), _draw((3, 72, 50), "bf16", 2)
     for shape in ((3, 40, 50), (50,)):

@@ -396,3 +396,29 @@ def test_attention_writes_its_transposed_result(plugin):
     assert kinds((2, 4, 128, 64), [0, 2, 1, 3], twice=True) == ["attention", "loop"]
     assert kinds((2, 4, 128, 64), [0, 1, 3, 2]) == ["attention", "loop"]
     assert kinds((2, 4, 8, 64), [0, 2, 1, 3]) == ["attention", "loop"]  # few queries
+
+
+@pytest.mark.parametrize("lhs,rhs,contract,add,stride", [
+    ((64, 128), (128, 8, 32), ((1,), (0,)), None, 256),            # heads and head dim: both are columns
+    ((512, 128), (512, 8, 32), ((0,), (0,)), None, 256),           # a [d, heads, head_dim] weight's gradient
+    ((4096, 128), (128,), ((1,), (0,)), None, 1),                  # a vector: one column
+    ((64, 128), (128, 2, 3, 4), ((1,), (0,)), None, 24),
+    ((16, 4, 128), (128, 40), ((2,), (0,)), None, 40),             # rows of two dims
+    ((64, 128), (128, 40), ((1,), (0,)), "row", 0),
+])
+def test_merged_addend_rows_are_the_products(plugin, lhs, rhs, contract, add, stride):
+    """An addend of the result's shape is read a product row at a time: its row
+    stride is all of the right operand's free dims, not the last one."""
+    b = Builder()
+    d = b.dot_general(b.param(lhs, "bf16"), b.param(rhs, "bf16"), contract=contract)
+    x = b.broadcast_in_dim(b.param((rhs[-1],), "bf16"), d.shape, [len(d.shape) - 1]) if add else b.param(d.shape, "bf16")
+    (step,) = plan(plugin, b.build([b.add(d, x)]))["steps"]
+    assert step["residual_stride"] == stride
+
+
+@pytest.mark.parametrize("rhs,batch,stride", [((3, 128), ((0,), (0,)), 1), ((3, 128, 4, 8), ((0,), (0,)), 32)])
+def test_merged_addend_rows_of_batched_products(plugin, rhs, batch, stride):
+    b = Builder()
+    d = b.dot_general(b.param((3, 40, 128), "bf16"), b.param(rhs, "bf16"), batch=batch, contract=((2,), (1,)))
+    (step,) = plan(plugin, b.build([b.add(b.param(d.shape, "bf16"), d)]))["steps"]
+    assert step["residual_stride"] == stride
