@@ -591,7 +591,9 @@ __global__ void __launch_bounds__(256, (PipeShape<D, NQT, KW>::kPerCu))
       for (int qt = 0; qt < NQT; ++qt) {
         float r = mx[qt];
         if constexpr (kRound) r = round16<kF16>(r);
-        const bool up = mx[qt] * c2 > limit[qt];
+        // On the rounded max: f16 scores below -65520 all round to -inf, and a
+        // block of those adds nothing (its max minus itself would be NaN).
+        const bool up = r * c2 > limit[qt];
         const float mnew = up ? r * c2 : mc[qt];
         const float alpha = limit[qt] == -INFINITY ? (up ? 0.f : 1.f) : __builtin_amdgcn_exp2f(mc[qt] - mnew);
         mc[qt] = mnew;

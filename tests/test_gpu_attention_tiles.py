@@ -71,6 +71,30 @@ def test_values_that_are_not_finite(client, sizes):
     assert_close16(np.where(keep, got, 0), np.where(keep, want, 0))
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("bh", [(1, 3), (4, 72)])        # 32 queries and two key ways, 128 queries
+@pytest.mark.parametrize("blocks", [(0,), (0, 1), (2,), (0, 1, 2, 3)])
+def test_f16_scores_that_overflow(client, d, bh, blocks):
+    """Key blocks of 64 whose f16 scores all round to -inf weigh nothing, also
+    before any other block was seen; a row of nothing else is NaN."""
+    b, h = bh
+    s = 256
+    rng = np.random.default_rng(d)
+    q, k, v = (rng.standard_normal((b, h, s, d)).astype(np.float32) for _ in range(3))
+    q = np.abs(q) / d ** 0.5 + 16
+    k /= 64
+    for blk in blocks:
+        k[:, :, 64 * blk:64 * blk + 64] = -66000 / (16 * d) - 8  # a score of -66000 and below
+    args = [to_bits(x, "f16") for x in (q, k, v)]
+    (out,) = client.compile(programs.c3_attention(b, h, s, d, False, dtype="f16"))(*args, dtypes=["f16"] * 3)
+    with np.errstate(invalid="ignore"):
+        want = A.attention_graph_ref(*(from_bits(x, "f16") for x in args), "f16")
+    got = from_bits(out, "f16")
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    assert np.isnan(want).all() == (len(blocks) == 4)
+    assert_close16(np.nan_to_num(got), np.nan_to_num(want))
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
 @pytest.mark.parametrize("shape", [(1, 16, 100, 128), (3, 5, 33, 64), (2, 3, 17, 40), (2, 130, 160, 128)])
 def test_result_written_transposed(client, shape, dt):
