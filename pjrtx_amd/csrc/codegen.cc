@@ -847,10 +847,10 @@ void KernelGen::loop(Step& s) {
     // (the window spans that dim, a multiple of vec): one store at the
     // window position of `base`.
     const Dims& od = prog_.type(ww->second.operand).dims;
-    out_ << "{ uint32_t rem = base, dst = 0;\n";
+    out_ << "{ idx_t rem = base, dst = 0;\n";
     int64_t stride = 1;
     for (int d = static_cast<int>(od.size()) - 1; d >= 0; --d) {
-      out_ << "{ const uint32_t c = rem % " << s.loop_shape[d] << "u; rem /= " << s.loop_shape[d] << "u; dst += (c + (uint32_t)ws"
+      out_ << "{ const idx_t c = rem % " << s.loop_shape[d] << "u; rem /= " << s.loop_shape[d] << "u; dst += (c + (idx_t)ws"
            << o << "_" << d << ") * " << stride << "u; }\n";
       stride *= od[d];
     }

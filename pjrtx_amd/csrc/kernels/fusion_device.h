@@ -130,8 +130,10 @@ PJRTX_DEV pjrtx_v4 ld16(const void* p) {
   else return *reinterpret_cast<const pjrtx_v4*>(p);
 }
 
-template <typename S, int N, bool NT = false>
-PJRTX_DEV void ldv(S (&dst)[N], const S* __restrict__ src, uint32_t base, uint32_t n, bool full) {
+// I, J: the kernel's index type (64 bits where a tensor has 2^31 elements or
+// more) or a literal's.
+template <typename S, int N, bool NT = false, typename I, typename J>
+PJRTX_DEV void ldv(S (&dst)[N], const S* __restrict__ src, I base, J n, bool full) {
   if (full) {
     constexpr int kBytes = (int)sizeof(S) * N;
     if constexpr (kBytes % 16 == 0) {
@@ -178,8 +180,8 @@ PJRTX_DEV void keep_live(const S (&a)[N]) {
   }
 }
 
-template <typename S, int N>
-PJRTX_DEV void stv(S* __restrict__ dst, uint32_t base, const S (&src)[N], uint32_t n, bool full) {
+template <typename S, int N, typename I, typename J>
+PJRTX_DEV void stv(S* __restrict__ dst, I base, const S (&src)[N], J n, bool full) {
   if (full) {
     constexpr int kBytes = (int)sizeof(S) * N;
     if constexpr (kBytes % 16 == 0) {

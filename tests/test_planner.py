@@ -3,6 +3,7 @@ kernel generator (no GPU). Structural counterparts of the reference's planner
 tests (reference: src/backend/mlx_metal/program_fusion.zig:116-227,
 executable_metal_graph_lowering_tests.zig:8-204)."""
 import json
+import re
 
 import pytest
 
@@ -422,3 +423,16 @@ def test_merged_addend_rows_of_batched_products(plugin, rhs, batch, stride):
     d = b.dot_general(b.param((3, 40, 128), "bf16"), b.param(rhs, "bf16"), batch=batch, contract=((2,), (1,)))
     (step,) = plan(plugin, b.build([b.add(b.param(d.shape, "bf16"), d)]))["steps"]
     assert step["residual_stride"] == stride
+
+
+@pytest.mark.parametrize("dims", [[0], [1]])
+def test_vector_accesses_take_64_bit_positions(plugin, dims):
+    """Past 2^32 elements a position does not fit 32 bits: the vector loads
+    and stores take the kernel's index type as it is."""
+    b = Builder()
+    x = b.param((65537, 65536), "bf16")
+    src = plugin.kernel_source(b.build([b.max(x, dims), b.add(x, x)]))
+    assert "typedef uint64_t idx_t" in src and "typedef uint32_t idx_t" not in src and "ldv<" in src and "stv<" in src
+    for fn in ("ldv", "stv"):
+        (sig,) = re.findall(r"PJRTX_DEV void %s\((.*)\) \{" % fn, src)
+        assert "uint32_t base" not in sig and "I base" in sig
