@@ -919,6 +919,25 @@ Executable::Loaded* Executable::loaded_for(Device* dev, bool may_evict) {
   return raw;
 }
 
+namespace {
+// What a step takes from an installed arena after this (partials, sort words,
+// copies of operands) goes back when the step has been queued: the next step's
+// work follows it on the stream.
+class StepTemporaries {
+ public:
+  explicit StepTemporaries(Arena* a) : a_(a), used_(a ? a->used : 0) {}
+  ~StepTemporaries() {
+    if (a_) a_->used = used_;
+  }
+  StepTemporaries(const StepTemporaries&) = delete;
+  StepTemporaries& operator=(const StepTemporaries&) = delete;
+
+ private:
+  Arena* a_;
+  size_t used_;
+};
+}  // namespace
+
 void Executable::run_step(Loaded* L, size_t si, std::vector<MemRef>& vals, int phase) {
   const Step& s = plan_.steps[si];
   Device* dev = L->dev;
@@ -938,7 +957,10 @@ void Executable::run_step(Loaded* L, size_t si, std::vector<MemRef>& vals, int p
       } else {
         for (int v : s.outputs) vals[v] = dev->allocate(prog_.type(v).bytes());
       }
-      run_library_step(dev, prog_, s, vals);
+      {
+        StepTemporaries temporaries(thread_arena());
+        run_library_step(dev, prog_, s, vals);
+      }
       stats_.library_calls++;
       return;
     case StepKind::kLoop:
@@ -959,12 +981,17 @@ void Executable::run_step(Loaded* L, size_t si, std::vector<MemRef>& vals, int p
       ptrs.reserve(s.inputs.size() + s.outputs.size() + 2);
       for (int v : s.inputs) ptrs.push_back(vals[v] ? vals[v]->ptr : nullptr);
       for (int v : s.outputs) ptrs.push_back(vals[v]->ptr);
+      StepTemporaries temporaries(thread_arena());
       MemRef arena_scratch;
       // A fused combine folds the partials inside the main launch when the
       // device places workgroups round-robin on its XCDs; otherwise the
       // `_combine` kernel runs after it.
       const uint32_t fused_mode = s.fused_combine && dev->xcd_round_robin() ? 1u : 0u;
-      if (s.scratch_bytes && thread_arena() && phase != 1) {
+      // Column splits also run where the fixed block is full: their partials
+      // then go to the step's own scratch, held since the program was loaded.
+      const bool in_arena = thread_arena() && phase != 1 &&
+                            !(s.col_lanes && scratch_left(dev) < static_cast<int64_t>(s.scratch_bytes));
+      if (s.scratch_bytes && in_arena) {
         // Allocation-free execute: partial slots from the fixed block; the
         // arrival counters of a one-launch fold must start at zero.
         arena_scratch = dev->allocate(s.scratch_bytes);

@@ -109,6 +109,38 @@ def test_noalloc_rejects_a_plan_beyond_the_fixed_block(client):
         np.testing.assert_array_equal(o.to_numpy(r.dtype, r.shape), r)
 
 
+def _check_noalloc(client, exe, arrays, dtypes):
+    args, ref = [DeviceArray.from_numpy(client.p, a) for a in arrays], exe(*arrays, dtypes=dtypes)
+    outs = [DeviceArray(client.p, r.nbytes) for r in ref]
+    exe.execute_noalloc([a.ptr for a in args], [o.ptr for o in outs])
+    client.p.hip_check(client.p.lib.pjrtx_hip_synchronize(0))
+    for o, r in zip(outs, ref):
+        np.testing.assert_array_equal(o.to_numpy(r.dtype, r.shape), r)
+    for d in args + outs:
+        d.free()
+
+
+def test_noalloc_steps_give_their_temporaries_back(client):
+    """Products whose k-split partials would fill the fixed block
+    between them: each step's go back before the next step's results."""
+    rng = np.random.default_rng(2)
+    b = Builder()
+    w = b.param((4096, 512), "bf16")
+    xs = [b.param((512, 4096), "bf16") for _ in range(28)]
+    # Of whole numbers: every order of their sums is exact, whatever the splits.
+    arrays = [ops.f32_to_bf16_bits(rng.integers(-2, 3, s.shape).astype(np.float32)) for s in [w] + xs]
+    exe = client.compile(b.build([b.dot_general(x, w, contract=((1,), (0,))) for x in xs]))
+    _check_noalloc(client, exe, arrays, ["bf16"] * 29)
+
+
+def test_noalloc_column_splits_without_room(client):
+    """A column sum beside a result that leaves 80 KB of the fixed block."""
+    b = Builder()
+    x = b.param((4090, 4096), "f32")
+    exe = client.compile(b.build([b.add(x, x), b.sum(x, [0])]))
+    _check_noalloc(client, exe, [np.random.default_rng(3).standard_normal((4090, 4096)).astype(np.float32)], ["f32"])
+
+
 def test_noalloc_rejects_bad_arguments(client):
     exe = client.compile(programs.c2_argmax_f16_reductions(8, 4096))
     with pytest.raises(PjrtError) as e:
