@@ -51,8 +51,10 @@ struct SortGather {
 };
 
 // Bytes of device scratch sort_rows needs for these rows and out_n, at most
-// about max_bytes where a path with less exists (rows that merge take two
-// buffers of 8 bytes an element; a bitonic network one of padded rows).
+// max_bytes where a path with less exists: rows that merge take two buffers of
+// 8 bytes an element, a bitonic network one of padded rows; up to 256 first
+// words take two lists, which longer chunks of the row make shorter. (257 to
+// 4096 first words have one path, with two lists of blocks of 8192.)
 size_t sort_scratch_bytes(const SortRows& r, int64_t out_n, int64_t max_bytes);
 
 // Sorts every row of operand 0 (`keys`) and writes the first `g.out_n`

@@ -14,9 +14,11 @@
 //    ... by merge path, and keeps the first `keep` words or writes the results.
 //  * merge_runs: merges neighbouring sorted runs of a row from HBM.
 //  * topk_select: the first k <= 256 words of a chunk, without sorting it.
+//  * merge_pieces: the first k words of rows whose positions a word does not
+//    hold (2^30 and more), from those of their pieces.
 //  * sort_local, bitonic_global, sort_write: a bitonic network over padded
 //    rows in one buffer, for a caller whose fixed scratch block does not hold
-//    the two buffers merging needs, and for rows of 2^30 elements and more.
+//    the two buffers merging needs, and for whole sorts of such rows.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -749,6 +751,40 @@ __global__ void __launch_bounds__(kTopkThreads) topk_half_kernel(TopkPass p) {
   topk_rank(p, row, blk, tid, m, cand);
 }
 
+// A row's results from the sorted first words of its pieces, whose words hold
+// positions within the piece: a word's rank is its own index plus the words
+// ahead of it in every other piece (equal keys of earlier pieces come first).
+struct PieceMerge {
+  SortRows r;
+  SortGather g;
+  const double* list = nullptr;  // [piece][row][out_n]
+  int pieces = 0;
+  int64_t piece_len = 0;         // of all but the last
+};
+__global__ void merge_pieces_kernel(PieceMerge p) {
+  const int64_t k = p.g.out_n, t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= p.pieces * p.r.rows * k) return;
+  const int piece = static_cast<int>(t / (p.r.rows * k));
+  const int64_t row = t / k % p.r.rows, i = t % k;
+  const auto words = [&](int q) { return min(k, min(p.piece_len, p.r.n - q * p.piece_len)); };
+  if (i >= words(piece)) return;
+  const double w = p.list[t];
+  int64_t rank = i;
+  for (int q = 0; q < p.pieces && rank < k; ++q) {
+    if (q == piece) continue;
+    const double* other = p.list + (q * p.r.rows + row) * k;
+    int64_t lo = 0, hi = words(q);
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      const uint32_t x = word_image(other[mid]);
+      if (x < word_image(w) || (x == word_image(w) && q < piece)) lo = mid + 1;
+      else hi = mid;
+    }
+    rank += lo;
+  }
+  if (rank < k) gather_one(p.g, p.r, row, rank, piece * p.piece_len + word_pos(w));
+}
+
 int64_t pow2_at_least(int64_t v) {
   int64_t p = 1;
   while (p < v) p <<= 1;
@@ -779,7 +815,9 @@ enum SortPath {
 struct Layout {
   SortPath path = kPathMerge;
   int share = 1;               // topk: eight-word groups a thread
-  int64_t len1 = 0;            // topk / keep: list length after round one
+  int pieces = 1;              // topk / keep: parts a row is taken in
+  int64_t piece_len = 0;       // elements of all but the last
+  int64_t len1 = 0;            // topk / keep: list length after a piece's round one
   int64_t p = 0;               // bitonic: padded row length
   size_t bytes = 0;
 };
@@ -804,17 +842,21 @@ Layout layout_of(const SortRows& r, int64_t out_n, int64_t max_bytes) {
     L.bytes = static_cast<size_t>(r.rows * L.p) * 8;
     return L;
   };
-  if (r.n >= kWordRows) return bitonic();
-  if (out_n < r.n && out_n <= kTopkMax) {
+  const bool topk = out_n < r.n && out_n <= kTopkMax, keep = r.n > kSortTile && out_n <= kSortTile / 2;
+  if (r.n >= kWordRows && !topk && !keep) return bitonic();
+  L.piece_len = r.n < kWordRows ? std::max<int64_t>(r.n, 1) : kWordRows / 2;
+  L.pieces = static_cast<int>(ceil_div(r.n, L.piece_len));
+  const size_t merged = L.pieces > 1 ? static_cast<size_t>(L.pieces * r.rows * out_n) * 8 : 0;
+  if (topk) {
     L.path = kPathTopk;
-    L.share = topk_share(r, r.n);
-    const int64_t blocks = topk_blocks(L.share, r.n);
+    L.share = topk_share(r, L.piece_len);
+    const int64_t blocks = topk_blocks(L.share, L.piece_len);
     L.len1 = blocks * out_n;
-    L.bytes = blocks > 1 ? static_cast<size_t>(2 * r.rows * L.len1) * 8 : 0;
-  } else if (r.n > kSortTile && out_n <= kSortTile / 2) {
+    L.bytes = blocks > 1 ? static_cast<size_t>(2 * r.rows * L.len1) * 8 + merged : 0;
+  } else if (keep) {
     L.path = kPathKeep;
-    L.len1 = ceil_div(r.n, kSortTile) * out_n;
-    L.bytes = static_cast<size_t>(2 * r.rows * L.len1) * 8;
+    L.len1 = ceil_div(L.piece_len, kSortTile) * out_n;
+    L.bytes = static_cast<size_t>(2 * r.rows * L.len1) * 8 + merged;
   } else {
     // One buffer per side of a merge round; the last round writes the results.
     L.bytes = r.n <= kSortTile ? 0 : static_cast<size_t>((r.n <= 2 * kSortTile ? 1 : 2) * r.rows * r.n) * 8;
@@ -854,6 +896,59 @@ void topk_blocks_launch(hipStream_t s, TopkPass p, int share) {
   check_launch("topk_select");
 }
 
+WordSource key_source(const SortRows& r, const void* keys) {
+  WordSource src;
+  src.keys = keys;
+  src.len = r.n;
+  src.vec = r.inner == 1 && r.key_bits >= 16 && (r.n * r.key_bits / 8) % 16 == 0 && reinterpret_cast<uintptr_t>(keys) % 16 == 0;
+  return src;
+}
+
+// The first out_n words of every row of `src` (kPathTopk, kPathKeep), as the
+// results or, with `dst`, as a list of out_n words a row (ends after the last
+// of fewer). `lists` holds two lists of len1 words a row.
+void first_words(hipStream_t s, const SortRows& r, const WordSource& src, const SortGather& g, const Layout& L,
+                 double* lists, double* dst) {
+  double *a = lists, *b = lists + r.rows * L.len1;
+  if (L.path == kPathTopk) {
+    TopkPass p;
+    p.r = r;
+    p.src = src;
+    p.need = static_cast<int>(g.out_n);
+    p.g = g;
+    int share = L.share;
+    for (;;) {
+      p.blocks_per_row = topk_blocks(share, p.src.len);
+      const bool last = p.blocks_per_row == 1;
+      p.dst = last ? dst : a;
+      topk_blocks_launch(s, p, share);
+      if (last) return;
+      p.src.list = a;
+      p.src.len = p.src.stride = p.blocks_per_row * p.need;
+      share = topk_share(r, p.src.len);
+      std::swap(a, b);
+    }
+  }
+  BlockPass p;
+  p.r = r;
+  p.src = src;
+  p.g = g;
+  p.keep = g.out_n;
+  while (p.src.len > kSortTile) {
+    p.blocks_per_row = ceil_div(p.src.len, kSortTile);
+    p.dst = a;
+    p.dst_stride = p.blocks_per_row * p.keep;
+    sort_blocks(s, p, kSortTile);
+    p.src.list = a;
+    p.src.len = p.src.stride = p.dst_stride;
+    std::swap(a, b);
+  }
+  p.blocks_per_row = 1;
+  p.dst = dst;
+  p.dst_stride = p.keep;
+  sort_blocks(s, p, dst ? std::max(p.src.len, p.keep) : p.src.len);
+}
+
 }  // namespace
 
 size_t sort_scratch_bytes(const SortRows& r, int64_t out_n, int64_t max_bytes) {
@@ -866,31 +961,34 @@ void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGat
   PJRTX_CHECK(r.key_bits == 8 || r.key_bits == 16 || r.key_bits == 32, Code::kUnimplemented,
               "sort: keys wider than 32 bits are not supported");
   const Layout L = layout_of(r, g.out_n, max_bytes);
-  WordSource src;
-  src.keys = keys;
-  src.len = r.n;
-  src.vec = r.inner == 1 && r.key_bits >= 16 && (r.n * r.key_bits / 8) % 16 == 0 && reinterpret_cast<uintptr_t>(keys) % 16 == 0;
-  double* a = static_cast<double*>(scratch);
-  double* b = a + r.rows * (L.path == kPathMerge ? r.n : L.len1);
-  if (L.path == kPathTopk) {
-    TopkPass p;
-    p.r = r;
-    p.src = src;
-    p.need = static_cast<int>(g.out_n);
-    p.g = g;
-    int share = L.share;
-    for (;;) {
-      p.blocks_per_row = topk_blocks(share, p.src.len);
-      p.dst = p.blocks_per_row == 1 ? nullptr : a;
-      topk_blocks_launch(s, p, share);
-      if (!p.dst) return;
-      p.src.list = a;
-      p.src.len = p.src.stride = p.blocks_per_row * p.need;
-      share = topk_share(r, p.src.len);
-      std::swap(a, b);
+  if (L.pieces > 1) {
+    PJRTX_CHECK(r.inner == 1, Code::kInternal, "sort: a row in pieces must be contiguous");
+    // Each piece's first out_n words, through the same two lists.
+    double* const lists = static_cast<double*>(scratch);
+    PieceMerge m;
+    m.r = r;
+    m.g = g;
+    m.pieces = L.pieces;
+    m.piece_len = L.piece_len;
+    double* const merged = lists + 2 * r.rows * L.len1;
+    m.list = merged;
+    for (int q = 0; q < L.pieces; ++q) {
+      WordSource src = key_source(r, static_cast<const char*>(keys) + q * L.piece_len * (r.key_bits / 8));
+      src.len = std::min(L.piece_len, r.n - q * L.piece_len);
+      first_words(s, r, src, g, L, lists, merged + q * r.rows * g.out_n);
     }
+    const unsigned grid = grid_of(ceil_div(L.pieces * r.rows * g.out_n, 256), 1);
+    hipLaunchKernelGGL(merge_pieces_kernel, dim3(grid), dim3(256), 0, s, m);
+    check_launch("merge_pieces");
+    return;
   }
-  if (L.path == kPathKeep || L.path == kPathMerge) {
+  const WordSource src = key_source(r, keys);
+  if (L.path == kPathTopk || L.path == kPathKeep) {
+    first_words(s, r, src, g, L, static_cast<double*>(scratch), nullptr);
+    return;
+  }
+  if (L.path == kPathMerge) {
+    double *a = static_cast<double*>(scratch), *b = a + r.rows * r.n;
     BlockPass p;
     p.r = r;
     p.src = src;
@@ -901,25 +999,9 @@ void sort_rows(hipStream_t s, const SortRows& r, const void* keys, const SortGat
     }
     p.blocks_per_row = ceil_div(r.n, kSortTile);
     p.dst = a;
-    p.keep = L.path == kPathKeep ? g.out_n : kSortTile;
-    p.dst_stride = L.path == kPathKeep ? p.blocks_per_row * p.keep : r.n;
+    p.keep = kSortTile;
+    p.dst_stride = r.n;
     sort_blocks(s, p, kSortTile);
-    if (L.path == kPathKeep) {
-      for (;;) {
-        p.src.list = a;
-        p.src.len = p.src.stride = p.dst_stride;
-        if (p.src.len <= kSortTile) break;
-        p.blocks_per_row = ceil_div(p.src.len, kSortTile);
-        p.dst_stride = p.blocks_per_row * p.keep;
-        p.dst = b;
-        sort_blocks(s, p, kSortTile);
-        std::swap(a, b);
-      }
-      p.blocks_per_row = 1;
-      p.dst = nullptr;
-      sort_blocks(s, p, p.src.len);
-      return;
-    }
     MergePass m;
     m.r = r;
     m.g = g;

@@ -1454,6 +1454,9 @@ std::string Plan::describe(const Program& prog) const {
           o << ",\"residual_add\":" << s.dot_add
             << ",\"residual_stride\":" << dot_addend_stride(prog, prog.ops[s.lib_op], s.dot_add_row);
       }
+      if (s.lib == LibKind::kSort)
+        o << ",\"scratch_bytes\":" << sort_op_scratch(prog, prog.ops[s.lib_op], int64_t(1) << 60)
+          << ",\"least_scratch_bytes\":" << sort_op_scratch(prog, prog.ops[s.lib_op], 0);
       if (s.lib == LibKind::kWhile) o << ",\"while_trips\":" << s.while_trips;
       if (s.lib == LibKind::kAttention) {  // q.k and p.v over every (query, key) pair
         const Op& d = prog.ops[s.lib_op];

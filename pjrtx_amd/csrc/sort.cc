@@ -140,6 +140,11 @@ bool fold_sort_iota(Program* prog) {
 
 void check_sort_supported(const Program& prog, const Op& op) { (void)spec_of(prog, op); }
 
+int64_t sort_op_scratch(const Program& prog, const Op& op, int64_t max_bytes) {
+  const SortSpec sp = spec_of(prog, op);
+  return static_cast<int64_t>(sort_scratch_bytes(sp.rows, sp.out_n, max_bytes));
+}
+
 void run_sort(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals) {
   const SortSpec sp = spec_of(prog, op);
   SortGather g;

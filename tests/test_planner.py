@@ -378,6 +378,27 @@ def test_sort_writes_positions_itself(plugin):
     assert len(_dot_steps(plugin, make(1, first=True))) == 2   # the key itself
 
 
+def _top_k_step(plugin, rows, n, k, dt="bf16"):
+    b = Builder()
+    (step,) = plan(plugin, b.build(list(b.top_k(b.param((rows, n), dt), k))))["steps"]
+    return step
+
+
+def _kept_words(rows, n, k):
+    """Bytes of two lists that hold the first k (rounded up to a power of two)
+    of every 4096 words of 8 bytes: what a top_k over long rows may take."""
+    return 2 * rows * -(-n // 4096) * (1 << (k - 1).bit_length()) * 8
+
+
+@pytest.mark.parametrize("dt", ["s8", "bf16"])
+@pytest.mark.parametrize("k", [1, 50, 256, 257, 2048])
+def test_top_k_of_rows_that_words_cannot_number(plugin, k, dt):
+    """A word holds 30 bits of position; longer rows are taken in pieces, not
+    sorted whole (16 GB of words and hundreds of passes at 2^30 elements)."""
+    for n in (2 ** 30 - 8, 2 ** 30, 2 ** 30 + 24, 2 ** 31 - 8):
+        assert _top_k_step(plugin, 2, n, k, dt)["scratch_bytes"] <= _kept_words(2, n, k)
+
+
 def attention_then_transpose(shape, perm, dt="bf16", twice=False):
     """c3_attention whose result is transposed (and also returned, `twice`)."""
     mlir = lambda d: "tensor<" + "x".join(map(str, d)) + f"x{dt}>"  # noqa: E731
