@@ -849,10 +849,13 @@ Layout layout_of(const SortRows& r, int64_t out_n, int64_t max_bytes) {
   const size_t merged = L.pieces > 1 ? static_cast<size_t>(L.pieces * r.rows * out_n) * 8 : 0;
   if (topk) {
     L.path = kPathTopk;
-    L.share = topk_share(r, L.piece_len);
-    const int64_t blocks = topk_blocks(L.share, L.piece_len);
-    L.len1 = blocks * out_n;
-    L.bytes = blocks > 1 ? static_cast<size_t>(2 * r.rows * L.len1) * 8 + merged : 0;
+    // Longer chunks, whose lists are shorter, where those of the best do not fit.
+    for (L.share = topk_share(r, L.piece_len);; L.share *= 2) {
+      const int64_t blocks = topk_blocks(L.share, L.piece_len);
+      L.len1 = blocks * out_n;
+      L.bytes = blocks > 1 ? static_cast<size_t>(2 * r.rows * L.len1) * 8 + merged : 0;
+      if (static_cast<int64_t>(L.bytes) <= max_bytes || L.share == 4) break;
+    }
   } else if (keep) {
     L.path = kPathKeep;
     L.len1 = ceil_div(L.piece_len, kSortTile) * out_n;

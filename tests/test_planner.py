@@ -399,6 +399,14 @@ def test_top_k_of_rows_that_words_cannot_number(plugin, k, dt):
         assert _top_k_step(plugin, 2, n, k, dt)["scratch_bytes"] <= _kept_words(2, n, k)
 
 
+@pytest.mark.parametrize("rows,n,k", [(1, 8193, 256), (3, 40000, 256), (16, 32000, 64), (64, 128256, 128), (200, 20000, 1),
+                                      (1, 10 ** 7, 256), (64, 128256, 300), (2, 50000, 4096), (1, 2 ** 30, 256)])
+def test_top_k_takes_no_more_room_than_kept_words(plugin, rows, n, k):
+    """Where scratch is a fixed block, a top_k makes do with the kept words of
+    each 4096, however few workgroups that leaves."""
+    assert _top_k_step(plugin, rows, n, k)["least_scratch_bytes"] <= _kept_words(rows, n, k)
+
+
 def attention_then_transpose(shape, perm, dt="bf16", twice=False):
     """c3_attention whose result is transposed (and also returned, `twice`)."""
     mlir = lambda d: "tensor<" + "x".join(map(str, d)) + f"x{dt}>"  # noqa: E731

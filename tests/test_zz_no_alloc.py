@@ -133,6 +133,15 @@ def test_noalloc_steps_give_their_temporaries_back(client):
     _check_noalloc(client, exe, arrays, ["bf16"] * 29)
 
 
+def test_noalloc_top_k_with_little_room(client):
+    """The room is what longer chunks' lists need, not the fastest chunks'."""
+    rng = np.random.default_rng(4)
+    b = Builder()
+    big, x = b.param((16262, 1024), "f32"), b.param((1, 300000), "f32")
+    exe = client.compile(b.build([b.add(big, big), *b.top_k(x, 256)]))
+    _check_noalloc(client, exe, [rng.standard_normal(s).astype(np.float32) for s in ((16262, 1024), (1, 300000))], ["f32"] * 2)
+
+
 def test_noalloc_column_splits_without_room(client):
     """A column sum beside a result that leaves 80 KB of the fixed block."""
     b = Builder()
