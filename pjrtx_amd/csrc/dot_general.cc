@@ -62,6 +62,27 @@ OperandView view_of(const TensorType& t, const Dims& batch, const Dims& contract
   return v;
 }
 
+// Both operands of a product as the block tiles read them: K-contiguous as it
+// is, else M- or N-contiguous. `ready` is false where an operand is neither.
+struct DotLayout {
+  bool ready = false, a_kmajor = false, b_kmajor = false;
+};
+DotLayout layout_of(const OperandView& a, const OperandView& b) {
+  DotLayout l;
+  l.a_kmajor = a.ks == 1 || a.k == 1;
+  l.b_kmajor = (b.ks == 1 || b.k == 1) && !(b.fs == 1 && b.free != 1);
+  l.ready = a.ok && b.ok && (l.a_kmajor || a.fs == 1 || a.free == 1) && (l.b_kmajor || b.fs == 1 || b.free == 1);
+  return l;
+}
+
+// True where every 16-byte piece of the operand's rows lies on a 16-byte
+// boundary (of an aligned base) and inside the operand: an operand with rows
+// that do not is copied into padded ones.
+bool whole_rows(const OperandView& v, bool kmajor) {
+  const int64_t rows = kmajor ? v.free : v.k, cols = kmajor ? v.k : v.free, ld = kmajor ? v.fs : v.ks;
+  return (rows == 1 || ld % 8 == 0) && (v.batch == 1 || v.bs % 8 == 0) && (cols % 8 == 0 || (!kmajor && rows > 1));
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 // Copies `t` into a canonical [batch][free][k] (or [batch][k][free] when
@@ -118,6 +139,16 @@ int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row) {
   return row ? 0 : view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract).free;
 }
 
+std::string describe_dot(const Program& prog, const Op& dot) {
+  const OperandView a = view_of(prog.type(dot.operands[0]), dot.lhs_batch, dot.lhs_contract);
+  const OperandView b = view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract);
+  const DotLayout l = layout_of(a, b);
+  const auto one = [](const OperandView& v, bool kmajor) {
+    return !v.ok ? "\"copied\"" : !whole_rows(v, kmajor) ? "\"padded\"" : "\"read\"";
+  };
+  return std::string("[") + one(a, l.a_kmajor) + "," + one(b, l.b_kmajor) + "]";
+}
+
 // Writes the product to the dot's result, plus `add` (GemmMember::add, its
 // row stride add_ld) where the block tiles run it; returns whether they did.
 bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector<MemRef>& vals, const void* add,
@@ -167,13 +198,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
       B = b_copy->ptr;
       b = OperandView{batch, N, K, N * K, K, 1, true};
     }
-    // K-contiguous as it is, else M- or N-contiguous; an operand with rows
-    // that are not 16-byte aligned is copied into padded ones.
-    bool a_kmajor = false, b_kmajor = false;
-    const auto aligned_rows = [&](const void* p, const OperandView& v, bool kc) {
-      const int64_t ld = kc ? v.fs : v.ks, rows = kc ? v.free : v.k;
-      return aligned16(p) && (rows == 1 || ld % 8 == 0) && (batch == 1 || v.bs % 8 == 0) && (!kc || K % 8 == 0);
-    };
+    const auto aligned_rows = [&](const void* p, const OperandView& v, bool kc) { return aligned16(p) && whole_rows(v, kc); };
     const auto pad = [&](const void** p, OperandView* v, bool kc, MemRef* mem) {
       const int64_t rows = kc ? v->free : v->k, cols = kc ? v->k : v->free, ldp = (cols + 7) / 8 * 8;
       if (batch >= 65536 || rows * (ldp / 8) >= (int64_t(1) << 38) || !fits(batch * rows * ldp * 2)) return false;
@@ -186,12 +211,9 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
       (kc ? v->ks : v->fs) = 1;
       return true;
     };
-    bool ready = a.ok && b.ok;
-    if (ready) {
-      a_kmajor = a.ks == 1 || K == 1;
-      b_kmajor = (b.ks == 1 || K == 1) && !(b.fs == 1 && N != 1);
-      ready = (a_kmajor || a.fs == 1 || M == 1) && (b_kmajor || b.fs == 1 || N == 1);
-    }
+    const DotLayout lay = layout_of(a, b);
+    const bool a_kmajor = lay.a_kmajor, b_kmajor = lay.b_kmajor;
+    bool ready = lay.ready;
     // Decode rows: W streamed once. (K may be any length for an N-contiguous
     // W; a K-contiguous one needs 16-byte rows.)
     if (ready && M <= 8 && (a.ks == 1 || K == 1) && aligned_rows(B, b, b_kmajor) && (b_kmajor || N % 8 == 0) &&

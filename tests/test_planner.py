@@ -465,3 +465,22 @@ def test_vector_accesses_take_64_bit_positions(plugin, dims):
     for fn in ("ldv", "stv"):
         (sig,) = re.findall(r"PJRTX_DEV void %s\((.*)\) \{" % fn, src)
         assert "uint32_t base" not in sig and "I base" in sig
+
+
+def _operands(plugin, lhs, rhs, contract, batch=((), ())):
+    b = Builder()
+    d = b.dot_general(b.param(lhs, "bf16"), b.param(rhs, "bf16"), batch=batch, contract=contract)
+    (step,) = plan(plugin, b.build([d]))["steps"]
+    return step["operands"]
+
+
+def test_operands_are_read_within_their_bounds(plugin):
+    """The block tiles read whole 16-byte pieces: an operand whose only row
+    ends inside one (an outer product's right side) is padded like ragged rows."""
+    assert _operands(plugin, (64, 40), (40, 24), ((1,), (0,))) == ["read", "read"]
+    assert _operands(plugin, (64, 40), (40, 23), ((1,), (0,))) == ["read", "padded"]
+    assert _operands(plugin, (40, 64), (40, 24), ((0,), (0,))) == ["read", "read"]
+    assert _operands(plugin, (64, 1), (1, 24), ((1,), (0,))) == ["padded", "read"]
+    assert _operands(plugin, (64, 1), (1, 23), ((1,), (0,))) == ["padded", "padded"]
+    assert _operands(plugin, (64,), (23,), ((), ())) == ["padded", "padded"]
+    assert _operands(plugin, (3, 64, 1), (3, 1, 24), ((2,), (1,)), ((0,), (0,))) == ["padded", "read"]
