@@ -28,21 +28,15 @@ bool merge(const Dims& dims, const int64_t* strides, const std::vector<int64_t>&
   *size = 1;
   *stride = 0;
   if (group.empty()) return true;
-  for (size_t i = 0; i < group.size(); ++i) {
-    const int64_t d = group[i];
-    if (i + 1 < group.size()) {
-      const int64_t nd = group[i + 1];
-      if (dims[nd] != 1 && dims[d] != 1 && strides[d] != strides[nd] * dims[nd]) return false;
-    }
-    *size *= dims[d];
-  }
-  // stride of the innermost non-unit dim of the group
   *stride = strides[group.back()];
-  for (auto it = group.rbegin(); it != group.rend(); ++it)
-    if (dims[*it] != 1) {
-      *stride = strides[*it];
-      break;
-    }
+  int64_t outer = -1;  // the non-unit dim before d: d follows it where d's extent is its stride
+  for (const int64_t d : group) {
+    *size *= dims[d];
+    if (dims[d] == 1) continue;
+    if (outer >= 0 && strides[outer] != strides[d] * dims[d]) return false;
+    outer = d;
+    *stride = strides[d];
+  }
   return true;
 }
 

@@ -85,6 +85,24 @@ def test_dimension_orders(client, sizes):
             _check(got, want, size["k"], "bf16", None)
 
 
+@pytest.mark.parametrize("lhs,rhs,out,contract", [
+    ("akum", "kn", "aumn", ((1,), (0,))),        # u: one element between two free dims that are apart
+    ("mk", "akun", "maun", ((1,), (1,))),
+    ("mkc", "knuc", "mnu", ((1, 2), (0, 3))),    # between two contracted ones
+    ("aumk", "kn", "aumn", ((3,), (0,))),        # between two that follow each other
+])
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_dims_of_one_element(client, lhs, rhs, out, contract, dt):
+    size = dict(a=2, c=6, k=40, m=12, n=24, u=1)
+    vals = [np.random.default_rng(i).integers(-3, 4, [size[c] for c in s]).astype(np.float32) for i, s in enumerate((lhs, rhs))]
+    b = Builder()
+    x, y = (b.param(v.shape, dt) for v in vals)
+    exe = client.compile(b.build([b.dot_general(x, y, contract=contract, out_dtype="f32")]))
+    (got,) = exe(*(to_bf16_bits(v) if dt == "bf16" else v for v in vals), dtypes=[dt] * 2)
+    # Whole numbers: every sum is exact in f32.
+    np.testing.assert_array_equal(got, np.einsum(f"{lhs},{rhs}->{out}", *vals))
+
+
 def test_same_bits_on_every_call(client):
     sizes = {"m": 100, "n": 520, "k": 4104}
     a, _ = _dot(client, "mk,kn", sizes)

@@ -484,3 +484,13 @@ def test_operands_are_read_within_their_bounds(plugin):
     assert _operands(plugin, (64, 1), (1, 23), ((1,), (0,))) == ["padded", "padded"]
     assert _operands(plugin, (64,), (23,), ((), ())) == ["padded", "padded"]
     assert _operands(plugin, (3, 64, 1), (3, 1, 24), ((2,), (1,)), ((0,), (0,))) == ["padded", "read"]
+
+
+def test_dims_of_one_element_do_not_merge_their_neighbours(plugin):
+    """Free (or contracted) dims are one stride only where the dims of more
+    than one element follow each other; one of 1 between them changes nothing."""
+    assert _operands(plugin, (2, 40, 1, 8), (40, 24), ((1,), (0,))) == ["copied", "read"]
+    assert _operands(plugin, (2, 40, 8), (40, 24), ((1,), (0,))) == ["copied", "read"]
+    assert _operands(plugin, (2, 1, 8, 40), (40, 24), ((3,), (0,))) == ["read", "read"]
+    assert _operands(plugin, (64, 2, 20), (2, 24, 1, 20), ((1, 2), (0, 3))) == ["read", "copied"]
+    assert _operands(plugin, (64, 1, 2, 20), (1, 2, 20, 24), ((1, 2, 3), (0, 1, 2))) == ["read", "read"]
