@@ -23,15 +23,16 @@ struct OperandView {
   bool ok = true;                  // groups mergeable into single strides
 };
 
-// Merges a group of dims (in the given order) into one (size, stride).
+// Merges a group of dims (in the given order) into one (size, stride). False
+// where the group has no one stride; the size is set all the same.
 bool merge(const Dims& dims, const int64_t* strides, const std::vector<int64_t>& group, int64_t* size, int64_t* stride) {
   *size = 1;
   *stride = 0;
   if (group.empty()) return true;
   *stride = strides[group.back()];
+  for (const int64_t d : group) *size *= dims[d];
   int64_t outer = -1;  // the non-unit dim before d: d follows it where d's extent is its stride
   for (const int64_t d : group) {
-    *size *= dims[d];
     if (dims[d] == 1) continue;
     if (outer >= 0 && strides[outer] != strides[d] * dims[d]) return false;
     outer = d;
@@ -51,8 +52,9 @@ OperandView view_of(const TensorType& t, const Dims& batch, const Dims& contract
   for (int d = 0; d < t.rank(); ++d)
     if (std::find(b.begin(), b.end(), d) == b.end() && std::find(c.begin(), c.end(), d) == c.end()) f.push_back(d);
   OperandView v;
-  v.ok = merge(t.dims, st, b, &v.batch, &v.bs) && merge(t.dims, st, f, &v.free, &v.fs) &&
-         merge(t.dims, st, c, &v.k, &v.ks);
+  const bool bo = merge(t.dims, st, b, &v.batch, &v.bs), fo = merge(t.dims, st, f, &v.free, &v.fs),
+             co = merge(t.dims, st, c, &v.k, &v.ks);
+  v.ok = bo && fo && co;
   return v;
 }
 

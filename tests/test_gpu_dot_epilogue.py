@@ -59,7 +59,7 @@ def test_added_row_and_residual(client, m, n, k, add, dt):
 # Right operands with no, two and three free dims; batched; contracted last.
 # 72 elements are summed in one launch of the block tiles, 8200 in k-splits.
 FREE_DIMS = [("mk", "k", "m"), ("mk", "kgh", "mgh"), ("mk", "ghk", "mgh"), ("km", "kgh", "mgh"), ("mk", "kfgh", "mfgh"),
-             ("amk", "kgh", "amgh"), ("bmk", "bk", "bm"), ("bmk", "bkgh", "bmgh"), ("bkm", "bghk", "bmgh")]
+             ("amk", "kgh", "amgh"), ("mk", "gkh", "mgh"), ("akm", "kgh", "amgh"), ("bmk", "bk", "bm"), ("bmk", "bkgh", "bmgh"), ("bkm", "bghk", "bmgh")]
 
 
 @pytest.mark.parametrize("k", [72, 8200])

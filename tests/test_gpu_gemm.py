@@ -90,9 +90,14 @@ def test_dimension_orders(client, sizes):
     ("mk", "akun", "maun", ((1,), (1,))),
     ("mkc", "knuc", "mnu", ((1, 2), (0, 3))),    # between two contracted ones
     ("aumk", "kn", "aumn", ((3,), (0,))),        # between two that follow each other
+    ("akm", "kn", "amn", ((1,), (0,))),          # free dims that are apart, contracted ones in another order
+    ("mk", "akn", "man", ((1,), (1,))),
+    ("akm", "nkc", "amnc", ((1,), (1,))),
+    ("mkc", "nck", "mn", ((1, 2), (2, 1))),
+    ("kcm", "nkc", "mn", ((1, 0), (2, 1))),
 ])
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
-def test_dims_of_one_element(client, lhs, rhs, out, contract, dt):
+def test_dims_that_do_not_merge(client, lhs, rhs, out, contract, dt):
     size = dict(a=2, c=6, k=40, m=12, n=24, u=1)
     vals = [np.random.default_rng(i).integers(-3, 4, [size[c] for c in s]).astype(np.float32) for i, s in enumerate((lhs, rhs))]
     b = Builder()

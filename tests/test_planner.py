@@ -434,6 +434,7 @@ def test_attention_writes_its_transposed_result(plugin):
     ((4096, 128), (128,), ((1,), (0,)), None, 1),                  # a vector: one column
     ((64, 128), (128, 2, 3, 4), ((1,), (0,)), None, 24),
     ((16, 4, 128), (128, 40), ((2,), (0,)), None, 40),             # rows of two dims
+    ((64, 128), (8, 128, 32), ((1,), (1,)), None, 256),            # columns that are apart
     ((64, 128), (128, 40), ((1,), (0,)), "row", 0),
 ])
 def test_merged_addend_rows_are_the_products(plugin, lhs, rhs, contract, add, stride):
