@@ -1216,8 +1216,13 @@ void Planner::shape_reduce(Step* s) {
     s->splits = 1;
     if (rank > 0 && nred > 0 && s->reduce_dims.back() != rank - 1 && rows > 0 && row_len >= 32) {
       size_t min_size = 8, slot = 0;
-      for (int v : s->inputs)
-        if (prog_.type(v).elements() == num_elements(shape)) min_size = std::min(min_size, dtype_size(prog_.type(v).dtype));
+      int64_t whole = 0, whole_bytes = 0;  // inputs of the reduced shape
+      for (int v : s->inputs) {
+        if (prog_.type(v).elements() != num_elements(shape)) continue;
+        min_size = std::min(min_size, dtype_size(prog_.type(v).dtype));
+        ++whole;
+        whole_bytes += prog_.type(v).bytes();
+      }
       for (const ReduceSpec& r : s->reduces) slot += (r.kind == ReducerKind::kArgMax || r.kind == ReducerKind::kArgMin) ? 16 : 8;
       int vec = std::max(1, std::min(8, static_cast<int>(16 / min_size)));
       while (vec > 1 && (shape[rank - 1] % vec != 0 || 256 * vec * slot > 48 * 1024)) vec /= 2;
@@ -1233,7 +1238,22 @@ void Planner::shape_reduce(Step* s) {
       int one = lanes;
       while (one > 8 && (blocks_of(one) < 256 || per_thread(one) > 32)) one /= 2;
       if (per_thread(one) <= 32) lanes = one;
-      if (256 * vec * slot <= 48 * 1024) {
+      // Rows of an odd number of elements are read one element a lane: 256
+      // lanes keep the pieces long ([1024, 40001] f32 111 -> 30 us, bf16 93 ->
+      // 22; below 256 elements 64 lanes are as fast).
+      if (vec == 1 && row_len >= 256 && blocks_of(256) >= 64) lanes = 256;
+      // From workgroups for seven of eight CUs on (57,344 outputs), one serial
+      // thread an output streams whole rows across the GPU. It is the better
+      // schedule for odd rows ([1024, 65537] f32 42 us against 176 with 64 lanes, 46
+      // with 256), for long columns of rows that are not whole 128-byte lines
+      // ([1024, 65540] f32 42 against 79), for three inputs and more, whose
+      // loads in flight cost the lanes' occupancy ([256, 65536] bf16 + 3 f32
+      // 33 against 41), and for many outputs of what the 256 MB memory-side
+      // cache holds ([64, 1048576] bf16 21 against 28).
+      const bool lines = shape[rank - 1] * static_cast<int64_t>(min_size) % 128 == 0;
+      const bool serial = (rows >= 57344 && row_len >= 64 && (vec == 1 || whole >= 3 || (row_len >= 256 && !lines))) ||
+                          (rows >= (1 << 19) && (vec == 1 || whole_bytes <= (int64_t(256) << 20)));
+      if (!serial && 256 * vec * slot <= 48 * 1024) {
         const int64_t blocks = blocks_of(lanes);
         int64_t splits = 1;
         if (per_thread(lanes) > 32)
@@ -1434,7 +1454,7 @@ std::string Plan::describe(const Program& prog) const {
       o << ",\"reducers\":[";
       for (size_t k = 0; k < s.reduces.size(); ++k) o << (k ? "," : "") << "\"" << reducer_name(s.reduces[k].kind) << "\"";
       o << "],\"row_schedule\":" << (s.row_schedule ? "true" : "false") << ",\"rows\":" << s.rows
-        << ",\"row_len\":" << s.row_len << ",\"splits\":" << s.splits << ",\"chunk\":" << s.chunk
+        << ",\"row_len\":" << s.row_len << ",\"column_lanes\":" << s.col_lanes << ",\"splits\":" << s.splits << ",\"chunk\":" << s.chunk
         << ",\"fused_combine\":" << (s.fused_combine ? "true" : "false");
     }
     if (s.kind == StepKind::kLibrary) {

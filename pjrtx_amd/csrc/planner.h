@@ -112,7 +112,7 @@ struct Step {
   Dims reduce_dims;          // sorted
   bool row_schedule = true;  // reduced dims are the trailing dims
   // Column schedule with the last dim kept: lanes of a workgroup that span
-  // outputs (each `vec` of them); 0 keeps one serial thread per output.
+  // outputs (each `vec` of them); 0: one serial thread per output.
   int col_lanes = 0;
   int64_t rows = 1;          // row schedule: product of kept dims
   int64_t row_len = 1;       // row schedule: product of reduced dims

@@ -495,3 +495,23 @@ def test_dims_of_one_element_do_not_merge_their_neighbours(plugin):
     assert _operands(plugin, (2, 1, 8, 40), (40, 24), ((3,), (0,))) == ["read", "read"]
     assert _operands(plugin, (64, 2, 20), (2, 24, 1, 20), ((1, 2), (0, 3))) == ["read", "copied"]
     assert _operands(plugin, (64, 1, 2, 20), (1, 2, 20, 24), ((1, 2, 3), (0, 1, 2))) == ["read", "read"]
+
+
+@pytest.mark.parametrize("shape,inputs,lanes", [
+    ((1024, 4096), ["f32"], "64"), ((256, 65536), ["f32"], "64"), ((64, 1 << 22), ["f32"], "64"),
+    ((64, 1 << 20), ["bf16"], 0),              # what the memory-side cache holds
+    ((1024, 65540), ["f32"], 0), ((1024, 65537), ["bf16"], 0), ((32, 65537), ["f32"], "64"),
+    ((256, 65536), ["bf16", "f32", "f32"], 0), ((256, 40960), ["bf16", "f32", "f32"], "64"),
+    ((1024, 40001), ["f32"], 256), ((1024, 9001), ["f32"], "64"), ((100, 40001), ["f32"], "64"),
+])
+def test_schedule_of_column_reductions(plugin, shape, inputs, lanes):
+    """Lanes that span outputs, or one serial thread an output where that
+    streams whole rows better."""
+    b = Builder()
+    x = [b.param(shape, dt) for dt in inputs]
+    total = b.convert(x[0], "f32") if inputs[0] != "f32" else x[0]
+    for y in x[1:]:
+        total = b.add(total, y)
+    (step,) = plan(plugin, b.build([b.sum(total, [0])]))["steps"]
+    assert not step["row_schedule"]
+    assert 8 <= step["column_lanes"] <= 64 if lanes == "64" else step["column_lanes"] == lanes
