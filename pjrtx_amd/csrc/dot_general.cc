@@ -327,6 +327,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
   f.b_bs = b.bs;
   f.b_ns = b.fs;
   f.b_ks = b.ks;
+  f.row_lanes = op.dot_swapped;
   launch_fma_gemm(dev->stream(), f, A, B, out, lt.dtype, ot.dtype);
   return false;
 }
@@ -513,6 +514,7 @@ bool fold_dot_transpose(Program* prog) {
     std::swap(r.lhs_batch, r.rhs_batch);
     std::swap(r.lhs_contract, r.rhs_contract);
     r.results = t.results;
+    r.dot_swapped = !d.dot_swapped;
     t = std::move(r);
     changed = true;
   }

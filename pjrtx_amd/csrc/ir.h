@@ -127,6 +127,9 @@ struct Op {
   // fold_gather_index_wrap. 0: indices are read as they are.
   int64_t index_wrap = 0;
 
+  // dot_general: its operands changed sides, to write a product transposed.
+  bool dot_swapped = false;
+
   // sort: results that are the sorted positions (their operand was an iota
   // along the sorted dim, and is not in `operands`).
   Dims iota_results;

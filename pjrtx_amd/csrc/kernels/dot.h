@@ -127,6 +127,7 @@ struct FmaGemmParams {
   int64_t batch = 1, M = 0, N = 0, K = 0;
   int64_t a_bs = 0, a_ms = 0, a_ks = 0;
   int64_t b_bs = 0, b_ns = 0, b_ks = 0;
+  bool row_lanes = false;  // lanes along C's rows (M) instead of its columns
 };
 void launch_fma_gemm(hipStream_t s, const FmaGemmParams& p, const void* A, const void* B, void* C, DType in, DType out);
 

@@ -492,15 +492,34 @@ __global__ void __launch_bounds__(256) gemv_k(GemvParams p, const uint16_t* __re
 }
 
 // --------------------------------------------------------------- fallback
+// The thread's element of C, at index i. Lanes follow C's columns, or with
+// `row_lanes` its rows: a product written transposed (its operands changed
+// sides for that) reads both as the product itself does, whose lanes share a
+// row of A and read neighbouring columns of B, and its stores are strided
+// instead, one to K loads. f32 [1000, 512] x [512, 2048], transposed: 3723 us
+// with lanes over C's columns, 363 as a product and a copy, 239 so.
+__device__ __forceinline__ bool fma_output(const FmaGemmParams& p, int64_t& b, int64_t& m, int64_t& n, int64_t& i) {
+  i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t each = (int64_t)p.M * p.N;
+  if (i >= p.batch * each) return false;
+  b = i / each;
+  const int64_t r = i - b * each;
+  if (p.row_lanes) {
+    n = r / p.M;
+    m = r - n * p.M;
+    i = b * each + m * p.N + n;
+  } else {
+    m = r / p.N;
+    n = r - m * p.N;
+  }
+  return true;
+}
+
 template <typename T, typename Acc>
 __global__ void __launch_bounds__(256) fma_gemm(FmaGemmParams p, const T* __restrict__ A, const T* __restrict__ B,
                                                 T* __restrict__ C) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t total = (int64_t)p.batch * p.M * p.N;
-  if (i >= total) return;
-  const int64_t b = i / ((int64_t)p.M * p.N);
-  const int64_t r = i - b * p.M * p.N;
-  const int64_t m = r / p.N, n = r - m * p.N;
+  int64_t b, m, n, i;
+  if (!fma_output(p, b, m, n, i)) return;
   Acc s = 0;
   const T* a = A + b * p.a_bs + m * p.a_ms;
   const T* bb = B + b * p.b_bs + n * p.b_ns;
@@ -512,12 +531,8 @@ __global__ void __launch_bounds__(256) fma_gemm(FmaGemmParams p, const T* __rest
 __global__ void __launch_bounds__(256) fma_gemm_16(FmaGemmParams p, const uint16_t* __restrict__ A,
                                                    const uint16_t* __restrict__ B, void* __restrict__ C, int in_f16,
                                                    int out_kind) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t total = (int64_t)p.batch * p.M * p.N;
-  if (i >= total) return;
-  const int64_t b = i / ((int64_t)p.M * p.N);
-  const int64_t r = i - b * p.M * p.N;
-  const int64_t m = r / p.N, n = r - m * p.N;
+  int64_t b, m, n, i;
+  if (!fma_output(p, b, m, n, i)) return;
   float s = 0.f;
   const uint16_t* a = A + b * p.a_bs + m * p.a_ms;
   const uint16_t* bb = B + b * p.b_bs + n * p.b_ns;

@@ -133,3 +133,18 @@ def test_transposed_result(client, batch, lhs, rhs, dt):
         # sigma, and a partial sum of N(0,1) products stays under 5 sqrt(k).
         tol = 20 * k * 2.0 ** -24 if dt == "f32" else ULP[dt] * np.abs(want) + 4e-6 * k ** 0.5
         assert (np.abs(got - want) <= tol).all()
+
+
+@pytest.mark.parametrize("batch,lhs,rhs", [("", "mk", "kn"), ("", "km", "nk"), ("b", "bmk", "bkn")])
+@pytest.mark.parametrize("dt", ["s32", "f32", "f64"])
+def test_transposed_result_of_whole_numbers(client, batch, lhs, rhs, dt):
+    """The types of the scalar kernel, whose lanes then follow the result's rows."""
+    for m, n, k in ((9, 300, 5), (257, 9, 70), (64, 64, 64)):
+        size = dict(b=3, m=m, n=n, k=k)
+        vals = [np.random.default_rng(i).integers(-9, 10, [size[c] for c in s]) for i, s in enumerate((lhs, rhs))]
+        vals = [v.astype({"s32": np.int32, "f32": np.float32, "f64": np.float64}[dt]) for v in vals]
+        b = Builder()
+        x, y = (b.param(v.shape, dt) for v in vals)
+        d = b.dot_general(x, y, batch=((0,), (0,)) if batch else ((), ()), contract=((lhs.index("k"),), (rhs.index("k"),)))
+        (got,) = client.compile(b.build([b.transpose(d, [0, 2, 1] if batch else [1, 0])]))(*vals, dtypes=[dt] * 2)
+        np.testing.assert_array_equal(got, np.einsum(f"{lhs},{rhs}->{batch}nm", *vals))
