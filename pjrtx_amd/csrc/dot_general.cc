@@ -197,7 +197,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
     const auto aligned_rows = [&](const void* p, const OperandView& v, bool kc) { return aligned16(p) && whole_rows(v, kc); };
     const auto pad = [&](const void** p, OperandView* v, bool kc, MemRef* mem) {
       const int64_t rows = kc ? v->free : v->k, cols = kc ? v->k : v->free, ldp = (cols + 7) / 8 * 8;
-      if (batch >= 65536 || rows * (ldp / 8) >= (int64_t(1) << 38) || !fits(batch * rows * ldp * 2)) return false;
+      if (rows * (ldp / 8) >= (int64_t(1) << 38) || !fits(batch * rows * ldp * 2)) return false;
       *mem = dev->allocate(static_cast<size_t>(batch * rows * ldp) * 2);
       const int64_t rs = kc ? (v->fs ? v->fs : cols) : (v->ks ? v->ks : cols);
       launch_pad_rows16(dev->stream(), *p, (*mem)->ptr, batch, v->bs, rows, rs, cols, ldp);

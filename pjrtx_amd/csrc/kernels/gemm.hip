@@ -803,9 +803,12 @@ void launch_pad_rows16(hipStream_t s, const void* in, void* out, int64_t batch, 
                        int64_t cols, int64_t ldp) {
   if (batch == 0 || rows == 0 || ldp == 0) return;
   const int64_t blocks = (rows * (ldp / 8) + 255) / 256;
-  PJRTX_CHECK(batch < 65536 && blocks < (int64_t(1) << 31), Code::kInternal, "pad_rows16: grid too large");
-  hipLaunchKernelGGL(pad_rows16, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(batch)), dim3(256), 0, s,
-                     static_cast<const uint16_t*>(in), static_cast<uint16_t*>(out), bs, rows, rs, cols, ldp);
+  PJRTX_CHECK(blocks < (int64_t(1) << 31), Code::kInternal, "pad_rows16: grid too large");
+  constexpr int64_t kMost = 65535;  // batches a launch's grid holds
+  for (int64_t b = 0; b < batch; b += kMost)
+    hipLaunchKernelGGL(pad_rows16, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(std::min(kMost, batch - b))),
+                       dim3(256), 0, s, static_cast<const uint16_t*>(in) + b * bs,
+                       static_cast<uint16_t*>(out) + b * rows * ldp, bs, rows, rs, cols, ldp);
   check("pad_rows16");
 }
 

@@ -108,6 +108,18 @@ def test_dims_that_do_not_merge(client, lhs, rhs, out, contract, dt):
     np.testing.assert_array_equal(got, np.einsum(f"{lhs},{rhs}->{out}", *vals))
 
 
+def test_ragged_rows_of_many_batches(client):
+    """More batches than a launch's grid holds of padded rows."""
+    b, m, k, n = 65541, 9, 16, 12
+    rng = np.random.default_rng(1)
+    x, y = (rng.integers(-3, 4, s).astype(np.float32) for s in ((b, m, k), (b, k, n)))
+    h = Builder()
+    d = h.dot_general(h.param(x.shape, "bf16"), h.param(y.shape, "bf16"), batch=((0,), (0,)), contract=((2,), (1,)),
+                      out_dtype="f32")
+    (got,) = client.compile(h.build([d]))(to_bf16_bits(x), to_bf16_bits(y), dtypes=["bf16"] * 2)
+    np.testing.assert_array_equal(got, np.matmul(x, y))
+
+
 def test_same_bits_on_every_call(client):
     sizes = {"m": 100, "n": 520, "k": 4104}
     a, _ = _dot(client, "mk,kn", sizes)
