@@ -79,6 +79,35 @@ bool whole_rows(const OperandView& v, bool kmajor) {
   return (rows == 1 || ld % 8 == 0) && (v.batch == 1 || v.bs % 8 == 0) && (cols % 8 == 0 || (!kmajor && rows > 1));
 }
 
+int64_t round8(int64_t n) { return (n + 7) / 8 * 8; }
+
+GemmParams gemm_params(const OperandView& a, const OperandView& b, const DotLayout& l) {
+  GemmParams g;
+  g.batch = static_cast<int>(a.batch);
+  g.M = static_cast<int>(a.free);
+  g.N = static_cast<int>(b.free);
+  g.K = static_cast<int>(a.k);
+  // One row only: its stride is not used; a multiple of 8.
+  g.lda = l.a_kmajor ? (a.free == 1 ? round8(a.k) : a.fs) : (a.k == 1 ? round8(a.free) : a.ks);
+  g.ldb = l.b_kmajor ? (b.free == 1 ? round8(b.k) : b.fs) : (b.k == 1 ? round8(b.free) : b.ks);
+  g.ldc = b.free;
+  g.a_batch_stride = a.batch == 1 ? 0 : a.bs;
+  g.b_batch_stride = a.batch == 1 ? 0 : b.bs;
+  return g;
+}
+GemmGroup gemm_group(const GemmParams& g) {
+  GemmGroup gg;
+  gg.batch = g.batch;
+  gg.M = g.M;
+  gg.K = g.K;
+  gg.lda = g.lda;
+  gg.a_batch_stride = g.a_batch_stride;
+  gg.m[0].N = g.N;
+  gg.m[0].ldb = g.ldb;
+  gg.m[0].b_batch_stride = g.b_batch_stride;
+  return gg;
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 // Copies `t` into a canonical [batch][free][k] (or [batch][k][free] when
@@ -136,13 +165,26 @@ int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row) {
 }
 
 std::string describe_dot(const Program& prog, const Op& dot) {
-  const OperandView a = view_of(prog.type(dot.operands[0]), dot.lhs_batch, dot.lhs_contract);
-  const OperandView b = view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract);
+  OperandView a = view_of(prog.type(dot.operands[0]), dot.lhs_batch, dot.lhs_contract);
+  OperandView b = view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract);
+  const bool a_copied = !a.ok, b_copied = !b.ok;
+  for (OperandView* v : {&a, &b})
+    if (!v->ok) *v = OperandView{v->batch, v->free, v->k, v->free * v->k, v->k, 1, true};
   const DotLayout l = layout_of(a, b);
-  const auto one = [](const OperandView& v, bool kmajor) {
-    return !v.ok ? "\"copied\"" : !whole_rows(v, kmajor) ? "\"padded\"" : "\"read\"";
+  const auto one = [](bool copied, const OperandView& v, bool kmajor) {
+    return copied ? "\"copied\"" : !whole_rows(v, kmajor) ? "\"padded\"" : "\"read\"";
   };
-  return std::string("[") + one(a, l.a_kmajor) + "," + one(b, l.b_kmajor) + "]";
+  // With the strides padding gives.
+  const auto taken = [](OperandView v, bool kmajor) {
+    if (!whole_rows(v, kmajor)) {
+      const int64_t rows = kmajor ? v.free : v.k, ld = round8(kmajor ? v.k : v.free);
+      v = OperandView{v.batch, v.free, v.k, rows * ld, kmajor ? ld : 1, kmajor ? 1 : ld, true};
+    }
+    return v;
+  };
+  const bool tiles = gemm_fits(gemm_group(gemm_params(taken(a, l.a_kmajor), taken(b, l.b_kmajor), l)), l.a_kmajor, l.b_kmajor);
+  return std::string("\"operands\":[") + one(a_copied, a, l.a_kmajor) + "," + one(b_copied, b, l.b_kmajor) +
+         "],\"block_tiles\":" + (tiles ? "true" : "false");
 }
 
 // Writes the product to the dot's result, plus `add` (GemmMember::add, its
@@ -196,7 +238,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
     }
     const auto aligned_rows = [&](const void* p, const OperandView& v, bool kc) { return aligned16(p) && whole_rows(v, kc); };
     const auto pad = [&](const void** p, OperandView* v, bool kc, MemRef* mem) {
-      const int64_t rows = kc ? v->free : v->k, cols = kc ? v->k : v->free, ldp = (cols + 7) / 8 * 8;
+      const int64_t rows = kc ? v->free : v->k, cols = kc ? v->k : v->free, ldp = round8(cols);
       if (rows * (ldp / 8) >= (int64_t(1) << 38) || !fits(batch * rows * ldp * 2)) return false;
       *mem = dev->allocate(static_cast<size_t>(batch * rows * ldp) * 2);
       const int64_t rs = kc ? (v->fs ? v->fs : cols) : (v->ks ? v->ks : cols);
@@ -258,32 +300,13 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
     if (ready && !aligned_rows(A, a, a_kmajor)) ready = pad(&A, &a, a_kmajor, &a_pad);
     if (ready && !aligned_rows(B, b, b_kmajor)) ready = pad(&B, &b, b_kmajor, &b_pad);
     if (ready) {
-      GemmParams g;
-      g.batch = static_cast<int>(batch);
-      g.M = static_cast<int>(M);
-      g.N = static_cast<int>(N);
-      g.K = static_cast<int>(K);
-      const auto round8 = [](int64_t n) { return (n + 7) / 8 * 8; };
-      // One row only: its stride is not used; a multiple of 8.
-      g.lda = a_kmajor ? (M == 1 ? round8(K) : a.fs) : (K == 1 ? round8(M) : a.ks);
-      g.ldb = b_kmajor ? (N == 1 ? round8(K) : b.fs) : (K == 1 ? round8(N) : b.ks);
-      g.ldc = N;
-      g.a_batch_stride = batch == 1 ? 0 : a.bs;
-      g.b_batch_stride = batch == 1 ? 0 : b.bs;
+      const GemmParams g = gemm_params(a, b, lay);
       if (a_kmajor && K % 8 == 0 && (b_kmajor || N % 8 == 0) && blaslt_wanted(g) &&
           blaslt_gemm(dev, g, A, B, out, f16, b_kmajor, out_kind == 2 ? 4 : 2))
         return false;
-      GemmGroup gg;
-      gg.batch = g.batch;
-      gg.M = g.M;
-      gg.K = g.K;
-      gg.lda = g.lda;
-      gg.a_batch_stride = g.a_batch_stride;
+      GemmGroup gg = gemm_group(g);
       gg.m[0].B = B;
       gg.m[0].C = out;
-      gg.m[0].N = g.N;
-      gg.m[0].ldb = g.ldb;
-      gg.m[0].b_batch_stride = g.b_batch_stride;
       const bool fuse = add && out_kind != 2 && aligned16(add) && aligned16(out);
       if (fuse) gg.m[0].add = add;
       gg.m[0].add_ld = add_ld;

@@ -703,7 +703,8 @@ bool gemm_fits(const GemmGroup& g, bool a_kmajor, bool b_kmajor) {
               ok(g.lda, g.a_batch_stride, a_kmajor, a_kmajor ? g.K : g.M);
   for (int i = 0; i < g.count && fits; ++i)
     fits = g.m[i].N > 0 && ok(g.m[i].ldb, g.m[i].b_batch_stride, b_kmajor, b_kmajor ? g.K : g.m[i].N);
-  return fits && tiles_of(g, kTiles[kGemmTiles - 1]) < (int64_t(1) << 24);
+  // Workgroups (splits only of few tiles) and their ids stay below 2^31.
+  return fits && tiles_of(g, kTiles[kGemmTiles - 1]) < (int64_t(1) << 30);
 }
 
 GemmPlan plan_gemm(const GemmGroup& g, int64_t max_workspace) {

@@ -259,8 +259,9 @@ bool fold_sort_iota(Program* prog);
 bool fold_dot_transpose(Program* prog);
 // Elements from one row of a merged addend to the next (dot_general.cc).
 int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row);
-// How the block tiles take each operand of a product of 16-byte aligned
-// buffers: "read" in place, "padded" or "copied" (dot_general.cc).
+// JSON members: how the block tiles take each operand of a product of 16-byte
+// aligned buffers ("read" in place, "padded" or "copied"), and whether its
+// sizes are within theirs (dot_general.cc).
 std::string describe_dot(const Program& prog, const Op& dot);
 
 // Turns decode-shaped dot and dot-group library steps into kGemv steps and

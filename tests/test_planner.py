@@ -487,6 +487,19 @@ def test_operands_are_read_within_their_bounds(plugin):
     assert _operands(plugin, (3, 64, 1), (3, 1, 24), ((2,), (1,)), ((0,), (0,))) == ["padded", "read"]
 
 
+@pytest.mark.parametrize("lhs,rhs,contract,tiles", [
+    ((1 << 20, 64), (64, 1 << 15), ((1,), (0,)), True),        # a 64 GB result: 2^24 of the smallest tiles
+    ((64, 1 << 22), ((1 << 22), 64), ((1,), (0,)), False),     # rows of 4M elements
+    ((64, (1 << 22) - 8), ((1 << 22) - 8, 64), ((1,), (0,)), True),
+    ((1 << 22, 64), (1 << 22, 64), ((0,), (0,)), True),        # contracted over long columns
+])
+def test_sizes_of_the_block_tiles(plugin, lhs, rhs, contract, tiles):
+    b = Builder()
+    d = b.dot_general(b.param(lhs, "bf16"), b.param(rhs, "bf16"), contract=contract)
+    (step,) = plan(plugin, b.build([d]))["steps"]
+    assert step["block_tiles"] is tiles
+
+
 def test_dims_of_one_element_do_not_merge_their_neighbours(plugin):
     """Free (or contracted) dims are one stride only where the dims of more
     than one element follow each other; one of 1 between them changes nothing."""
