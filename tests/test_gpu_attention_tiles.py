@@ -47,6 +47,16 @@ def test_workgroup_shapes(client, dt, d, sizes):
         np.testing.assert_array_equal(np.asarray(out)[:, 0], np.repeat(np.asarray(v)[:, 0], hq // hkv, axis=1))
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sizes", [(1, 17, 1, 17, 1, 0), (2, 64, 3, 700, 3, 636), (4, 330, 15, 470, 5, 139), (1, 256, 8, 256, 8, 0)])
+def test_register_staged_tiles(client, dt, d, sizes, monkeypatch):
+    """attn_tiles, which takes heads whose keys or values span 2 GiB."""
+    monkeypatch.setenv("PJRTX_ATTN_PIPE", "0")
+    got, want, _, _ = _run(client, dt, d, sizes)
+    assert_close16(got, want)
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("sizes", [(1, 40, 2, 150, 1, -3), (4, 300, 16, 300, 4, -1), (8, 140, 48, 140, 48, -2)])
 def test_queries_with_no_allowed_key(client, d, sizes):

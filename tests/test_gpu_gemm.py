@@ -120,6 +120,24 @@ def test_ragged_rows_of_many_batches(client):
     np.testing.assert_array_equal(got, np.matmul(x, y))
 
 
+@pytest.mark.parametrize("spec,dt,out_dt", [("mk,kn", "bf16", "f32"), ("mk,nk", "bf16", "f32"), ("mk,kn", "f16", "f32"),
+                                            ("mk,nk", "f16", "f32"), ("mk,nk", "bf16", "bf16"), ("mk,kn", "bf16", "bf16")])
+def test_rows_of_four_million_elements(client, spec, dt, out_dt):
+    """Rows past the block tiles' 32-bit offsets go to mfma_gemm; a ragged
+    last k-tile. Whole numbers whose partial sums (a random walk, deviation
+    8,200) stay far below 2^24: every f32 sum is exact."""
+    m, n, k = 9, 16, (1 << 22) + 72
+    rng = np.random.default_rng(5)
+    x, y = (rng.integers(-2, 3, s).astype(np.float32) for s in ((m, k), (k, n) if spec == "mk,kn" else (n, k)))
+    b = Builder()
+    contract = ((1,), (0,) if spec == "mk,kn" else (1,))
+    dot = b.dot_general(b.param(x.shape, dt), b.param(y.shape, dt), contract=contract, out_dtype=out_dt)
+    store = to_bf16_bits if dt == "bf16" else (lambda v: v.astype(np.float16))
+    (got,) = client.compile(b.build([dot]))(store(x), store(y), dtypes=[dt] * 2)
+    want = x @ (y if spec == "mk,kn" else y.T)
+    np.testing.assert_array_equal(got, want if out_dt == "f32" else to_bf16_bits(want))
+
+
 def test_same_bits_on_every_call(client):
     sizes = {"m": 100, "n": 520, "k": 4104}
     a, _ = _dot(client, "mk,kn", sizes)
