@@ -33,15 +33,16 @@
 //    waves share a sub-tile each takes 4 / WK of the slabs, which divides the
 //    fragment reads, and the sums meet through LDS once at the end.
 //
-// Measured on MI355X, bf16, B N-contiguous (before: one 256 x 256 kernel whose
-// loads were waited for a tile early, and 128 x 128 tiles transposed through
-// 2-byte LDS stores):
-//   8192 x 8192 x 8192    256 x 256 tiles   914 -> 808 us (1360 TFLOP/s)
-//   1000 x 2048 x 5632    128 x 256         104 -> 31 us
-//   512 x 2048 x 5632     128 x 128          99 -> 19 us
-//   512 x 5632 x 2048     64 x 64           233 -> 23 us
-//   512 x 2048 x 2048     64 x 64            93 -> 11.4 us
-//   64 x 4096 x 4096      64 x 64, k-split  171 -> 13 us
+// Measured on MI355X, bf16, B N-contiguous, executes back to back on the same
+// operands (before: one 256 x 256 kernel whose loads were waited for a tile
+// early, and 128 x 128 tiles transposed through 2-byte LDS stores); operands
+// that change from call to call come from HBM and take up to 8 us more:
+//   8192 x 8192 x 8192    256 x 256 tiles   887 -> 807 us (807-846 with the clock; 1300-1360 TFLOP/s)
+//   1000 x 2048 x 5632    128 x 256         148 -> 37 us
+//   512 x 2048 x 5632     128 x 128          98 -> 23 us
+//   512 x 5632 x 2048     64 x 64           233 -> 25 us
+//   512 x 2048 x 2048     64 x 64            91 -> 12.4 us
+//   64 x 4096 x 4096      64 x 64, k-split  170 -> 13 us
 // What bounds it: the large tile, power (the clock drops to about 1.6 GHz)
 // and LDS reads; the small ones, the loads (a 64 x 64 k-tile brings 16 KB per
 // CU, 0.157 us alone, against 0.073 us of matrix work) and the issue slots of

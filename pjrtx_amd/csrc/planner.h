@@ -120,7 +120,7 @@ struct Step {
   int64_t chunk = 0;         // elements per split
   int unroll = 1;            // 256*vec-element sub-chunks loaded together per thread
   size_t scratch_bytes = 0;  // partial accumulators (splits > 1)
-  uint32_t combine_grid = 0; // splits > 1: workgroups of `<name>_combine` (4 rows each)
+  uint32_t combine_grid = 0; // splits > 1: workgroups of `<name>_combine` (a wave per row: 4 rows; col_lanes: 256 rows)
   // splits > 1 and no combine launch: the last workgroup of a row to finish
   // folds the row's partials (per-row arrival counters after the slots).
   bool fused_combine = false;

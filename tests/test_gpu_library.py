@@ -438,7 +438,7 @@ def test_dot_f32_fallback_and_rank3_rank2(client):
 
 def test_matmul_8192_sampled_rows(client):
     """C3d at full size on the default route, the hand-written MFMA kernel
-    (gemm_nt_256, B read N-contiguous); sampled rows against float64, both
+    (gemm_tile, B read N-contiguous); sampled rows against float64, both
     ends and tile boundaries."""
     n = 8192
     rng = np.random.default_rng(9)
