@@ -547,7 +547,7 @@ struct TopkPass {
   SortGather g;
 };
 struct TopkLds {
-  double least[kTopkThreads];
+  double least[2 * kTopkThreads];
   double bound;
   uint32_t bound_image;
   int count;
@@ -589,25 +589,49 @@ __device__ __forceinline__ void topk_rank(const TopkPass& p, int64_t row, int64_
 
 // The words at or below T of 256 threads' kShare * 8 words each: T is the
 // need-th smallest of the threads' own least words, so at most need * 8 *
-// kShare words go to `cand`. Returns how many.
+// kShare words go to `cand`. Returns how many. Where `need` is most of the
+// threads, the least of each half of a thread's words are taken: the 256th of
+// 256 is the largest of them, with many words below it ([64, 8192] f32, k =
+// 256: 105 us, 27 with halves). The longer count costs 5 us a round: at 200 of
+// 256 it is the slower one ([17, 54716] 32 and 40).
 template <int kShare>
 __device__ __forceinline__ int topk_bound(const double (&w)[kShare][kGroup], int need, int tid, TopkLds& lds, double* cand) {
   const double end = as_word(kWordEnd);
-  double lo = end;
+  double half[2] = {end, end};
 #pragma unroll
   for (int q = 0; q < kShare; ++q)
 #pragma unroll
-    for (int e = 0; e < kGroup; ++e) asm("v_min_f64 %0, %0, %1" : "+v"(lo) : "v"(w[q][e]));
-  lds.least[tid] = lo;
+    for (int e = 0; e < kGroup; ++e) asm("v_min_f64 %0, %0, %1" : "+v"(half[e & 1]) : "v"(w[q][e]));
+  const double lo = half[0] < half[1] ? half[0] : half[1];
+  const bool halves = need > kTopkThreads * 7 / 8;
+  if (halves) {
+    lds.least[2 * tid] = half[0];
+    lds.least[2 * tid + 1] = half[1];
+  } else {
+    lds.least[tid] = lo;
+  }
   if (tid == 0) {
-    lds.bound = as_word(kWordEnd - 1);  // fewer than `need` threads hold words: all of them
+    lds.bound = as_word(kWordEnd - 1);  // fewer than `need` of them hold words: all words
     lds.count = 0;
   }
   __syncthreads();
-  int rank = 0;
+  if (halves) {
+    int rank[2] = {0, 0};
 #pragma unroll 8
-  for (int i = 0; i < kTopkThreads; ++i) rank += lds.least[i] < lo ? 1 : 0;
-  if (rank == need - 1 && lo < end) lds.bound = lo;
+    for (int i = 0; i < 2 * kTopkThreads; ++i) {
+      const double x = lds.least[i];
+      rank[0] += x < half[0] ? 1 : 0;
+      rank[1] += x < half[1] ? 1 : 0;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (rank[h] == need - 1 && half[h] < end) lds.bound = half[h];
+  } else {
+    int rank = 0;
+#pragma unroll 8
+    for (int i = 0; i < kTopkThreads; ++i) rank += lds.least[i] < lo ? 1 : 0;
+    if (rank == need - 1 && lo < end) lds.bound = lo;
+  }
   __syncthreads();
   const double T = lds.bound;
   if (lo <= T) {
@@ -621,6 +645,29 @@ __device__ __forceinline__ int topk_bound(const double (&w)[kShare][kGroup], int
   return lds.count;
 }
 
+// The candidates again where they are many: m words in `cand`. Rows and lists
+// in some order can give every thread words of like rank (lists of 256 words
+// put word k of each in thread k: T is then near the last of them all, and
+// ranking by counting is quadratic). A thread takes words a golden ratio of the
+// list apart, which are of many ranks in any such order.
+template <int kShare>
+__device__ __forceinline__ int topk_again(int m, int need, int tid, TopkLds& lds, double* cand) {
+  if (m <= 2 * need + kTopkThreads / 2) return m;
+  int bits = 8;
+  while ((1 << bits) < m) ++bits;  // m <= 256 * 8 * kShare
+  const uint32_t each = 1u << (bits - 8), step = (0x9e3779b1u >> (32 - bits)) | 1u, mask = (1u << bits) - 1u;
+  double w[kShare][kGroup];
+#pragma unroll
+  for (int q = 0; q < kShare; ++q)
+#pragma unroll
+    for (int e = 0; e < kGroup; ++e) {
+      const uint32_t j = q * kGroup + e, c = ((tid * each + j) * step) & mask;
+      w[q][e] = j < each && (int)c < m ? cand[c] : as_word(kWordEnd);
+    }
+  __syncthreads();
+  return topk_bound<kShare>(w, need, tid, lds, cand);
+}
+
 // Any source.
 template <int kShare>
 __device__ __forceinline__ int topk_words(const TopkPass& p, int64_t row, int64_t blk, int tid, TopkLds& lds, double* cand) {
@@ -628,7 +675,7 @@ __device__ __forceinline__ int topk_words(const TopkPass& p, int64_t row, int64_
 #pragma unroll
   for (int q = 0; q < kShare; ++q)
     load_words(p.src, p.r, row, (blk * kShare + q) * (kTopkThreads * kGroup), tid, kTopkThreads, w[q]);
-  return topk_bound<kShare>(w, p.need, tid, lds, cand);
+  return topk_again<kShare>(topk_bound<kShare>(w, p.need, tid, lds, cand), p.need, tid, lds, cand);
 }
 
 template <int kShare>
@@ -735,18 +782,7 @@ __global__ void __launch_bounds__(kTopkThreads) topk_half_kernel(TopkPass p) {
       cand[c] = make_word(key_image(from[at], map), base + at);
     }
     __syncthreads();
-    if (m > 2 * p.need + kTopkThreads / 2) {
-      double w[kShare][kGroup];
-#pragma unroll
-      for (int q = 0; q < kShare; ++q)
-#pragma unroll
-        for (int e = 0; e < kGroup; ++e) {
-          const int c = (q * kGroup + e) * kTopkThreads + tid;  // room <= 256 * 8 * kShare
-          w[q][e] = c < m ? cand[c] : as_word(kWordEnd);
-        }
-      __syncthreads();
-      m = topk_bound<kShare>(w, p.need, tid, lds, cand);
-    }
+    m = topk_again<kShare>(m, p.need, tid, lds, cand);
   }
   topk_rank(p, row, blk, tid, m, cand);
 }

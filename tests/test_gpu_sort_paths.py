@@ -66,7 +66,7 @@ def test_argsort_other_dims(client, shape, dim):
 
 @pytest.mark.parametrize("rows,n,k", [(1, 300, 256), (3, 2048, 1), (3, 2049, 256), (64, 8192, 50), (5, 8193, 50),
                                       (2, 100000, 256), (1, 1000000, 200), (3, 9000, 257), (3, 50000, 4096),
-                                      (3, 50000, 4097), (300, 2050, 5)])
+                                      (3, 50000, 4097), (300, 2050, 5), (3, 8192, 256), (7, 5000, 200)])
 @pytest.mark.parametrize("distinct", [0, 2, 40])
 def test_top_k_edges(client, rows, n, k, distinct):
     """Chunks of one, two and four groups a thread, one to three rounds, and
@@ -81,6 +81,31 @@ def test_top_k_edges(client, rows, n, k, distinct):
         wv, wi = S.top_k(x, k, bf16=dt == "bf16")
         _same(idx, wi)
         _same(vals, wv)
+
+
+@pytest.mark.parametrize("order", ["random", "ascending", "descending", "equal"])
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_top_k_as_many_as_threads(client, dt, order):
+    """k = 256, where the threads' least words bound little and sorted lists
+    give every thread words of like rank: the results, and that few words are
+    ranked (by counting, quadratic: 18 times k = 50's time and more when every
+    word was; at most 5 times since)."""
+    def run(rows, n, k):
+        x = np.random.default_rng(n).standard_normal((rows, n)).astype(np.float32)
+        x = {"random": x, "ascending": np.sort(x, 1), "descending": -np.sort(x, 1), "equal": np.ones_like(x)}[order]
+        x = to_bf16_bits(x) if dt == "bf16" else x
+        b = Builder("jit_topk")
+        exe = client.compile(b.build(list(b.top_k(b.param(x.shape, dt), k))))
+        args = [client.buffer(x, dt)]
+        vals, idx = (o.to_numpy() for o in exe.execute_buffers(args))
+        wv, wi = S.top_k(x, k, bf16=dt == "bf16")
+        _same(idx, wi)
+        _same(vals, wv)
+        exe.run_loop(args, 3)
+        return min(exe.run_loop(args, 10) for _ in range(5))
+
+    for rows, n in ((17, 54716), (64, 8192)):
+        assert run(rows, n, 256) < 12 * run(rows, n, 50)
 
 
 def test_sort_in_a_fixed_block(client, plugin):
