@@ -306,13 +306,14 @@ struct WordSource {
   int64_t len = 0;      // words of a row
   int64_t stride = 0;   // list: words from one row to the next
   int vec = 0;          // keys: 16-byte loads (inner == 1, rows 16-byte aligned)
+  int near = 0;         // keys: a thread's eight are neighbours
 };
 
 // The images of the thread's eight of keys [base, base + 8 threads) of a row
 // (any of them, since a word carries its position): key e is at position
 // base + key_at(src, tid, threads, e), past the row when that is >= src.len.
 __device__ __forceinline__ int key_at(const WordSource& src, int tid, int threads, int e) {
-  return src.vec ? tid * kGroup + e : tid + e * threads;
+  return src.vec || src.near ? tid * kGroup + e : tid + e * threads;
 }
 __device__ __forceinline__ void load_images(const WordSource& src, const SortRows& r, const KeyMap& map, int64_t row,
                                             int64_t base, int tid, int threads, uint32_t (&img)[kGroup]) {
@@ -339,7 +340,7 @@ __device__ __forceinline__ void load_images(const WordSource& src, const SortRow
     const int64_t row0 = outer * r.n * r.inner + j;
 #pragma unroll
     for (int e = 0; e < kGroup; ++e) {
-      const int64_t i = base + tid + (int64_t)e * threads;
+      const int64_t i = base + key_at(src, tid, threads, e);
       raw[e] = i < end ? load_key(src.keys, row0 + i * r.inner, r.key_bits) : 0u;
     }
   }
@@ -389,8 +390,8 @@ struct BlockPass {
 // the pair's two runs (a binary search), then reads its N words in one LDS
 // latency and merges them in registers. Rounds within a wave's words need no
 // barrier. Bound by instruction issue, most of it the searches (which is why
-// a thread holds 16 words and not 8, unless rows are short). Whole sorts with
-// positions, bitonic blocks and passes before -> now: [4096, 1024] 101 -> 45 us,
+// a thread holds 16 words and not 8 in long rows). Whole sorts with
+// positions, bitonic blocks and passes before -> now: [4096, 1024] 118 -> 42 us,
 // [64, 32000] 187 -> 57, [64, 128256] bf16 735 -> 212, [1, 2^20] 329 -> 116.
 template <int N>
 __global__ void __launch_bounds__(kSortThreads) sort_block_kernel(BlockPass p) {
@@ -410,9 +411,27 @@ __global__ void __launch_bounds__(kSortThreads) sort_block_kernel(BlockPass p) {
   }
   sort_words(w);
   const int mine = tid * N;
+  // The words of a short row lie in the first threads: one run holds them all
+  // before the block is sorted.
+  int words = p.src.near ? (int)p.src.len : threads * N;
+  if constexpr (N == kGroup) {
+    if (p.src.near && p.g.out_n <= N) {
+      // The first eight of two threads' sorted eights: the smaller of one
+      // ascending and the other descending, which is bitonic.
+      for (int d = 1; d * N < words; d *= 2) {
+        double o[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) o[e] = __shfl_xor(w[N - 1 - e], d, 64);
+#pragma unroll
+        for (int e = 0; e < N; ++e) asm("v_min_f64 %0, %0, %1" : "+v"(w[e]) : "v"(o[e]));
+        merge_words(w);
+      }
+      words = 0;  // thread 0 has them
+    }
+  }
 #pragma unroll
   for (int e = 0; e < N; ++e) sw[slot(mine + e)] = w[e];
-  for (int run = N; run < threads * N; run *= 2) {
+  for (int run = N; run < words; run *= 2) {
     const bool wave = 2 * run <= 64 * N;
     if (wave) wave_sync();
     else __syncthreads();
@@ -878,7 +897,12 @@ Layout layout_of(const SortRows& r, int64_t out_n, int64_t max_bytes) {
     L.bytes = static_cast<size_t>(r.rows * L.p) * 8;
     return L;
   };
-  const bool topk = out_n < r.n && out_n <= kTopkMax, keep = r.n > kSortTile && out_n <= kSortTile / 2;
+  // Short rows are sorted whole: a bound costs its 256 counts however few the
+  // words are. us bounded / sorted: [256, 64] k = 20 8.5 / 5.7, [256, 500] k =
+  // 5 7.9 / 8.5, k = 50 8.8 / 8.4, k = 250 26 / 9.6, [4096, 500] k = 50 42 / 15;
+  // longer ones [256, 1000] k = 50 8.6 / 9.9, [17, 2047] k = 256 22 / 15.
+  const bool whole = r.n <= 64 * kGroup || (r.n <= 2048 && out_n > kTopkThreads / 2);
+  const bool topk = out_n < r.n && out_n <= kTopkMax && !whole, keep = r.n > kSortTile && out_n <= kSortTile / 2;
   if (r.n >= kWordRows && !topk && !keep) return bitonic();
   L.piece_len = r.n < kWordRows ? std::max<int64_t>(r.n, 1) : kWordRows / 2;
   L.pieces = static_cast<int>(ceil_div(r.n, L.piece_len));
@@ -910,9 +934,14 @@ unsigned grid_of(int64_t rows, int64_t per_row) {
   return static_cast<unsigned>(grid);
 }
 
-// Blocks of `words` <= kSortTile words.
-void sort_blocks(hipStream_t s, const BlockPass& p, int64_t words) {
-  const int n = words <= 64 * kGroup ? kGroup : 16;
+// Blocks of `words` <= kSortTile words. A whole row of one wave's words (512)
+// is merged only as far as it goes ([1024, 8] f32 argsort 8.8 us with all six
+// rounds, 4.1 so), and rows of up to 2048 words by threads of 8, whose rounds
+// are shorter ([16, 1000] 18.1 us with 16 a thread, 13.2 with 8; [4096, 1000] 45
+// and 42, but [4096, 4000] 128 and 134).
+void sort_blocks(hipStream_t s, BlockPass p, int64_t words) {
+  p.src.near = !p.src.list && p.blocks_per_row == 1 && words <= 64 * kGroup;
+  const int n = words <= 2048 ? kGroup : 16;
   const int threads = static_cast<int>(std::max<int64_t>(64, pow2_at_least(ceil_div(words, n))));
   const dim3 grid(grid_of(p.r.rows, p.blocks_per_row));
   if (n == kGroup) hipLaunchKernelGGL((sort_block_kernel<kGroup>), grid, dim3(threads), words_lds(threads * n), s, p);

@@ -66,7 +66,9 @@ def test_argsort_other_dims(client, shape, dim):
 
 @pytest.mark.parametrize("rows,n,k", [(1, 300, 256), (3, 2048, 1), (3, 2049, 256), (64, 8192, 50), (5, 8193, 50),
                                       (2, 100000, 256), (1, 1000000, 200), (3, 9000, 257), (3, 50000, 4096),
-                                      (3, 50000, 4097), (300, 2050, 5), (3, 8192, 256), (7, 5000, 200)])
+                                      (3, 50000, 4097), (300, 2050, 5), (3, 8192, 256), (7, 5000, 200),
+                                      (5, 9, 8), (5, 8, 1), (300, 512, 8), (3, 511, 9), (3, 513, 8), (3, 65, 7),
+                                      (3, 512, 511), (3, 2048, 129), (3, 2049, 129)])
 @pytest.mark.parametrize("distinct", [0, 2, 40])
 def test_top_k_edges(client, rows, n, k, distinct):
     """Chunks of one, two and four groups a thread, one to three rounds, and
@@ -106,6 +108,22 @@ def test_top_k_as_many_as_threads(client, dt, order):
 
     for rows, n in ((17, 54716), (64, 8192)):
         assert run(rows, n, 256) < 12 * run(rows, n, 50)
+
+
+def test_short_rows_take_less(client):
+    """Rows are merged only as far as they go, and short ones are not bounded
+    first: each took as long as the longest a wave holds (times of launches of
+    4 and 12 us; 9 and 9 before)."""
+    def best(n, k):
+        b = Builder("jit_short")
+        p = b.param((256, n), "f32")
+        exe = client.compile(b.build(list(b.top_k(p, k) if k else b.sort([p, b.iota((256, n), 1)], 1))))
+        args = [client.buffer(np.random.default_rng(n).standard_normal((256, n)).astype(np.float32))]
+        exe.run_loop(args, 10)
+        return min(exe.run_loop(args, 50) for _ in range(5))
+
+    assert best(8, 0) < 0.75 * best(512, 0)
+    assert best(64, 20) < 0.85 * best(2000, 20)
 
 
 def test_sort_in_a_fixed_block(client, plugin):
