@@ -108,6 +108,49 @@ GemmGroup gemm_group(const GemmParams& g) {
   return gg;
 }
 
+// True where one launch of the scalar kernel is faster than the launches the
+// matrix-core kernels take for this 16-bit product with its copies and pads.
+// Measured: 2.2 us + 0.19 a contracted element (its loads are a chain), or + 2 us
+// a million results + 0.42 a million multiplications (0.66 where neighbouring
+// results read B rows apart), against 4.1 us for the tiles with 0.75 a million
+// results (of whole 64 x 64 tiles), 6.3 for the GEMV of a ragged K (3.7 with one
+// row) and 2.6 for every launch before or after them.
+// us scalar / padded: [256, 256] K = 9 3.9 / 9.4, K = 28 7.2 / 9.5, K = 44 10.2
+// / 9.5; [1000, 520] K = 5 4.5 / 7.2, K = 20 8.1 / 7.4; [4096, 512] K = 5 10.4 /
+// 8.3. `add_apart`: an addend the tiles would add in place.
+bool scalar_is_faster(OperandView a, OperandView b, bool a_aligned, bool b_aligned, bool add_apart) {
+  const int64_t M = a.free, N = b.free, K = a.k, batch = a.batch;
+  int extra = 0;  // launches the scalar kernel does without (an operand with no one stride is copied for it, too)
+  for (OperandView* v : {&a, &b})
+    if (!v->ok) {
+      *v = OperandView{v->batch, v->free, v->k, v->free * v->k, v->k, 1, true};
+      (v == &a ? a_aligned : b_aligned) = true;
+    }
+  if (a.ks != 1 && K != 1 && M <= 8) {
+    a = OperandView{batch, M, K, M * K, K, 1, true};
+    a_aligned = true;
+    ++extra;
+  }
+  const DotLayout l = layout_of(a, b);
+  if (!l.ready) return false;
+  const bool b_whole = b_aligned && whole_rows(b, l.b_kmajor);
+  double other = 4.1;
+  if (M <= 8 && (a.ks == 1 || K == 1) && b_whole && (l.b_kmajor || N % 8 == 0) &&
+      (!l.b_kmajor || (a_aligned && (M == 1 || a.fs % 8 == 0) && (batch == 1 || a.bs % 8 == 0)))) {
+    if (extra == 0 && (K % 8 == 0 || M == 1)) return false;
+    other = M == 1 ? 3.7 : 6.3;
+    add_apart = false;  // the GEMV's result is added to in another launch as well
+  } else {
+    extra += !(a_aligned && whole_rows(a, l.a_kmajor)) + !b_whole;
+    if (extra == 0 && K % 8 == 0) return false;
+    other += 0.75e-6 * 4096 * static_cast<double>(batch) * ((M + 63) / 64) * ((N + 63) / 64);
+  }
+  const double results = static_cast<double>(batch) * M * N;
+  const double chain = std::max(3.8, 2.2 + 0.19 * K);
+  const double stream = 2.2 + results * (2e-6 + K * (b.fs == 1 || N == 1 ? 0.42e-6 : 0.66e-6));
+  return std::max(chain, stream) + (add_apart ? 2.6 : 0.0) < other + 2.6 * extra;
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 // Copies `t` into a canonical [batch][free][k] (or [batch][k][free] when
@@ -164,10 +207,11 @@ int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row) {
   return row ? 0 : view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract).free;
 }
 
-std::string describe_dot(const Program& prog, const Op& dot) {
+std::string describe_dot(const Program& prog, const Op& dot, bool add) {
   OperandView a = view_of(prog.type(dot.operands[0]), dot.lhs_batch, dot.lhs_contract);
   OperandView b = view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract);
   const bool a_copied = !a.ok, b_copied = !b.ok;
+  const bool scalar = scalar_is_faster(a, b, true, true, add);
   for (OperandView* v : {&a, &b})
     if (!v->ok) *v = OperandView{v->batch, v->free, v->k, v->free * v->k, v->k, 1, true};
   const DotLayout l = layout_of(a, b);
@@ -184,7 +228,7 @@ std::string describe_dot(const Program& prog, const Op& dot) {
   };
   const bool tiles = gemm_fits(gemm_group(gemm_params(taken(a, l.a_kmajor), taken(b, l.b_kmajor), l)), l.a_kmajor, l.b_kmajor);
   return std::string("\"operands\":[") + one(a_copied, a, l.a_kmajor) + "," + one(b_copied, b, l.b_kmajor) +
-         "],\"block_tiles\":" + (tiles ? "true" : "false");
+         "],\"block_tiles\":" + (tiles ? "true" : "false") + ",\"scalar\":" + (scalar ? "true" : "false");
 }
 
 // Writes the product to the dot's result, plus `add` (GemmMember::add, its
@@ -217,7 +261,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
     launch_zero(dev->stream(), out, ot.elements() * static_cast<int64_t>(dtype_size(ot.dtype)));
     return false;
   }
-  if (low_precision && out_ok) {
+  if (low_precision && out_ok && !scalar_is_faster(a, b, aligned16(A), aligned16(B), add != nullptr)) {
     const bool f16 = lt.dtype == DType::kF16;
     const int out_kind = ot.dtype == DType::kBF16 ? 0 : (ot.dtype == DType::kF16 ? 1 : 2);
     MemRef a_copy, b_copy, a_pad, b_pad;

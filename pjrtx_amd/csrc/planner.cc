@@ -1469,7 +1469,7 @@ std::string Plan::describe(const Program& prog) const {
           flops += 2 * prog.type(d.results[0]).elements() * kc;
         }
         o << ",\"flops\":" << flops;
-        if (s.lib == LibKind::kDot) o << "," << describe_dot(prog, prog.ops[s.lib_op]);
+        if (s.lib == LibKind::kDot) o << "," << describe_dot(prog, prog.ops[s.lib_op], s.dot_add >= 0);
         if (s.lib == LibKind::kDotGroup) o << ",\"group_size\":" << s.group_ops.size();
         if (s.dot_add >= 0)
           o << ",\"residual_add\":" << s.dot_add

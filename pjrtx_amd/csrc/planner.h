@@ -260,9 +260,10 @@ bool fold_dot_transpose(Program* prog);
 // Elements from one row of a merged addend to the next (dot_general.cc).
 int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row);
 // JSON members: how the block tiles take each operand of a product of 16-byte
-// aligned buffers ("read" in place, "padded" or "copied"), and whether its
-// sizes are within theirs (dot_general.cc).
-std::string describe_dot(const Program& prog, const Op& dot);
+// aligned buffers ("read" in place, "padded" or "copied"), whether its sizes are
+// within theirs, and whether, with 16-bit operands, it goes to the scalar kernel
+// (dot_general.cc). `add`: an addend is merged into it.
+std::string describe_dot(const Program& prog, const Op& dot, bool add);
 
 // Turns decode-shaped dot and dot-group library steps into kGemv steps and
 // absorbs their row-fused prologues and elementwise epilogues

@@ -148,3 +148,43 @@ def test_transposed_result_of_whole_numbers(client, batch, lhs, rhs, dt):
         d = b.dot_general(x, y, batch=((0,), (0,)) if batch else ((), ()), contract=((lhs.index("k"),), (rhs.index("k"),)))
         (got,) = client.compile(b.build([b.transpose(d, [0, 2, 1] if batch else [1, 0])]))(*vals, dtypes=[dt] * 2)
         np.testing.assert_array_equal(got, np.einsum(f"{lhs},{rhs}->{batch}nm", *vals))
+
+
+@pytest.mark.parametrize("form", ["plain", "f32", "row", "full", "transposed", "members"])
+@pytest.mark.parametrize("spec", ["mk,kn", "mk,nk", "km,kn", "km,nk", "akm,kn", "mk,nak"])
+def test_small_ragged_products(client, form, spec):
+    """Products whose operands would be padded for the tiles, of few enough
+    multiplications to go to the scalar kernel in one launch (and, k = 61,
+    too many): whole numbers, exact in every form."""
+    ls, rs = spec.split(",")
+    for dt in ("bf16", "f16"):
+        for m, n, k in [(1, 17, 3), (3, 40, 9), (8, 1000, 3), (9, 16, 5), (40, 33, 12), (257, 65, 2), (33, 40, 61)]:
+            size = dict(a=3, m=m, n=n, k=k)
+            rng = np.random.default_rng(k)
+            x, y, y2 = (rng.integers(-3, 4, [size[c] for c in s]).astype(np.float32) for s in (ls, rs, rs))
+            store = (lambda v: ops.f32_to_bf16_bits(v)) if dt == "bf16" else (lambda v: v.astype(np.float16))
+            b = Builder()
+            px, py = b.param(x.shape, dt), b.param(y.shape, dt)
+            kw = dict(contract=((ls.index("k"),), (rs.index("k"),)), out_dtype="f32" if form == "f32" else None)
+            d = b.dot_general(px, py, **kw)
+            lf, rf = ls.replace("k", ""), rs.replace("k", "")
+            want = np.einsum(f"{ls},{rs}->{lf}{rf}", x, y)
+            args, outs, wants = [x, y], [d], [want]
+            if form in ("row", "full"):
+                z = rng.integers(-3, 4, want.shape[-1:] if form == "row" else want.shape).astype(np.float32)
+                pz = b.param(z.shape, dt)
+                outs = [b.add(d, b.broadcast_in_dim(pz, want.shape, [want.ndim - 1]) if form == "row" else pz)]
+                args, wants = args + [z], [want + z]
+            if form == "transposed":
+                perm = list(range(len(lf), want.ndim)) + list(range(len(lf)))
+                outs, wants = [b.transpose(d, perm)], [want.transpose(perm)]
+            if form == "members":
+                outs.append(b.dot_general(px, b.param(y.shape, dt), **kw))
+                args, wants = args + [y2], wants + [np.einsum(f"{ls},{rs}->{lf}{rf}", x, y2)]
+            got = client.compile(b.build(outs))(*(store(v) for v in args), dtypes=[dt] * len(args))
+            for g, w in zip(got, wants):
+                # |sums| <= 9 * 61 + 3: beyond 256 bf16 rounds the product and the sum to even numbers.
+                if form == "f32":
+                    np.testing.assert_array_equal(g, w)
+                else:
+                    assert (np.abs(_f64(g, dt) - w) <= (0 if np.abs(w).max() < 250 else 2)).all()

@@ -74,7 +74,7 @@ def test_k_splits(client, m, n, k):
 
 
 @pytest.mark.parametrize("sizes", [(2, 19, 21, 13), (3, 65, 130, 67), (1, 100, 9, 1), (2, 1, 40, 70), (2, 40, 1, 70),
-                                   (2, 5, 24, 64), (1, 8, 23, 65)])
+                                   (2, 5, 24, 64), (1, 8, 23, 65), (2, 19, 21, 61), (1, 100, 9, 57)])
 def test_dimension_orders(client, sizes):
     """Every order of the operands' dimensions, odd sizes (rows that are not
     16-byte aligned are padded first), unit dimensions, decode rows."""

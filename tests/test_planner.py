@@ -475,6 +475,29 @@ def _operands(plugin, lhs, rhs, contract, batch=((), ())):
     return step["operands"]
 
 
+@pytest.mark.parametrize("lhs,rhs,contract,scalar", [
+    ((256, 9), (9, 256), ((1,), (0,)), True),            # padded first, 2.6 us more a launch
+    ((256, 9), (256, 9), ((1,), (1,)), True),
+    ((256, 28), (256, 28), ((1,), (1,)), True),          # both padded
+    ((256, 28), (28, 256), ((1,), (0,)), False),         # one
+    ((256, 44), (256, 44), ((1,), (1,)), False),
+    ((256, 8), (8, 256), ((1,), (0,)), False),           # nothing to pad
+    ((12, 256), (12, 256), ((0,), (0,)), False),
+    ((5, 256), (5, 256), ((0,), (0,)), True),            # less than a k-tile's launch
+    ((512, 2), (4096, 2), ((1,), (1,)), True),
+    ((1000, 5), (5, 520), ((1,), (0,)), True),
+    ((4096, 5), (5, 4096), ((1,), (0,)), False),         # too many results
+    ((3, 9), (9, 8192), ((1,), (0,)), True),             # decode rows: the GEMV of a ragged K
+    ((1, 9), (9, 8192), ((1,), (0,)), False),
+    ((3, 64), (64, 8192), ((1,), (0,)), False),
+])
+def test_small_ragged_products_go_to_the_scalar_kernel(plugin, lhs, rhs, contract, scalar):
+    b = Builder()
+    d = b.dot_general(b.param(lhs, "bf16"), b.param(rhs, "bf16"), contract=contract)
+    (step,) = plan(plugin, b.build([d]))["steps"]
+    assert step.get("scalar", False) is scalar
+
+
 def test_operands_are_read_within_their_bounds(plugin):
     """The block tiles read whole 16-byte pieces: an operand whose only row
     ends inside one (an outer product's right side) is padded like ragged rows."""
