@@ -1238,6 +1238,10 @@ void Planner::shape_reduce(Step* s) {
       int one = lanes;
       while (one > 8 && (blocks_of(one) < 256 || per_thread(one) > 32)) one /= 2;
       if (per_thread(one) <= 32) lanes = one;
+      // The fold of a workgroup's lane rows is a chain: few outputs of columns
+      // that stay one launch take idle lanes and 32 lane rows (f32 [64, 1] 6.3
+      // us with 256 of them, 3.1 so, [1000, 2] 6.5 and 3.6).
+      while (lanes < 8 && per_thread(8) <= 32) lanes *= 2;
       // Rows of an odd number of elements are read one element a lane: 256
       // lanes keep the pieces long ([1024, 40001] f32 111 -> 30 us, bf16 93 ->
       // 22; below 256 elements 64 lanes are as fast).

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 # Below and at the schedule's threshold (32), one split and many, vectors of
 # 8, 4, 2 and 1 elements, lanes past the last output, one output.
 SHAPES = [((31, 40), (0,)), ((32, 40), (0,)), ((1000, 5632), (0,)), ((1001, 7), (0,)), ((4099, 1), (0,)),
-          ((70, 33, 6), (0,)), ((33, 70, 514), (1,)), ((16, 9, 12, 20), (0, 2)), ((40, 50, 24), (0, 1)), ((65, 0), (0,))]
+          ((70, 33, 6), (0,)), ((33, 70, 514), (1,)), ((16, 9, 12, 20), (0, 2)), ((40, 50, 24), (0, 1)), ((65, 0), (0,)),
+          ((64, 1), (0,)), ((200, 16), (0,)), ((3, 256, 2), (1,)), ((1024, 3), (0,)), ((1025, 2), (0,))]
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "s32", "f64"])

@@ -539,6 +539,7 @@ def test_dims_of_one_element_do_not_merge_their_neighbours(plugin):
     ((1024, 65540), ["f32"], 0), ((1024, 65537), ["bf16"], 0), ((32, 65537), ["f32"], "64"),
     ((256, 65536), ["bf16", "f32", "f32"], 0), ((256, 40960), ["bf16", "f32", "f32"], "64"),
     ((1024, 40001), ["f32"], 256), ((1024, 9001), ["f32"], "64"), ((100, 40001), ["f32"], "64"),
+    ((64, 1), ["f32"], 8), ((200, 16), ["bf16"], 8),  # short columns of few outputs: 32 lane rows
 ])
 def test_schedule_of_column_reductions(plugin, shape, inputs, lanes):
     """Lanes that span outputs, or one serial thread an output where that
