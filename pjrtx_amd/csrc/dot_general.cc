@@ -151,6 +151,15 @@ bool scalar_is_faster(OperandView a, OperandView b, bool a_aligned, bool b_align
   return std::max(chain, stream) + (add_apart ? 2.6 : 0.0) < other + 2.6 * extra;
 }
 
+// Decode rows with few and ragged N-contiguous columns: B is transposed for the
+// K-contiguous GEMV, which spreads each column's K over lanes, where padded rows
+// would go to the tiles and their k-splits. us transposed / padded: 1 x 2048 x
+// 33 6.8 / 12.0, x 257 8.8 / 12.7, x 1001 15.5 / 15.4; 3 x 4096 x 257 14.8 /
+// 15.9; 8 x 4096 x 33 19.2 / 13.3; with K = 256 they are equal.
+bool few_ragged_columns(const OperandView& a, const OperandView& b) {
+  return b.ok && a.batch == 1 && a.free <= 4 && b.free <= 512 && b.free % 8 != 0 && b.k >= 512 && b.k % 8 == 0 && b.ks != 1;
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 // Copies `t` into a canonical [batch][free][k] (or [batch][k][free] when
@@ -210,10 +219,10 @@ int64_t dot_addend_stride(const Program& prog, const Op& dot, bool row) {
 std::string describe_dot(const Program& prog, const Op& dot, bool add) {
   OperandView a = view_of(prog.type(dot.operands[0]), dot.lhs_batch, dot.lhs_contract);
   OperandView b = view_of(prog.type(dot.operands[1]), dot.rhs_batch, dot.rhs_contract);
-  const bool a_copied = !a.ok, b_copied = !b.ok;
+  const bool a_copied = !a.ok, b_copied = !b.ok || few_ragged_columns(a, b);
   const bool scalar = scalar_is_faster(a, b, true, true, add);
   for (OperandView* v : {&a, &b})
-    if (!v->ok) *v = OperandView{v->batch, v->free, v->k, v->free * v->k, v->k, 1, true};
+    if (v == &a ? a_copied : b_copied) *v = OperandView{v->batch, v->free, v->k, v->free * v->k, v->k, 1, true};
   const DotLayout l = layout_of(a, b);
   const auto one = [](bool copied, const OperandView& v, bool kmajor) {
     return copied ? "\"copied\"" : !whole_rows(v, kmajor) ? "\"padded\"" : "\"read\"";
@@ -275,7 +284,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
       A = a_copy->ptr;
       a = OperandView{batch, M, K, M * K, K, 1, true};
     }
-    if (!b.ok && fits(rt.bytes())) {
+    if ((!b.ok || few_ragged_columns(a, b)) && fits(rt.bytes())) {
       b_copy = canonicalize(dev, rt, op.rhs_batch, op.rhs_contract, B, true);  // [batch][N][K]
       B = b_copy->ptr;
       b = OperandView{batch, N, K, N * K, K, 1, true};

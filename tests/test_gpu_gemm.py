@@ -138,6 +138,15 @@ def test_rows_of_four_million_elements(client, spec, dt, out_dt):
     np.testing.assert_array_equal(got, want if out_dt == "f32" else to_bf16_bits(want))
 
 
+@pytest.mark.parametrize("m", [1, 3, 4])
+@pytest.mark.parametrize("n,k", [(9, 512), (33, 2048), (257, 1032), (511, 520)])
+def test_decode_rows_of_few_ragged_columns(client, m, n, k):
+    for spec in LAYOUTS:
+        for dt, out_dt in (("bf16", None), ("f16", "f32")):
+            got, want = _dot(client, spec, {"m": m, "n": n, "k": k}, dt, out_dt, seed=n)
+            _check(got, want, k, dt, out_dt)
+
+
 def test_same_bits_on_every_call(client):
     sizes = {"m": 100, "n": 520, "k": 4104}
     a, _ = _dot(client, "mk,kn", sizes)

@@ -523,6 +523,18 @@ def test_sizes_of_the_block_tiles(plugin, lhs, rhs, contract, tiles):
     assert step["block_tiles"] is tiles
 
 
+def test_few_ragged_columns_are_transposed_for_decode_rows(plugin):
+    """The K-contiguous GEMV is the faster one there (2048 x 257: 8.8 us, 12.7
+    padded for the tiles)."""
+    kn = ((1,), (0,))
+    assert _operands(plugin, (1, 2048), (2048, 257), kn) == ["read", "copied"]
+    assert _operands(plugin, (4, 512), (512, 10), kn) == ["read", "copied"]
+    assert _operands(plugin, (5, 2048), (2048, 257), kn) == ["read", "padded"]
+    assert _operands(plugin, (1, 2048), (2048, 513), kn) == ["read", "padded"]
+    assert _operands(plugin, (1, 2044), (2044, 257), kn) == ["padded", "padded"]
+    assert _operands(plugin, (1, 2048), (257, 2048), ((1,), (1,))) == ["read", "read"]
+
+
 def test_dims_of_one_element_do_not_merge_their_neighbours(plugin):
     """Free (or contracted) dims are one stride only where the dims of more
     than one element follow each other; one of 1 between them changes nothing."""
