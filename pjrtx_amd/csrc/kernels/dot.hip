@@ -10,7 +10,8 @@
 //    runs of tiles so neighbouring tiles share an L2.
 //  * gemv: M <= 8 rows (decode), split over K with a deterministic second
 //    pass; memory-bound on the weight stream.
-//  * fma_gemm: scalar fallback for f32 / f64 and unaligned layouts.
+//  * fma_gemm: the scalar kernel, for f32, f64 and s32, layouts the others do not
+//    take, and small ragged 16-bit products, which padding would cost more.
 //
 // Replaces the reference's dot_general (reference:
 // src/backend/mlx_metal/api.cc:3349-3498, mlx::matmul / tensordot) and the
