@@ -900,8 +900,9 @@ Layout layout_of(const SortRows& r, int64_t out_n, int64_t max_bytes) {
   // Short rows are sorted whole: a bound costs its 256 counts however few the
   // words are. us bounded / sorted: [256, 64] k = 20 8.5 / 5.7, [256, 500] k =
   // 5 7.9 / 8.5, k = 50 8.8 / 8.4, k = 250 26 / 9.6, [4096, 500] k = 50 42 / 15;
-  // longer ones [256, 1000] k = 50 8.6 / 9.9, [17, 2047] k = 256 22 / 15.
-  const bool whole = r.n <= 64 * kGroup || (r.n <= 2048 && out_n > kTopkThreads / 2);
+  // longer ones [256, 1000] k = 20 8.2 / 9.9, bf16 k = 64 10.9 / 9.9,
+  // [17, 2047] k = 256 22 / 15.
+  const bool whole = r.n <= 64 * kGroup || (r.n <= 1024 && out_n > 40) || (r.n <= 2048 && out_n > kTopkThreads / 2);
   const bool topk = out_n < r.n && out_n <= kTopkMax && !whole, keep = r.n > kSortTile && out_n <= kSortTile / 2;
   if (r.n >= kWordRows && !topk && !keep) return bitonic();
   L.piece_len = r.n < kWordRows ? std::max<int64_t>(r.n, 1) : kWordRows / 2;
@@ -953,6 +954,10 @@ void topk_blocks_launch(hipStream_t s, TopkPass p, int share) {
   const dim3 grid(grid_of(p.r.rows, p.blocks_per_row)), block(kTopkThreads);
   const size_t lds = static_cast<size_t>(p.need * share * kGroup + kTopkPad) * 8;
   p.group = p.need <= 56 ? 4 : p.need <= 112 ? 2 : 1;
+  // As many groups as `need` hold words, or the bound takes them all (bf16 [9,
+  // 576] k = 20 14.7 us, 8.6 so).
+  const int64_t holding = std::min<int64_t>(kTopkThreads, ceil_div(p.src.len, kGroup));
+  while (p.group > 1 && holding / p.group < p.need) p.group /= 2;
   const bool half = !p.src.list && p.src.vec && p.r.key_bits == 16 && p.r.key_class != kSortKeyFloat;
 #define PJRTX_TOPK(SHARE)                                                                  \
   if (half) hipLaunchKernelGGL((topk_half_kernel<SHARE>), grid, block, lds, s, p);         \

@@ -68,7 +68,8 @@ def test_argsort_other_dims(client, shape, dim):
                                       (2, 100000, 256), (1, 1000000, 200), (3, 9000, 257), (3, 50000, 4096),
                                       (3, 50000, 4097), (300, 2050, 5), (3, 8192, 256), (7, 5000, 200),
                                       (5, 9, 8), (5, 8, 1), (300, 512, 8), (3, 511, 9), (3, 513, 8), (3, 65, 7),
-                                      (3, 512, 511), (3, 2048, 129), (3, 2049, 129)])
+                                      (3, 512, 511), (3, 2048, 129), (3, 2049, 129),
+                                      (9, 576, 20), (9, 576, 40), (9, 1024, 41), (5, 1032, 41), (5, 1032, 100)])
 @pytest.mark.parametrize("distinct", [0, 2, 40])
 def test_top_k_edges(client, rows, n, k, distinct):
     """Chunks of one, two and four groups a thread, one to three rounds, and
@@ -114,16 +115,18 @@ def test_short_rows_take_less(client):
     """Rows are merged only as far as they go, and short ones are not bounded
     first: each took as long as the longest a wave holds (times of launches of
     4 and 12 us; 9 and 9 before)."""
-    def best(n, k):
+    def best(n, k, dt="f32"):
         b = Builder("jit_short")
-        p = b.param((256, n), "f32")
+        p = b.param((256, n), dt)
         exe = client.compile(b.build(list(b.top_k(p, k) if k else b.sort([p, b.iota((256, n), 1)], 1))))
-        args = [client.buffer(np.random.default_rng(n).standard_normal((256, n)).astype(np.float32))]
+        x = _keys(np.random.default_rng(n), (256, n), dt, 0)
+        args = [client.buffer(x, dt)]
         exe.run_loop(args, 10)
         return min(exe.run_loop(args, 50) for _ in range(5))
 
     assert best(8, 0) < 0.75 * best(512, 0)
     assert best(64, 20) < 0.85 * best(2000, 20)
+    assert best(576, 20, "bf16") < 1.4 * best(2048, 20, "bf16")  # 8.6 and 7.2 us, 14.7 before
 
 
 def test_sort_in_a_fixed_block(client, plugin):
