@@ -108,12 +108,17 @@ GemmGroup gemm_group(const GemmParams& g) {
   return gg;
 }
 
+// Decode rows that contract a short ragged K go to the tiles with padded rows:
+// the GEMV walks K's rows one at a time. us GEMV / tiles: 4 x 44 x 512 9.4 /
+// 6.7, 6 x 58 x 16 16.4 / 6.7, three batches of 7 x 73 x 896 19 / 7.
+bool short_ragged_rows(const OperandView& a) { return a.free >= 2 && a.free <= 8 && a.k % 8 != 0 && a.k <= 128; }
+
 // True where one launch of the scalar kernel is faster than the launches the
 // matrix-core kernels take for this 16-bit product with its copies and pads.
 // Measured: 2.2 us + 0.19 a contracted element (its loads are a chain), or + 2 us
 // a million results + 0.42 a million multiplications (0.66 where neighbouring
 // results read B rows apart), against 4.1 us for the tiles with 0.75 a million
-// results (of whole 64 x 64 tiles), 6.3 for the GEMV of a ragged K (3.7 with one
+// results (of whole 64 x 64 tiles), 6.3 for the GEMV of decode rows (3.7 with one
 // row) and 2.6 for every launch before or after them.
 // us scalar / padded: [256, 256] K = 9 3.9 / 9.4, K = 28 7.2 / 9.5, K = 44 10.2
 // / 9.5; [1000, 520] K = 5 4.5 / 7.2, K = 20 8.1 / 7.4; [4096, 512] K = 5 10.4 /
@@ -126,7 +131,8 @@ bool scalar_is_faster(OperandView a, OperandView b, bool a_aligned, bool b_align
       *v = OperandView{v->batch, v->free, v->k, v->free * v->k, v->k, 1, true};
       (v == &a ? a_aligned : b_aligned) = true;
     }
-  if (a.ks != 1 && K != 1 && M <= 8) {
+  const bool gemv = M <= 8 && !short_ragged_rows(a);
+  if (a.ks != 1 && K != 1 && gemv) {
     a = OperandView{batch, M, K, M * K, K, 1, true};
     a_aligned = true;
     ++extra;
@@ -135,7 +141,7 @@ bool scalar_is_faster(OperandView a, OperandView b, bool a_aligned, bool b_align
   if (!l.ready) return false;
   const bool b_whole = b_aligned && whole_rows(b, l.b_kmajor);
   double other = 4.1;
-  if (M <= 8 && (a.ks == 1 || K == 1) && b_whole && (l.b_kmajor || N % 8 == 0) &&
+  if (gemv && (a.ks == 1 || K == 1) && b_whole && (l.b_kmajor || N % 8 == 0) &&
       (!l.b_kmajor || (a_aligned && (M == 1 || a.fs % 8 == 0) && (batch == 1 || a.bs % 8 == 0)))) {
     if (extra == 0 && (K % 8 == 0 || M == 1)) return false;
     other = M == 1 ? 3.7 : 6.3;
@@ -279,7 +285,8 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
     const auto fits = [&](int64_t bytes) { return scratch_left(dev) >= bytes + 4096; };
     // (An M-contiguous A goes to the GEMV kernels and to rows too long for
     // 32-bit offsets as a copy.)
-    if ((!a.ok || (a.ks != 1 && K != 1 && (M <= 8 || a.ks >= int64_t(1) << 23))) && fits(lt.bytes())) {
+    const bool gemv_rows = M <= 8 && !short_ragged_rows(a);
+    if ((!a.ok || (a.ks != 1 && K != 1 && (gemv_rows || a.ks >= int64_t(1) << 23))) && fits(lt.bytes())) {
       a_copy = canonicalize(dev, lt, op.lhs_batch, op.lhs_contract, A, true);
       A = a_copy->ptr;
       a = OperandView{batch, M, K, M * K, K, 1, true};
@@ -307,7 +314,7 @@ bool run_dot_general(Device* dev, const Program& prog, const Op& op, std::vector
     bool ready = lay.ready;
     // Decode rows: W streamed once. (K may be any length for an N-contiguous
     // W; a K-contiguous one needs 16-byte rows.)
-    if (ready && M <= 8 && (a.ks == 1 || K == 1) && aligned_rows(B, b, b_kmajor) && (b_kmajor || N % 8 == 0) &&
+    if (ready && gemv_rows && (a.ks == 1 || K == 1) && aligned_rows(B, b, b_kmajor) && (b_kmajor || N % 8 == 0) &&
         (!b_kmajor || (aligned16(A) && (M == 1 || a.fs % 8 == 0) && (batch == 1 || a.bs % 8 == 0)))) {
       if (batch == 1 && !b_kmajor && N < (int64_t(1) << 30) &&
           gemv_wide_fits(static_cast<int>(M), static_cast<int>(K), single_wide_tiles(N))) {

@@ -147,6 +147,15 @@ def test_decode_rows_of_few_ragged_columns(client, m, n, k):
             _check(got, want, k, dt, out_dt)
 
 
+@pytest.mark.parametrize("sizes", [(1, 2, 16, 58), (1, 6, 512, 44), (3, 7, 896, 73), (1, 8, 40, 127), (2, 5, 33, 129)])
+def test_decode_rows_of_a_short_ragged_contraction(client, sizes):
+    size = dict(zip("bmnk", sizes))
+    for spec in ("bmk,bkn", "bmk,bnk", "bkm,bkn", "bkm,bnk"):
+        for dt, out_dt in (("bf16", None), ("f16", "f32")):
+            got, want = _dot(client, spec, size, dt, out_dt, seed=size["k"])
+            _check(got, want, size["k"], dt, out_dt)
+
+
 def test_same_bits_on_every_call(client):
     sizes = {"m": 100, "n": 520, "k": 4104}
     a, _ = _dot(client, "mk,kn", sizes)
